@@ -135,6 +135,39 @@ PL_HD29 void mont29(const uint32_t* a, const uint32_t* w, uint32_t* t) {
   t[8] = (uint32_t)acc;
 }
 
+// t = x w for a fixed factor w given as nine pre-reduced rows: rows[9 j + i]
+// holds digit j of W_i = w 2^(29 (i + D)) mod r, W_i in (-0.51 r, 0.51 r) with
+// balanced digits (rows29_entry builds them).  V = sum_i x_i W_i is congruent
+// to x w 2^(29 D) and only about 2^34 r large, so D Montgomery digits instead
+// of nine bring it back: 81 + 8 D multiply-adds and 8 + D column closes
+// against mont29's 153 and 17.  The rows are 81 words per factor, which pays
+// where the factor is the same for all lanes and they stay in SGPRs.
+// With X = sum |x_i|, T = (V - m r) / 2^(29 D), m in [0, 2^(29 D)), lies in
+//   (-(0.51 X / 2^(29 D) + 1) r, 0.51 X / 2^(29 D) r]:
+// D = 2 gives (-1.001 r, 0.001 r) for any |x_i| < 2^31; D = 1 gives
+// (-10.2 r, 9.2 r) for |x_i| <= 2^30 and (-5.6 r, 4.6 r) for |x_i| <= 2^29.
+// Column bound: 9 * 2^31 * 2^28 + D * 2^58 + 2^34 < 2^62.3.  BT takes the
+// output digits t_0..t_7 balanced.
+template <int D, bool BT>
+PL_HD29 void rows29(const uint32_t* x, const uint32_t* rows, uint32_t* t) {
+  uint32_t m[D];
+  int64_t acc = 0;
+#pragma unroll
+  for (int k = 0; k < 8 + D; k++) {
+    if (k <= 8)
+      for (int i = 0; i < 9; i++) acc += (int64_t)(int32_t)x[i] * (int64_t)(int32_t)rows[9 * k + i];
+    for (int j = 0; j < D; j++)
+      if (k - j >= 1 && k - j <= 8) acc -= (int64_t)(int32_t)m[j] * (int64_t)r29(k - j);
+    const uint32_t dig = k >= D && BT ? sext29((uint32_t)acc) : ((uint32_t)acc & kMask29);
+    if (k < D)
+      m[k] = dig;
+    else
+      t[k - D] = dig;
+    acc = (acc - (int64_t)(int32_t)dig) >> 29;  // exact
+  }
+  t[8] = (uint32_t)acc;
+}
+
 // x (eight 32-bit limbs, a value mod 2^256) += r
 PL_HD29 void add_r256(uint32_t* x) {
   constexpr uint32_t kR[8] = {0x00000001u, 0xffffffffu, 0xfffe5bfeu, 0x53bda402u,
@@ -261,6 +294,15 @@ PL_HD29 void reduce_below_2r(const uint32_t* v, uint32_t* t) {
   t[8] = (uint32_t)(acc + (int64_t)(int32_t)v[8] - (int64_t)q * (int64_t)r29(8));
 }
 
+// column-major digits of one row of a rows29 factor: W_i given in [0, r) as
+// eight 32-bit limbs -> rows[9 j + i], j < 9
+PL_HD29 void rows29_row(const uint32_t* w, int i, uint32_t* rows) {
+  uint32_t a[9], b[9];
+  unpack_ext(w, a);
+  reduce_centered(a, b);
+  for (int j = 0; j < 9; j++) rows[9 * j + i] = b[j];
+}
+
 #undef PL_HD29
 
 }  // namespace pl
@@ -293,6 +335,60 @@ __device__ __forceinline__ void mont29_dev(const uint32_t* x, const uint32_t* w,
   });
   Mont29Col<17, UB, BT>::run(acc[17], acc[16], x, w, m);
   t[8] = (uint32_t)acc[17];
+}
+
+#include "rows29_columns.inc"
+
+// wave-uniform read-only words (loaded to SGPRs)
+typedef const __attribute__((address_space(4))) uint32_t* uwords;
+
+// Three columns (27 words) of a rows29 factor, in SGPRs.  rows29_open's loads
+// are issued where it stands: the scheduling barrier lets vector and LDS
+// instructions pass but neither the scalar loads nor the column blocks, so
+// they are in flight while the blocks before their use run.
+struct rows_cols {
+  uint32_t w[27];
+};
+__device__ __forceinline__ rows_cols rows29_open(uwords w, int group) {
+  rows_cols g;
+  asm volatile("" : "+s"(w));  // a fresh load: no rows held from product to product
+#pragma unroll
+  for (int i = 0; i < 27; i++) g.w[i] = w[27 * group + i];
+  __builtin_amdgcn_sched_barrier(0x0002 | 0x0004 | 0x0010 | 0x0080);
+  return g;
+}
+
+// rows29 on the device: x w for the wave-uniform factor whose rows are at w.
+// The 81 words come in three groups of three columns, each opened a group
+// (two columns, about 90 issue cycles) ahead of its use: all at once beside the kernel's
+// own they would not fit the scalar registers (180-230 spilled), and loaded
+// where they are used a lone wave waits for each group.  g holds the first group;
+// `next`, the factor of the product that follows, leaves its first group there.
+template <int D, bool BT>
+__device__ __forceinline__ void rows29_dev(const uint32_t* x, uwords w, rows_cols& g, uint32_t* t, uwords next) {
+  uint32_t m[D];
+  uint64_t acc[9 + D];
+  rows_cols g1, g2, gn;
+  static_for<0, 8 + D>([&](auto k_) {
+    constexpr int k = decltype(k_)::value;
+    // after the group's first column: scalar loads return in any order, so
+    // its wait would be for the new group's loads too
+    if constexpr (k == 1) g1 = rows29_open(w, 1);
+    if constexpr (k == 4) g2 = rows29_open(w, 2);
+    if constexpr (k == 7) gn = rows29_open(next, 0);
+    // block k closes column k - 1, an output column (balanced if BT) from D on
+    constexpr bool RND = BT && k - 1 >= D;
+    Rows29Col<k, D, RND>::run(acc[k], k ? acc[k ? k - 1 : 0] : 0, x, (k < 3 ? g : k < 6 ? g1 : g2).w + 9 * (k % 3),
+                              m);
+    const uint32_t lo = (uint32_t)acc[k];
+    if constexpr (k < D)
+      m[k] = lo & kMask29;
+    else
+      t[k - D] = BT ? sext29(lo) : (lo & kMask29);
+  });
+  Rows29Col<8 + D, D, BT>::run(acc[8 + D], acc[7 + D], x, g2.w, m);
+  t[8] = (uint32_t)acc[8 + D];
+  g = gn;
 }
 
 // a w / R' mod r for a < 2^256 (stored form, lazily reduced) and w given as
@@ -342,6 +438,14 @@ template <bool UB, bool BM, bool BT>
 __device__ __forceinline__ v9 v9_mul(const v9& x, const uint32_t (&w)[9]) {
   v9 t;
   mont29_dev<UB, BM, BT>(x.l, w, t.l);
+  return t;
+}
+
+// x w for the wave-uniform factor whose rows are at w (rows29_dev)
+template <int D, bool BT>
+__device__ __forceinline__ v9 v9_mul_rows(const v9& x, uwords w, rows_cols& g, uwords next) {
+  v9 t;
+  rows29_dev<D, BT>(x.l, w, g, t.l, next);
   return t;
 }
 

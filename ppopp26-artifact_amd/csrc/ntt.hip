@@ -87,6 +87,32 @@ __global__ void pbd_kernel(fr* t, uint64_t n) {
   fr_store(t + i, o);
 }
 
+// rows29 tables (fr29.hpp) of the in-register DFTs' factors (ntt_pass.hpp
+// kDftI ..), forward then inverse: one thread per row of a table.  c29, half
+// and inv32 are 2^29, 1/2 and 1/32 in stored form.
+__global__ void dft_rows_kernel(uint32_t* out, fr c29, fr half, fr inv32) {
+  const int t = threadIdx.x;
+  if (t >= 2 * kDftFactors * 9) return;
+  const int i = t % 9, e = t / 9 % kDftFactors, dir = t / (9 * kDftFactors);
+  auto root = [&](int k) {  // w_16^(+-k), stored form
+    uint32_t d[9];
+    reduce_below_2r(kW16b[dir][k], d);
+    fr v;
+    join29(d, v.l);
+    return fr_mul(fr_reduce_once(v), inv32);
+  };
+  fr w = root(4);
+  if (e != kDftI) {
+    const fr a = root(2), b = root(6);
+    w = fr_mul(e == kDftC1 ? fr_add(a, b) : fr_sub(a, b), half);
+  }
+  for (int k = 0; k < i + 1; k++) w = fr_mul(w, c29);  // D = 1
+  fr plain = fr_zero();
+  plain.l[0] = 1;
+  w = fr_mul(w, plain);  // the row as a plain integer below r
+  rows29_row(w.l, i, out + (dir * kDftFactors + e) * kRowWords);
+}
+
 static inline fr to_dev(const host::fr64& h) {
   fr f;
   memcpy(f.l, h.l, 32);
@@ -182,7 +208,8 @@ hipError_t domain_build(Domain& d, int lg, hipStream_t s) {
   d.lg = lg;
   d.plan = make_plan(lg);
   const NttPlan& P = d.plan;
-  size_t count = 4 * 256 + 2 * 16384;  // inner tables (both forms), w_N power windows
+  constexpr size_t kRowsFr = (2 * kDftFactors * kRowWords * sizeof(uint32_t) + sizeof(fr) - 1) / sizeof(fr);
+  size_t count = 4 * 256 + 2 * 16384 + kRowsFr;  // inner tables (both forms), w_N power windows, DFT factors
   for (int p = 0; p + 1 < P.P; p++) count += 2 * (1ull << P.lgM[p]);
   d.bytes = count * sizeof(fr);
   hipError_t e = hipMalloc((void**)&d.block, d.bytes);
@@ -190,6 +217,7 @@ hipError_t domain_build(Domain& d, int lg, hipStream_t s) {
   fr* cur = d.block;
   d.pw0 = cur; cur += 16384;
   d.pw1 = cur; cur += 16384;
+  d.dft = (uint32_t*)cur; cur += kRowsFr;
   d.inner_fwd = cur; cur += 256;
   d.inner_inv = cur; cur += 256;
   d.inner29_fwd = cur; cur += 256;
@@ -214,6 +242,8 @@ hipError_t domain_build(Domain& d, int lg, hipStream_t s) {
     hipLaunchKernelGGL(pow_direct_kernel, dim3(grid_for(16384, 256)), dim3(256), 0, s, d.pw1, (uint64_t)16384, b, 14u,
                        one);
   }
+  hipLaunchKernelGGL(dft_rows_kernel, dim3(1), dim3(64), 0, s, d.dft, to_dev(host::from_u64(1u << 29)),
+                     to_dev(host::inv(host::from_u64(2))), to_dev(host::inv(c32)));
   if ((e = fill_pow(d.inner_fwd, 256, 0, w256, nullptr, win, s)) != hipSuccess) goto done;
   if ((e = fill_pow(d.inner_inv, 256, 0, w256i, nullptr, win, s)) != hipSuccess) goto done;
   if ((e = fill_pow(d.inner29_fwd, 256, 0, w256, &c32, win, s)) != hipSuccess) goto done;
@@ -336,6 +366,7 @@ static void fill_pass_args(const Domain& d, const NttCall& c, int p, const fr* i
   memset(&a, 0, sizeof(a));
   a.inner = c.inverse ? d.inner_inv : d.inner_fwd;
   a.inner29 = c.inverse ? d.inner29_inv : d.inner29_fwd;
+  a.dft = d.dft + (c.inverse ? kDftFactors * kRowWords : 0);
   a.lgN = lg;
   a.lgI = c.lgI;
   a.pm_mask = c.pm_mask;

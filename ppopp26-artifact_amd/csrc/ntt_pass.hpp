@@ -24,8 +24,8 @@
 // exchange through LDS (16 KiB per workgroup in two rounds), then DFT_A over
 // rho1 (8/A per lane, in registers).  The tile holds C = 1024/M' adjacent
 // columns, so every global access moves C*32 >= 512 contiguous bytes.  The
-// in-register DFTs are radix-2 DIF networks whose twiddles (powers of w_16)
-// are compile-time constants read from SGPRs.  Between passes the data is
+// factors inside an in-register DFT are the same for all lanes and come as
+// pre-reduced rows in SGPRs (rows29, fr29.hpp).  Between passes the data is
 // held as pbd words (fr29.hpp), not reduced; the last pass writes canonical
 // values in [0, r).
 #pragma once
@@ -35,8 +35,8 @@
 namespace pl {
 
 // w_16^e and w_16^-e, e = 0..7, as w R' mod r (R' = 2^261) in balanced
-// digits (b_i in [-2^28, 2^28), sum b_i 2^(29 i)): the wave-uniform factor of
-// the radix-2^29 product (fr29.hpp)
+// digits (b_i in [-2^28, 2^28), sum b_i 2^(29 i)); domain_build derives the
+// in-register DFTs' factors (PassArgs::dft) from e = 2, 4, 6
 static __constant__ const uint32_t kW16b[2][8][9] = {
     {{0xffffffbau, 0x00000230u, 0xfcb61180u, 0x0a4e5c01u, 0x0ee8b1a2u, 0xf6e6aedfu, 0xf907f8bcu, 0x0853ddf8u, 0x004d043fu},
      {0x04056c96u, 0x0f64e4d8u, 0xfc1c7b56u, 0xfcbda468u, 0xf4e761dbu, 0xf28ae057u, 0xfd2f3145u, 0x0f463b6eu, 0x006dc1feu},
@@ -55,12 +55,6 @@ static __constant__ const uint32_t kW16b[2][8][9] = {
      {0xf7a20118u, 0xf0b66a14u, 0x06553e8au, 0xf01fbca8u, 0x014f2019u, 0x0cdb0e2bu, 0x0d733ac9u, 0xfcf2606bu, 0x00474763u},
      {0xfbfa936bu, 0xf09b1b20u, 0x037a846au, 0xfe8a6198u, 0x0898f361u, 0xf979247au, 0xf7f19ba3u, 0xfb1ef842u, 0x00062ba9u}}};
 
-template <bool INV>
-__device__ __forceinline__ void w16b(int e, uint32_t (&w)[9]) {
-#pragma unroll
-  for (int i = 0; i < 9; i++) w[i] = kW16b[INV ? 1 : 0][e][i];
-}
-
 // an ordering point for the eight limbs of v (no instruction)
 __device__ __forceinline__ void pin(fr& v) {
   asm volatile("" : "+v"(v.l[0]), "+v"(v.l[1]), "+v"(v.l[2]), "+v"(v.l[3]), "+v"(v.l[4]), "+v"(v.l[5]),
@@ -73,45 +67,73 @@ __host__ __device__ constexpr int brev(int v, int bits) {
   return r;
 }
 
-// Radix-2 DIF DFT of size 2^LOGB on x[OFF + i], natural order in,
-// bit-reversed order out: afterwards x[OFF + brev(k)] = X[k].  Elements are
-// signed-limb values (v9): sums and differences are limb-wise, and with every
-// input limb a balanced digit (|l| <= 2^28) each output limb is a signed sum
-// of at most 2^LOGB balanced digits or product digits (below 2^29), which
-// stays within 32 bits for LOGB <= 3 (the first term of every such sum enters
-// with a plus sign, so the extremes are 2^31 - 1 and -2^31).
-template <int LOGB, bool INV, int OFF, int NX>
-__device__ __forceinline__ void dft_dif(v9 (&x)[NX]) {
+// Factors of the in-register DFTs, in the order of their rows29 tables
+// (PassArgs::dft; 81 words each, D = 1): i = w_8^2, (w_8 + w_8^3) / 2 and
+// (w_8 - w_8^3) / 2 (inverse transforms: of w_8^-1).
+enum { kDftI = 0, kDftC1 = 1, kDftC2 = 2, kDftFactors = 3 };
+constexpr int kRowWords = 81;
+
+// DFT of size 2^LOGB (at most 8) on x[OFF + i], natural order in, bit-reversed
+// order out: afterwards x[OFF + brev(k)] = X[k].  The odd outputs of the DFT_8
+// need w d1 + w^3 d3 and w^3 d1 + w d3 (w = w_8): as A + B and A - B with
+// A = (w + w^3)/2 (d1 + d3), B = (w - w^3)/2 (d1 - d3) they take two products
+// where the radix-2 network takes three, four in all instead of five.  Every
+// factor is wave-uniform, so the products are rows29 (fr29.hpp) with one
+// Montgomery digit: about 107 VALU instructions against mont29's 196.
+// NTT 2^24: 1.64 -> 1.43 ms; 2^16: 46 -> 43.7 us (a lone wave per SIMD).
+//
+// Bounds, with input limbs balanced digits (|l| <= 2^28) of values within V:
+// d = x_i - x_(i+4) has |l| <= 2^29, the products' inputs |l| <= 2^30, and the
+// products' limbs lie in [0, 2^29).  y0, y4 = sums of eight digits, first sign
+// plus, so within [-2^31, 2^31); e0 +- i e1 within 2^30 + 2^29; f = d0 +- i d2
+// within [-2^29, 2^30), so y1 = f + A + B within [-2^29, 2^31) and the others
+// smaller.  Values: i d2 within 5.6 r, i e1, A, B within 10.2 r, so every
+// output is within max(8 V, 2 V + 26 r).
+template <int LOGB, int OFF, int NX>
+__device__ __forceinline__ void dft_dif(v9 (&x)[NX], uwords f) {
   static_assert(LOGB <= 3, "limb growth: at most three butterfly levels");
-  constexpr int B = 1 << LOGB;
-  static_for<0, LOGB>([&](auto st_) {
-    constexpr int st = decltype(st_)::value;
-    constexpr int h = B >> (st + 1);
-    static_for<0, (1 << st)>([&](auto blk_) {
-      constexpr int s = decltype(blk_)::value * 2 * h;
-      static_for<0, h>([&](auto i_) {
-        constexpr int i = decltype(i_)::value;
-        // one butterfly at a time: the empty asm statements order the
-        // butterflies, so the live set stays at the lane's elements plus one
-        // butterfly's temporaries
-        v9 a = x[OFF + s + i];
-        v9 b = x[OFF + s + i + h];
-        pin9(a);
-        pin9(b);
-        v9 sum = v9_add(a, b);
-        v9 d = v9_sub(a, b);
-        if constexpr (i != 0) {
-          uint32_t w[9];
-          w16b<INV>((i * 8) / h, w);
-          d = v9_mul<true, false, false>(d, w);
-        }
-        pin9(sum);
-        pin9(d);
-        x[OFF + s + i] = sum;
-        x[OFF + s + i + h] = d;
-      });
-    });
-  });
+  // one butterfly at a time: the empty asm statements order them, so the live
+  // set stays at the lane's elements plus one butterfly's temporaries
+  auto bfly = [](v9& a, v9& b) {
+    pin9(a);
+    pin9(b);
+    const v9 s = v9_add(a, b);
+    b = v9_sub(a, b);
+    a = s;
+    pin9(a);
+    pin9(b);
+  };
+  // x times factor e; n is the next product's
+  rows_cols g;
+  if constexpr (LOGB >= 2) g = rows29_open(f + kRowWords * kDftI, 0);
+  auto mul = [&](v9& a, int e, int n) {
+    a = v9_mul_rows<1, false>(a, f + kRowWords * e, g, f + kRowWords * n);
+    pin9(a);
+  };
+  if constexpr (LOGB == 1) {
+    bfly(x[OFF], x[OFF + 1]);
+  } else if constexpr (LOGB == 2) {
+    bfly(x[OFF], x[OFF + 2]);      // a0, d0
+    bfly(x[OFF + 1], x[OFF + 3]);  // a1, d1
+    mul(x[OFF + 3], kDftI, kDftI);  // i d1
+    bfly(x[OFF], x[OFF + 1]);      // y0, y2
+    bfly(x[OFF + 2], x[OFF + 3]);  // y1, y3
+  } else if constexpr (LOGB == 3) {
+    static_for<0, 4>([&](auto i_) { bfly(x[OFF + decltype(i_)::value], x[OFF + decltype(i_)::value + 4]); });
+    bfly(x[OFF], x[OFF + 2]);      // b0, e0
+    bfly(x[OFF + 1], x[OFF + 3]);  // b1, e1
+    bfly(x[OFF], x[OFF + 1]);      // y0, y4
+    mul(x[OFF + 3], kDftI, kDftI);  // i e1
+    bfly(x[OFF + 2], x[OFF + 3]);  // y2, y6
+    mul(x[OFF + 6], kDftI, kDftC1);  // i d2
+    bfly(x[OFF + 4], x[OFF + 6]);  // f+, f-
+    bfly(x[OFF + 5], x[OFF + 7]);  // d1 + d3, d1 - d3
+    mul(x[OFF + 5], kDftC1, kDftC2);  // A
+    mul(x[OFF + 7], kDftC2, kDftI);   // B
+    bfly(x[OFF + 5], x[OFF + 7]);  // A + B, A - B
+    bfly(x[OFF + 4], x[OFF + 5]);  // y1, y5
+    bfly(x[OFF + 6], x[OFF + 7]);  // y3, y7
+  }
 }
 
 struct PassArgs {
@@ -121,6 +143,7 @@ struct PassArgs {
   const fr* tw;         // !LAST: pass twiddles (pbd words of w R' mod r), index j + S*k within the sub-problem
   const fr* inner;      // w_256^e (or w_256^-e), e < 256, stored form (small-size kernel)
   const fr* inner29;    // the same as pbd words of w R' mod r (pass kernels)
+  const uint32_t* dft;  // rows29 tables of the in-register DFTs' factors (dft_dif)
   uint64_t in_pstride;  // element stride between input polys (0: shared input)
   uint64_t nlines;      // lines (columns) in this launch
   uint32_t pm_mask;
@@ -318,7 +341,8 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
       for (int i = 0; i < 9; i++) x[decltype(r2_)::value].l[i] = 0;
     });
   }
-  dft_dif<kLgPerT, INV, 0>(x);  // x[brev3(k2)] = sum_rho2 z[rho1 + A rho2] w8^(rho2 k2)
+  const uwords dft = (uwords)a.dft;
+  dft_dif<kLgPerT, 0>(x, dft);  // x[brev3(k2)] = sum_rho2 z[rho1 + A rho2] w8^(rho2 k2)
   if constexpr (LA > 0) {
     // k2 = 0 takes no twiddle: back to balanced digits of a small value, so
     // that DFT_A again starts from balanced digits (the products' outputs
@@ -399,7 +423,7 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
     asm volatile("" : "+v"(base));
   }
   if constexpr (LA > 0) {
-    static_for<0, F2>([&](auto f_) { dft_dif<LA, INV, decltype(f_)::value * A>(y); });
+    static_for<0, F2>([&](auto f_) { dft_dif<LA, decltype(f_)::value * A>(y, dft); });
   }
   // y[f*A + brev_LA(k1)] = Z[k2 + kPerT*k1], k2 = g*F2 + f
 

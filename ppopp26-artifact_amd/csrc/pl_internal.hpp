@@ -46,6 +46,7 @@ struct Domain {
   fr* inner_inv = nullptr;
   fr* inner29_fwd = nullptr;       // the same times 32 (pass kernels)
   fr* inner29_inv = nullptr;
+  uint32_t* dft = nullptr;         // rows29 tables of the in-register DFTs' factors, forward then inverse
   fr* block = nullptr;             // single allocation holding all tables
   size_t bytes = 0;
   host::fr64 n_inv;
