@@ -342,6 +342,29 @@ __device__ __forceinline__ void mont29_dev(const uint32_t* x, const uint32_t* w,
 // wave-uniform read-only words (loaded to SGPRs)
 typedef const __attribute__((address_space(4))) uint32_t* uwords;
 
+// (a w + b v) / 2^261 mod r: two per-lane products with one reduction, 234
+// multiply-adds where two mont29 take 306.  For |a_i|, |b_i| <= 2^29 and
+// balanced factor digits a column stays below 18 * 2^57 + 8 * 2^58 + 2^34 <
+// 2^62; the value is within (T - r, T], T = (a w + b v) / 2^261.  Output digits
+// balanced.
+__device__ __forceinline__ void dual29_dev(const uint32_t* a, const uint32_t* w, const uint32_t* b,
+                                           const uint32_t* v, uint32_t* t) {
+  uint32_t m[9];
+  uint64_t acc[18];
+  static_for<0, 17>([&](auto k_) {
+    constexpr int k = decltype(k_)::value;
+    Mont29Col<k, false, (k >= 10)>::run(acc[k], k ? acc[k ? k - 1 : 0] : 0, a, w, m);
+    Mac29Col<k>::run(acc[k], b, v);
+    const uint32_t lo = (uint32_t)acc[k];
+    if constexpr (k <= 8)
+      m[k] = lo & kMask29;
+    else
+      t[k - 9] = sext29(lo);
+  });
+  Mont29Col<17, false, true>::run(acc[17], acc[16], a, w, m);
+  t[8] = (uint32_t)acc[17];
+}
+
 // Three columns (27 words) of a rows29 factor, in SGPRs.  rows29_open's loads
 // are issued where it stands: the scheduling barrier lets vector and LDS
 // instructions pass but neither the scalar loads nor the column blocks, so

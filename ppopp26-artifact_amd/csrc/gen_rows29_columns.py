@@ -1,6 +1,7 @@
 #!/usr/bin/env python3
 """Writes rows29_columns.inc: the wave-uniform constant product of fr29.hpp
-(rows29) as one inline-asm block per column.
+(rows29) as one inline-asm block per column, and the column blocks that add a
+second product to mont29's (dual29).
 
 Column k (0..8) adds x_i * W_{i,k} for i = 0..8, the column's words w[i] held
 in SGPRs, and columns 1..7 + D subtract the D Montgomery digits' multiples of r
@@ -11,6 +12,8 @@ arithmetic shift right by 29, after adding 2^28 when RND says that the
 previous column's digit was taken balanced; the previous accumulator stays
 intact for that digit.  Block 7 + D is the last that adds terms; block 8 + D
 only closes it.
+
+Mac29Col<k> adds x_i * w_{k-i} (both per lane) to the accumulator of column k.
 
     python3 gen_rows29_columns.py > rows29_columns.inc
 """
@@ -61,6 +64,23 @@ def emit(k, d, rnd):
     print("};")
 
 
+def emit_mac(k):
+    lines, ins, nxt = [], [], 2
+    for i in range(max(0, k - 8), min(k, 8) + 1):
+        lines.append("v_mad_i64_i32 %%0, %%1, %%%d, %%%d, %%0" % (nxt, nxt + 1))
+        ins += ['"v"(x[%d])' % i, '"v"(w[%d])' % (k - i)]
+        nxt += 2
+    print("template <> struct Mac29Col<%d> {" % k)
+    print("  __device__ __forceinline__ static void run(uint64_t& acc, const uint32_t* x, const uint32_t* w) {")
+    print("    uint64_t d;")
+    print('    asm("%s"' % "\\n\\t".join(lines))
+    print('        : "+v"(acc), "=&s"(d)')
+    print("        : %s);" % ", ".join(ins))
+    print("    (void)d;")
+    print("  }")
+    print("};")
+
+
 def main():
     print("// Generated by gen_rows29_columns.py: one asm block per column of the")
     print("// wave-uniform constant product in fr29.hpp (see that script).")
@@ -70,6 +90,9 @@ def main():
             # only the output columns (digit k - 1 >= d) can be balanced
             for k in range(d + 1 if rnd else 0, 9 + d):
                 emit(k, d, rnd)
+    print("template <int K> struct Mac29Col;")
+    for k in range(17):
+        emit_mac(k)
 
 
 if __name__ == "__main__":

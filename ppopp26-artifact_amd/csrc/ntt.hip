@@ -185,10 +185,15 @@ static hipError_t fill_pow(fr* out, uint64_t n, uint32_t lgS, const host::fr64& 
                            fr* win, hipStream_t s) {
   fr one = to_dev(host::one());
   fr b = to_dev(base);
-  hipLaunchKernelGGL(pow_direct_kernel, dim3(grid_for(16384, 256)), dim3(256), 0, s, win, (uint64_t)16384, b, 0u, one);
-  hipLaunchKernelGGL(pow_direct_kernel, dim3(grid_for(16384, 256)), dim3(256), 0, s, win + 16384, (uint64_t)16384, b,
-                     14u, one);
   fr sc = scale ? to_dev(*scale) : one;
+  if (n <= 16384 && lgS == 0) {
+    hipLaunchKernelGGL(pow_direct_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, out, n, b, 0u, sc);
+    return hipGetLastError();
+  }
+  // exponents are below n: no more of the windows than they reach
+  const uint64_t n0 = n < 16384 ? n : 16384, n1 = (n + 16383) >> 14;
+  hipLaunchKernelGGL(pow_direct_kernel, dim3(grid_for(n0, 256)), dim3(256), 0, s, win, n0, b, 0u, one);
+  hipLaunchKernelGGL(pow_direct_kernel, dim3(grid_for(n1, 256)), dim3(256), 0, s, win + 16384, n1, b, 14u, one);
   hipLaunchKernelGGL(pow_window_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, out, n, (const fr*)win,
                      (const fr*)(win + 16384), lgS, sc, scale ? 1u : 0u);
   return hipGetLastError();
@@ -211,6 +216,8 @@ hipError_t domain_build(Domain& d, int lg, hipStream_t s) {
   constexpr size_t kRowsFr = (2 * kDftFactors * kRowWords * sizeof(uint32_t) + sizeof(fr) - 1) / sizeof(fr);
   size_t count = 4 * 256 + 2 * 16384 + kRowsFr;  // inner tables (both forms), w_N power windows, DFT factors
   for (int p = 0; p + 1 < P.P; p++) count += 2 * (1ull << P.lgM[p]);
+  const bool lane = lg >= 4 && lg <= kLaneMaxLg;
+  if (lane) count += kLaneFin + (1ull << lg);
   d.bytes = count * sizeof(fr);
   hipError_t e = hipMalloc((void**)&d.block, d.bytes);
   if (e != hipSuccess) return e;
@@ -225,6 +232,11 @@ hipError_t domain_build(Domain& d, int lg, hipStream_t s) {
   for (int p = 0; p + 1 < P.P; p++) {
     d.tw_fwd[p] = cur; cur += 1ull << P.lgM[p];
     d.tw_inv[p] = cur; cur += 1ull << P.lgM[p];
+  }
+  fr* lane_fin = nullptr;
+  if (lane) {
+    d.lane_lin = cur; cur += 1ull << lg;
+    lane_fin = d.block + count - kLaneFin;
   }
   fr* win = nullptr;
   e = hipMalloc((void**)&win, 2 * 16384 * sizeof(fr));
@@ -256,8 +268,14 @@ hipError_t domain_build(Domain& d, int lg, hipStream_t s) {
     // the inverse transform's 2^-lg rides on the first pass's twiddles
     if ((e = fill_pow(d.tw_inv[p], n, P.lgS[p], wi, p == 0 ? &n_inv32 : &c32, win, s)) != hipSuccess) goto done;
   }
+  if (lane) {
+    // from the windows of w_N above
+    hipLaunchKernelGGL(pow_window_kernel, dim3(grid_for(1ull << lg, 256)), dim3(256), 0, s, d.lane_lin, 1ull << lg,
+                       (const fr*)d.pw0, (const fr*)d.pw1, 0u, to_dev(c32), 1u);
+    if ((e = lane_tables(d, lane_fin, s)) != hipSuccess) goto done;
+  }
   {
-    // the pass kernels' tables (inner29_*, tw_*) are contiguous to the end
+    // the pass kernels' tables (inner29_*, tw_*, lane_lin) are contiguous to here
     const uint64_t n29 = (uint64_t)(cur - d.inner29_fwd);
     hipLaunchKernelGGL(pbd_kernel, dim3(grid_for(n29, 256)), dim3(256), 0, s, d.inner29_fwd, n29);
     if ((e = hipGetLastError()) != hipSuccess) goto done;
@@ -396,6 +414,13 @@ static void fill_pass_args(const Domain& d, const NttCall& c, int p, const fr* i
   }
 }
 
+// c.tmp = c.in times the factor table
+static void launch_premul(const Domain& d, const NttCall& c, hipStream_t s) {
+  const uint64_t total = (uint64_t)c.npoly << d.lg;
+  hipLaunchKernelGGL(premul_kernel, dim3(grid_for(total, 256)), dim3(256), 0, s, c.in, c.tmp, c.in_pstride, c.premul,
+                     c.pm_mask, (uint32_t)d.lg, total);
+}
+
 // Pass p of the plan.  Intermediate passes keep the in-place layout, so in
 // may equal out for them; the last pass writes natural order.
 hipError_t ntt_launch_one(const Domain& d, const NttCall& c, int p, const fr* in, uint64_t in_pstride,
@@ -407,9 +432,11 @@ hipError_t ntt_launch_one(const Domain& d, const NttCall& c, int p, const fr* in
     // scale the input into the scratch buffer first.  The scratch copy also
     // makes a shared-input call (in_pstride 0) safe when out aliases in.
     if (!c.tmp) return hipErrorInvalidValue;
-    uint64_t total = (uint64_t)c.npoly << lg;
-    hipLaunchKernelGGL(premul_kernel, dim3(grid_for(total, 256)), dim3(256), 0, s, in, c.tmp, in_pstride, premul,
-                       c.pm_mask, (uint32_t)lg, total);
+    NttCall m = c;
+    m.in = in;
+    m.in_pstride = in_pstride;
+    m.premul = premul;
+    launch_premul(d, m, s);
     in = c.tmp;
     in_pstride = 1ull << lg;
     premul = nullptr;
@@ -468,6 +495,18 @@ bool pass_args_regular(const Domain& d, const NttCall& c, int p, PassArgs& a) {
 hipError_t ntt_launch(const Domain& d, const NttCall& c, hipStream_t s) {
   const int np = d.plan.P == 0 ? 1 : d.plan.P;
   const uint64_t N = 1ull << d.lg;
+  if (lane_form(d, c)) {
+    NttCall l = c;
+    if (c.premul && d.lg <= kLaneOne) {
+      // one launch has no pass before the one that stores: scale first
+      if (!c.tmp) return hipErrorInvalidValue;
+      launch_premul(d, c, s);
+      l.in = c.tmp;
+      l.in_pstride = N;
+      l.premul = nullptr;
+    }
+    return lane_launch(d, l, s);
+  }
   for (int p = 0; p < np; p++) {
     const bool last = p == np - 1;
     hipError_t e = ntt_launch_one(d, c, p, p == 0 ? c.in : c.tmp, p == 0 ? c.in_pstride : N,

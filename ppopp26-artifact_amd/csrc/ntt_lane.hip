@@ -1,0 +1,292 @@
+// Small transforms: one element per lane.
+//
+// The pass kernels (ntt_pass.hpp) hold eight elements per lane, so a lane
+// works through some 23 products one after the other and a transform of 2^16
+// elements occupies 128 waves of the 1024 that the chip's SIMDs could each take;
+// below about 2^19 elements their time is that chain of products, not the
+// chip's rate.  Here a lane holds one element and a column of M' = 2^m points
+// (4 <= m <= 10) is one workgroup or part of one: m / 2 radix-4 steps (a
+// radix-2 step first when m is odd), each one exchange through LDS and one
+// product per lane.  A quad of lanes holds the four inputs x_q of a radix-4
+// step; lane k forms its output with the twiddle that follows,
+//
+//   z_k = t_k (x_0 + (-1)^k x_2) + t_k i^k (x_1 + (-1)^k x_3),
+//
+// the sums by quad permutes of the limbs (DPP) and the two products with one
+// reduction (dual29_dev, 234 multiply-adds): one chain of about 280 VALU
+// instructions per two stages, against 107-196 per product and 23 products per
+// six stages.  All factors come from one table of w_N^e, e < N, pbd words of
+// w R' mod r (inverse: index N - e); the last step of the last pass takes its
+// own four pairs, which carry 2^-lg for the inverse.
+//
+// lg <= kLaneOne: one launch.  Above: two, M'0 = 2^ceil(lg/2) columns at stride
+// N / M'0 into the caller's scratch as pbd words with the twiddle w_N^(J kappa),
+// then contiguous rows in natural order.  Against the pass kernels, one forward
+// transform: 2^9 24.6 -> 9.2 us, 2^12 30.3 -> 10.5, 2^14 42.0 -> 11.5, 2^16
+// 46.0 -> 14.5, 2^18 57.4 -> 43.2 (the caller's own launches take 7.4 of it).
+//
+// Bounds: inputs are balanced digits (|l| <= 2^28), so the sums have |l| <= 2^29;
+// values: a caller's 2^256 < 2.21 r makes the first sums 4.42 r each and the
+// step's result within (-1.126 r, 0.126 r), later steps within (-1.065 r,
+// 0.065 r) (x w / 2^261 < 0.01415 |x| for w < r), which fits a pbd word
+// (1.104 r).
+#include <type_traits>
+
+#include "ntt_pass.hpp"
+
+namespace pl {
+
+struct LaneArgs {
+  const fr* in;
+  fr* out;
+  const fr* premul;     // optional factor per input element [(poly & pm_mask) << lgN | pos], pbd words of c R'
+  const fr* lin;        // w_N^e, e < N, pbd words of w R'
+  const fr* fin;        // (s, s i^k), k < 4: s = 1, or 1/N for the inverse (pbd words times R')
+  uint64_t in_pstride;  // element stride between input polys (0: shared input)
+  uint64_t nlines;
+  uint32_t pm_mask;
+  uint32_t lgN;
+  uint32_t lgI;         // LAST: output interleave
+  uint32_t inverse;
+  uint32_t in_ext;      // caller data (any 256-bit values), not pbd words
+};
+
+// the limb of lane CTRL's choice within the quad
+template <int P0, int P1, int P2, int P3>
+__device__ __forceinline__ uint32_t quad(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, P0 | P1 << 2 | P2 << 4 | P3 << 6, 0xf, 0xf, true);
+}
+
+// log2 radix of step s and log2 size of its sub-problems, for 2^m points
+constexpr int lane_lr(int m, int s) { return (m & 1) && s == 0 ? 1 : 2; }
+constexpr int lane_mu(int m, int s) { return (m & 1) ? (s == 0 ? m : m - 1 - 2 * (s - 1)) : m - 2 * s; }
+
+// position in the column of the element that lane tau holds in a step of
+// radix 2^lr on sub-problems of 2^mu points: the radix's inputs are adjacent lanes
+__device__ __forceinline__ uint32_t lane_pos(uint32_t tau, int mu, int lr) {
+  const uint32_t q = tau & ((1u << lr) - 1), rest = tau >> lr;
+  const uint32_t j = rest & ((1u << (mu - lr)) - 1), sub = rest >> (mu - lr);
+  return (sub << mu) + (q << (mu - lr)) + j;
+}
+
+constexpr int lane_threads(int m) { return 1 << (m > 8 ? m : 8); }
+
+template <int m, bool LAST>
+__global__ void __launch_bounds__(lane_threads(m), 4) ntt_lane_kernel(LaneArgs a) {
+  constexpr int T = lane_threads(m);
+  constexpr int C = T >> m;  // columns per workgroup
+  constexpr int LGC = C == 1 ? 0 : 8 - m;
+  constexpr int NS = (m + 1) / 2;
+  constexpr bool DB = T <= 512;  // two exchange buffers: one barrier per step
+  __shared__ uint3 ex[DB ? 2 : 1][3][T];
+
+  const uint32_t tid = threadIdx.x;
+  const uint32_t c = (tid >> 2) & (C - 1);
+  const uint32_t tau = (tid & 3) | ((tid >> (2 + LGC)) << 2);
+  const uint32_t lg = a.lgN;
+  const uint32_t nmask = (1u << lg) - 1;
+  const uint32_t lgL = lg - m;  // log2 lines per polynomial
+  const uint64_t line_of = (uint64_t)blockIdx.x * C + c;
+  // lanes beyond the launch's lines work on its last line and store nothing
+  const uint64_t line = line_of < a.nlines ? line_of : a.nlines - 1;
+  uint64_t poly;
+  uint32_t lp;
+  if (LAST && a.lgI) {
+    poly = line & ((1ull << a.lgI) - 1);
+    lp = (uint32_t)(line >> a.lgI);
+  } else {
+    poly = line >> lgL;
+    lp = (uint32_t)(line & ((1ull << lgL) - 1));
+  }
+  auto lin = [&](uint32_t e) {  // w_N^(+-e)
+    return fr_load(a.lin + ((a.inverse ? 0u - e : e) & nmask));
+  };
+  // twiddles of step s for this lane, not those after the pass
+  auto twiddle = [&](auto s_, fr& w1, fr& w2) {
+    constexpr int s = decltype(s_)::value, mu = lane_mu(m, s), lr = lane_lr(m, s);
+    const uint32_t k = tau & ((1u << lr) - 1), j = (tau >> lr) & ((1u << (mu - lr)) - 1);
+    w1 = lin((j * k) << (lg - mu));
+    if constexpr (lr == 2) w2 = lin((k * (j + (1u << (mu - 2)))) << (lg - mu));
+  };
+
+  fr w1, w2;
+  twiddle(std::integral_constant<int, 0>(), w1, w2);
+  v9 x;
+  {
+    const uint32_t pos = lane_pos(tau, lane_mu(m, 0), lane_lr(m, 0));
+    const uint32_t at = LAST ? (lp << m) + pos : lp + (pos << lgL);
+    const fr raw = fr_load(a.in + poly * a.in_pstride + at);
+    if (a.in_ext) {
+      unpack_ext(raw.l, x.l);
+      if (!LAST && a.premul) {
+        uint32_t w[9];
+        pbd_unpack(fr_load(a.premul + (((poly & a.pm_mask) << lg) + at)).l, w);
+        x = v9_mul<false, false, true>(x, w);
+      }
+    } else {
+      pbd_unpack(raw.l, x.l);
+    }
+  }
+  // kappa, the output index of this lane's last element: its position's
+  // digits reversed
+  uint32_t kappa = 0;
+  {
+    const uint32_t pos = tau;  // lane_pos of the last step
+    int hi = m, sh = 0;
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      const int lr = lane_lr(m, s);
+      hi -= lr;
+      kappa |= ((pos >> hi) & ((1u << lr) - 1)) << sh;
+      sh += lr;
+    }
+  }
+  static_for<0, NS>([&](auto s_) {
+    constexpr int s = decltype(s_)::value, lr = lane_lr(m, s);
+    uint32_t f1[9], f2[9];
+    pbd_unpack(w1.l, f1);
+    if constexpr (lr == 2) pbd_unpack(w2.l, f2);
+    // the next step's factors, in flight during this step's product
+    if constexpr (s + 2 < NS) {
+      twiddle(std::integral_constant<int, s + 1>(), w1, w2);
+    } else if constexpr (s + 1 < NS) {
+      if constexpr (LAST) {
+        w1 = fr_load(a.fin + 2 * (tau & 3));
+        w2 = fr_load(a.fin + 2 * (tau & 3) + 1);
+      } else {
+        // w_N^(J kappa), and times i^k
+        w1 = lin(lp * kappa);
+        w2 = lin(lp * kappa + ((tau & 3) << (lg - 2)));
+      }
+    }
+    v9 u, v;
+    if constexpr (lr == 1) {
+      const uint32_t neg = 0u - (tau & 1);
+#pragma unroll
+      for (int i = 0; i < 9; i++) u.l[i] = quad<0, 0, 2, 2>(x.l[i]) + ((quad<1, 1, 3, 3>(x.l[i]) ^ neg) - neg);
+      x = v9_mul<false, false, true>(u, f1);
+    } else {
+      // lanes 0, 1: x_q + x_(q+2); lanes 2, 3: x_(q-2) - x_q
+      const uint32_t neg = 0u - ((tau >> 1) & 1);
+      uint32_t p[9];
+#pragma unroll
+      for (int i = 0; i < 9; i++) p[i] = quad<2, 3, 0, 1>(x.l[i]) + ((x.l[i] ^ neg) - neg);
+#pragma unroll
+      for (int i = 0; i < 9; i++) {
+        u.l[i] = quad<0, 2, 0, 2>(p[i]);
+        v.l[i] = quad<1, 3, 1, 3>(p[i]);
+      }
+      dual29_dev(u.l, f1, v.l, f2, x.l);
+    }
+    if constexpr (s + 1 < NS) {
+      const uint32_t wr = (c << m) + lane_pos(tau, lane_mu(m, s), lr);
+      const uint32_t rd = (c << m) + lane_pos(tau, lane_mu(m, s + 1), lane_lr(m, s + 1));
+      uint3(*const b)[T] = ex[DB ? s & 1 : 0];
+      if constexpr (!DB && s > 0) __syncthreads();  // the previous exchange's reads are done
+#pragma unroll
+      for (int h = 0; h < 3; h++) b[h][wr] = make_uint3(x.l[3 * h], x.l[3 * h + 1], x.l[3 * h + 2]);
+      __syncthreads();
+#pragma unroll
+      for (int h = 0; h < 3; h++) {
+        const uint3 g = b[h][rd];
+        x.l[3 * h] = g.x;
+        x.l[3 * h + 1] = g.y;
+        x.l[3 * h + 2] = g.z;
+      }
+    }
+  });
+  if (line_of >= a.nlines) return;
+  if constexpr (LAST) {
+    const uint32_t lgI = a.lgI;
+    fr* const dst = a.out + ((poly >> lgI) << (lg + lgI)) + (poly & ((1ull << lgI) - 1));
+    fr_store(dst + ((uint64_t)(lp + (kappa << lgL)) << lgI), v9_canonical(x));
+  } else {
+    fr o;
+    pbd_pack(x.l, o.l);
+    fr_store(a.out + (poly << lg) + lp + (kappa << lgL), o);
+  }
+}
+
+template <int m, bool LAST>
+static void launch_lane(const LaneArgs& a, hipStream_t s) {
+  constexpr int C = lane_threads(m) >> m;
+  hipLaunchKernelGGL((ntt_lane_kernel<m, LAST>), dim3((unsigned)((a.nlines + C - 1) / C)), dim3(lane_threads(m)), 0, s,
+                     a);
+}
+
+static void launch_lane_m(int m, bool last, const LaneArgs& a, hipStream_t s) {
+  switch (m) {
+    case 4: launch_lane<4, true>(a, s); break;
+    case 5: last ? launch_lane<5, true>(a, s) : launch_lane<5, false>(a, s); break;
+    case 6: last ? launch_lane<6, true>(a, s) : launch_lane<6, false>(a, s); break;
+    case 7: last ? launch_lane<7, true>(a, s) : launch_lane<7, false>(a, s); break;
+    case 8: last ? launch_lane<8, true>(a, s) : launch_lane<8, false>(a, s); break;
+    case 9: last ? launch_lane<9, true>(a, s) : launch_lane<9, false>(a, s); break;
+    default: last ? launch_lane<10, true>(a, s) : launch_lane<10, false>(a, s); break;
+  }
+}
+
+// fin[dir][k] = (s, s i^(+-k)) in the factors' form; ii[dir] = i^(+-1) = w_256^(+-64)
+__global__ void lane_fin_kernel(fr* fin, const fr* w256, const fr* w256i, fr c32, fr n_inv32) {
+  const int k = threadIdx.x & 3, dir = threadIdx.x >> 2;
+  if (threadIdx.x >= 8) return;
+  const fr s = dir ? n_inv32 : c32;
+  fr o;
+  to_pbd(s.l, o.l);
+  fr_store(fin + 8 * dir + 2 * k, o);
+  const fr v = fr_mul(s, fr_load((dir ? w256i : w256) + 64 * k));
+  to_pbd(v.l, o.l);
+  fr_store(fin + 8 * dir + 2 * k + 1, o);
+}
+
+hipError_t lane_tables(Domain& d, fr* fin, hipStream_t s) {
+  auto dev = [](const host::fr64& h) {
+    fr f;
+    memcpy(f.l, h.l, 32);
+    return f;
+  };
+  const host::fr64 c32 = host::from_u64(32);
+  d.lane_fin = fin;
+  hipLaunchKernelGGL(lane_fin_kernel, dim3(1), dim3(64), 0, s, fin, (const fr*)d.inner_fwd, (const fr*)d.inner_inv,
+                     dev(c32), dev(host::mul(d.n_inv, c32)));
+  return hipGetLastError();
+}
+
+bool lane_form(const Domain& d, const NttCall& c) {
+  return d.lane_lin && ((uint64_t)c.npoly << d.lg) <= kLaneMaxElems;
+}
+
+hipError_t lane_launch(const Domain& d, const NttCall& c, hipStream_t s) {
+  const int lg = d.lg;
+  const bool one = lg <= kLaneOne;
+  if (c.premul && one) return hipErrorInvalidValue;  // the caller multiplies first
+  LaneArgs a;
+  memset(&a, 0, sizeof(a));
+  a.lin = d.lane_lin;
+  a.fin = d.lane_fin + (c.inverse ? 8 : 0);
+  a.lgN = lg;
+  a.lgI = c.lgI;
+  a.inverse = c.inverse;
+  a.in = c.in;
+  a.in_pstride = c.in_pstride;
+  a.in_ext = 1;
+  a.pm_mask = c.pm_mask;
+  const int m0 = one ? lg : (lg + 1) / 2, m1 = lg - m0;
+  if (!one) {
+    if (!c.tmp) return hipErrorInvalidValue;
+    a.premul = c.premul;
+    a.out = c.tmp;
+    a.nlines = (uint64_t)c.npoly << (lg - m0);
+    launch_lane_m(m0, false, a, s);
+    a.premul = nullptr;
+    a.in = c.tmp;
+    a.in_pstride = 1ull << lg;
+    a.in_ext = 0;
+  }
+  a.out = c.out;
+  a.nlines = one ? c.npoly : (uint64_t)c.npoly << (lg - m1);
+  launch_lane_m(one ? m0 : m1, true, a, s);
+  return hipGetLastError();
+}
+
+}  // namespace pl

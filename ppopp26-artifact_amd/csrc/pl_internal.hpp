@@ -46,6 +46,10 @@ struct Domain {
   fr* inner_inv = nullptr;
   fr* inner29_fwd = nullptr;       // the same times 32 (pass kernels)
   fr* inner29_inv = nullptr;
+  // small transforms (ntt_lane.hip), null above kLaneMaxLg: w_N^e, e < N, and
+  // the last step's factor pairs (forward, inverse), pbd words of w R'
+  fr* lane_lin = nullptr;
+  fr* lane_fin = nullptr;
   uint32_t* dft = nullptr;         // rows29 tables of the in-register DFTs' factors, forward then inverse
   fr* block = nullptr;             // single allocation holding all tables
   size_t bytes = 0;
@@ -86,6 +90,19 @@ struct NttCall {
   uint32_t lgI = 0;            // output interleave: out[(pos << lgI) + (poly & (2^lgI-1))]
   bool inverse = false;
 };
+
+// The one-element-per-lane form: whole transforms of 2^4 .. 2^kLaneMaxLg points
+// whose call has at most kLaneMaxElems elements in all; one launch up to
+// 2^kLaneOne points, where a column still fits one CU well (us per call, one
+// transform: 2^9 in one launch 9.2, 2^10 in one 16.4 and in two 10.3).  At
+// 2^19 elements in all it takes 85 us against the pass kernels' 95; above,
+// their eight elements per lane fill the chip and need half the instructions.
+constexpr int kLaneMaxLg = 19, kLaneOne = 9;
+constexpr uint64_t kLaneMaxElems = 1ull << 19;
+constexpr int kLaneFin = 16;  // elements of the factor pairs
+hipError_t lane_tables(Domain& d, fr* fin, hipStream_t s);
+bool lane_form(const Domain& d, const NttCall& c);
+hipError_t lane_launch(const Domain& d, const NttCall& c, hipStream_t s);
 
 hipError_t ntt_launch(const Domain& d, const NttCall& c, hipStream_t s);
 hipError_t ntt_launch_one(const Domain& d, const NttCall& c, int p, const fr* in, uint64_t in_pstride,
