@@ -260,8 +260,8 @@ int pl_div_linear(void* d_inout, uint64_t n, const void* d_c, void* d_rem, void*
  *  ntt.cu:1494-1500, lde.cu:1834-1846)
  * A size-2^lg transform runs as P passes of 2^m[p]-point columns (3 <= m <= 6,
  * sum = lg); every split gives the same exact result.  (Whole transforms of at
- * most 2^19 elements in all do not use the split: they run as one or two
- * launches with one element per lane.)  pl_autotune times the
+ * most 2^18 elements in all, and some up to 2^19, do not use the split: they
+ * run as one or two launches with one element per lane.)  pl_autotune times the
  * candidate splits of each lg in [lg_lo, lg_hi] on the current device (a
  * batch of max(1, 2^22 / N) polynomials per call), keeps the fastest and
  * records the choices in cache_path ("<lg> <P> <m0..> <ms>" lines); sizes

@@ -91,8 +91,8 @@ static hipError_t ntt_host(const Domain& d, const fr* h_in, fr* h_out, uint32_t 
   const bool grouped = P.P >= 2;
   const int m0 = grouped ? P.m[0] : 0, mL = grouped ? P.m[P.P - 1] : 0;
   const uint64_t S0 = N >> m0, L = N >> mL;
-  const uint64_t G0 = grouped ? pow2_groups(lg_k, S0, kTile >> m0) : 1;
-  const uint64_t G1 = grouped ? pow2_groups(lg_k, L, kTile >> mL) : 1;
+  const uint64_t G0 = grouped ? pow2_groups(lg_k, S0, kLines) : 1;
+  const uint64_t G1 = grouped ? pow2_groups(lg_k, L, kLines) : 1;
   const uint64_t W0 = S0 / G0, W1 = L / G1;
   std::vector<hipEvent_t> ev_in(G0), ev_out(G1);
   for (auto& v : ev_in)

@@ -87,13 +87,15 @@ __global__ void pbd_kernel(fr* t, uint64_t n) {
   fr_store(t + i, o);
 }
 
-// rows29 tables (fr29.hpp) of the in-register DFTs' factors (ntt_pass.hpp
-// kDftI ..), forward then inverse: one thread per row of a table.  c29, half
-// and inv32 are 2^29, 1/2 and 1/32 in stored form.
-__global__ void dft_rows_kernel(uint32_t* out, fr c29, fr half, fr inv32) {
-  const int t = threadIdx.x;
-  if (t >= 2 * kDftFactors * 9) return;
-  const int i = t % 9, e = t / 9 % kDftFactors, dir = t / (9 * kDftFactors);
+// rows29 tables (fr29.hpp) of the pass kernels' wave-uniform factors
+// (ntt_pass.hpp kDftI .. kInner), forward then inverse: one thread per row of a
+// table.  c29, half and inv32 are 2^29, 1/2 and 1/32 in stored form; w256 and
+// w256i the inner tables (w_256^+-e).
+__global__ void __launch_bounds__(256)
+    rows_kernel(uint32_t* out, const fr* w256, const fr* w256i, fr c29, fr half, fr inv32) {
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= 2 * kRowFactors * 9) return;
+  const int i = t % 9, e = t / 9 % kRowFactors, dir = t / (9 * kRowFactors);
   auto root = [&](int k) {  // w_16^(+-k), stored form
     uint32_t d[9];
     reduce_below_2r(kW16b[dir][k], d);
@@ -101,16 +103,22 @@ __global__ void dft_rows_kernel(uint32_t* out, fr c29, fr half, fr inv32) {
     join29(d, v.l);
     return fr_mul(fr_reduce_once(v), inv32);
   };
-  fr w = root(4);
-  if (e != kDftI) {
+  fr w;
+  int D = 1;
+  if (e == kDftI) {
+    w = root(4);
+  } else if (e < kInner) {
     const fr a = root(2), b = root(6);
     w = fr_mul(e == kDftC1 ? fr_add(a, b) : fr_sub(a, b), half);
+  } else {
+    w = fr_load((dir ? w256i : w256) + 4 * (e - kInner));
+    D = 2;
   }
-  for (int k = 0; k < i + 1; k++) w = fr_mul(w, c29);  // D = 1
+  for (int k = 0; k < i + D; k++) w = fr_mul(w, c29);
   fr plain = fr_zero();
   plain.l[0] = 1;
   w = fr_mul(w, plain);  // the row as a plain integer below r
-  rows29_row(w.l, i, out + (dir * kDftFactors + e) * kRowWords);
+  rows29_row(w.l, i, out + (dir * kRowFactors + e) * kRowWords);
 }
 
 static inline fr to_dev(const host::fr64& h) {
@@ -213,8 +221,8 @@ hipError_t domain_build(Domain& d, int lg, hipStream_t s) {
   d.lg = lg;
   d.plan = make_plan(lg);
   const NttPlan& P = d.plan;
-  constexpr size_t kRowsFr = (2 * kDftFactors * kRowWords * sizeof(uint32_t) + sizeof(fr) - 1) / sizeof(fr);
-  size_t count = 4 * 256 + 2 * 16384 + kRowsFr;  // inner tables (both forms), w_N power windows, DFT factors
+  constexpr size_t kRowsFr = (2 * kRowFactors * kRowWords * sizeof(uint32_t) + sizeof(fr) - 1) / sizeof(fr);
+  size_t count = 2 * 256 + 2 * 16384 + kRowsFr;  // inner tables, w_N power windows, wave-uniform factors
   for (int p = 0; p + 1 < P.P; p++) count += 2 * (1ull << P.lgM[p]);
   const bool lane = lg >= 4 && lg <= kLaneMaxLg;
   if (lane) count += kLaneFin + (1ull << lg);
@@ -224,11 +232,10 @@ hipError_t domain_build(Domain& d, int lg, hipStream_t s) {
   fr* cur = d.block;
   d.pw0 = cur; cur += 16384;
   d.pw1 = cur; cur += 16384;
-  d.dft = (uint32_t*)cur; cur += kRowsFr;
+  d.rows = (uint32_t*)cur; cur += kRowsFr;
   d.inner_fwd = cur; cur += 256;
   d.inner_inv = cur; cur += 256;
-  d.inner29_fwd = cur; cur += 256;
-  d.inner29_inv = cur; cur += 256;
+  fr* const tw = cur;
   for (int p = 0; p + 1 < P.P; p++) {
     d.tw_fwd[p] = cur; cur += 1ull << P.lgM[p];
     d.tw_inv[p] = cur; cur += 1ull << P.lgM[p];
@@ -254,12 +261,11 @@ hipError_t domain_build(Domain& d, int lg, hipStream_t s) {
     hipLaunchKernelGGL(pow_direct_kernel, dim3(grid_for(16384, 256)), dim3(256), 0, s, d.pw1, (uint64_t)16384, b, 14u,
                        one);
   }
-  hipLaunchKernelGGL(dft_rows_kernel, dim3(1), dim3(64), 0, s, d.dft, to_dev(host::from_u64(1u << 29)),
-                     to_dev(host::inv(host::from_u64(2))), to_dev(host::inv(c32)));
   if ((e = fill_pow(d.inner_fwd, 256, 0, w256, nullptr, win, s)) != hipSuccess) goto done;
   if ((e = fill_pow(d.inner_inv, 256, 0, w256i, nullptr, win, s)) != hipSuccess) goto done;
-  if ((e = fill_pow(d.inner29_fwd, 256, 0, w256, &c32, win, s)) != hipSuccess) goto done;
-  if ((e = fill_pow(d.inner29_inv, 256, 0, w256i, &c32, win, s)) != hipSuccess) goto done;
+  hipLaunchKernelGGL(rows_kernel, dim3(grid_for(2 * kRowFactors * 9, 256)), dim3(256), 0, s, d.rows,
+                     (const fr*)d.inner_fwd, (const fr*)d.inner_inv, to_dev(host::from_u64(1u << 29)),
+                     to_dev(host::inv(host::from_u64(2))), to_dev(host::inv(c32)));
   for (int p = 0; p + 1 < P.P; p++) {
     host::fr64 w = host::root_of_unity(P.lgM[p]);
     host::fr64 wi = host::inv(w);
@@ -274,12 +280,12 @@ hipError_t domain_build(Domain& d, int lg, hipStream_t s) {
                        (const fr*)d.pw0, (const fr*)d.pw1, 0u, to_dev(c32), 1u);
     if ((e = lane_tables(d, lane_fin, s)) != hipSuccess) goto done;
   }
-  {
-    // the pass kernels' tables (inner29_*, tw_*, lane_lin) are contiguous to here
-    const uint64_t n29 = (uint64_t)(cur - d.inner29_fwd);
-    hipLaunchKernelGGL(pbd_kernel, dim3(grid_for(n29, 256)), dim3(256), 0, s, d.inner29_fwd, n29);
-    if ((e = hipGetLastError()) != hipSuccess) goto done;
+  if (cur > tw) {
+    // the pass kernels' factor tables (tw_*, lane_lin) are contiguous to here
+    const uint64_t n29 = (uint64_t)(cur - tw);
+    hipLaunchKernelGGL(pbd_kernel, dim3(grid_for(n29, 256)), dim3(256), 0, s, tw, n29);
   }
+  if ((e = hipGetLastError()) != hipSuccess) goto done;
   e = hipStreamSynchronize(s);
 done:
   (void)hipFree(win);
@@ -383,8 +389,7 @@ static void fill_pass_args(const Domain& d, const NttCall& c, int p, const fr* i
   const int lg = d.lg;
   memset(&a, 0, sizeof(a));
   a.inner = c.inverse ? d.inner_inv : d.inner_fwd;
-  a.inner29 = c.inverse ? d.inner29_inv : d.inner29_fwd;
-  a.dft = d.dft + (c.inverse ? kDftFactors * kRowWords : 0);
+  a.rows = d.rows + (c.inverse ? kRowFactors * kRowWords : 0);
   a.lgN = lg;
   a.lgI = c.lgI;
   a.pm_mask = c.pm_mask;

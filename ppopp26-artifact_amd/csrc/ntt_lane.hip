@@ -3,7 +3,7 @@
 // The pass kernels (ntt_pass.hpp) hold eight elements per lane, so a lane
 // works through some 23 products one after the other and a transform of 2^16
 // elements occupies 128 waves of the 1024 that the chip's SIMDs could each take;
-// below about 2^19 elements their time is that chain of products, not the
+// below about 2^18 elements their time is that chain of products, not the
 // chip's rate.  Here a lane holds one element and a column of M' = 2^m points
 // (4 <= m <= 10) is one workgroup or part of one: m / 2 radix-4 steps (a
 // radix-2 step first when m is odd), each one exchange through LDS and one
@@ -253,7 +253,8 @@ hipError_t lane_tables(Domain& d, fr* fin, hipStream_t s) {
 }
 
 bool lane_form(const Domain& d, const NttCall& c) {
-  return d.lane_lin && ((uint64_t)c.npoly << d.lg) <= kLaneMaxElems;
+  const uint64_t n = (uint64_t)c.npoly << d.lg;
+  return d.lane_lin && (n <= 1ull << 18 || (d.lg > 12 && n < 1ull << 19));
 }
 
 hipError_t lane_launch(const Domain& d, const NttCall& c, hipStream_t s) {

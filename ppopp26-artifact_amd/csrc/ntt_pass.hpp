@@ -16,18 +16,26 @@
 // (ntt.cu:979-1037; ntt_kernel/algorithm.cuh:8-59; ct_mixed_radix_wide.cuh:47-189)
 // with the same mathematical result.
 //
-// Workgroup: 128 lanes own a tile of 1024 elements (8 per lane, all in
-// VGPRs, about 110-128 VGPRs per lane, so four waves share each SIMD: one
-// wave alone cannot issue multiply-adds back to back, and four reach ~15 %
-// more than two).  A column of M' = 8*A points is computed as DFT_8 over
-// rho2 (one per lane, in registers), an inner twiddle w_M'^(rho1 k2), one
-// exchange through LDS (16 KiB per workgroup in two rounds), then DFT_A over
-// rho1 (8/A per lane, in registers).  The tile holds C = 1024/M' adjacent
-// columns, so every global access moves C*32 >= 512 contiguous bytes.  The
-// factors inside an in-register DFT are the same for all lanes and come as
-// pre-reduced rows in SGPRs (rows29, fr29.hpp).  Between passes the data is
-// held as pbd words (fr29.hpp), not reduced; the last pass writes canonical
-// values in [0, r).
+// Workgroup: A waves own a tile of 64 adjacent columns of M' = 8 A points,
+// one column per lane, 8 elements of it in VGPRs (about 110-128 VGPRs per
+// lane, so four waves share each SIMD: one wave alone cannot issue
+// multiply-adds back to back, and four reach ~15 % more than two).  A column
+// is computed as DFT_8 over rho2 (wave rho1), an inner twiddle
+// w_M'^(rho1 k2), one exchange through LDS (48 KiB per workgroup for A = 8,
+// in three rounds), then DFT_A over rho1 (wave k2).  With one column per lane
+// everything that varies inside a column is the same for the whole wave: the
+// factors inside the DFTs and the inner twiddles come as pre-reduced rows in
+// SGPRs (rows29, fr29.hpp), 107-117 VALU instructions per product instead of
+// 196 and an unpack (13 x iNTT 2^15: 67.6 -> 56.5 us; proof batch of 2^12 ..
+// 2^20: 2.98 -> 2.64 ms; the per-lane twiddles of a 16-column tile of two
+// waves before).  Longer tiles leave two workgroups of eight waves on a CU,
+// so loads and stores hide less behind the other's products than with eight
+// of two: 2^24, a middle pass, 534 VALU instructions per element (0.28 ms
+// at the multiply-add probe's rate) in 0.33 ms, where 757 took 0.42.
+// Global accesses move 64 * 32 contiguous bytes, except the last pass's
+// loads, where a lane reads its own sub-row and the waves of a workgroup use
+// up each line between them.  Between passes the data is held as pbd words
+// (fr29.hpp), not reduced; the last pass writes canonical values in [0, r).
 #pragma once
 #include "fr29.hpp"
 #include "pl_internal.hpp"
@@ -36,7 +44,7 @@ namespace pl {
 
 // w_16^e and w_16^-e, e = 0..7, as w R' mod r (R' = 2^261) in balanced
 // digits (b_i in [-2^28, 2^28), sum b_i 2^(29 i)); domain_build derives the
-// in-register DFTs' factors (PassArgs::dft) from e = 2, 4, 6
+// in-register DFTs' factors (PassArgs::rows) from e = 2, 4, 6
 static __constant__ const uint32_t kW16b[2][8][9] = {
     {{0xffffffbau, 0x00000230u, 0xfcb61180u, 0x0a4e5c01u, 0x0ee8b1a2u, 0xf6e6aedfu, 0xf907f8bcu, 0x0853ddf8u, 0x004d043fu},
      {0x04056c96u, 0x0f64e4d8u, 0xfc1c7b56u, 0xfcbda468u, 0xf4e761dbu, 0xf28ae057u, 0xfd2f3145u, 0x0f463b6eu, 0x006dc1feu},
@@ -67,10 +75,11 @@ __host__ __device__ constexpr int brev(int v, int bits) {
   return r;
 }
 
-// Factors of the in-register DFTs, in the order of their rows29 tables
-// (PassArgs::dft; 81 words each, D = 1): i = w_8^2, (w_8 + w_8^3) / 2 and
-// (w_8 - w_8^3) / 2 (inverse transforms: of w_8^-1).
-enum { kDftI = 0, kDftC1 = 1, kDftC2 = 2, kDftFactors = 3 };
+// The pass kernels' wave-uniform factors, as rows29 tables of 81 words each
+// (PassArgs::rows): i = w_8^2, (w_8 + w_8^3) / 2 and (w_8 - w_8^3) / 2 for the
+// in-register DFTs (D = 1), then w_64^e, e < 64, for the inner twiddles
+// (D = 2); inverse transforms: of w_8^-1 and w_64^-1.
+enum { kDftI = 0, kDftC1 = 1, kDftC2 = 2, kInner = 3, kRowFactors = 3 + 64 };
 constexpr int kRowWords = 81;
 
 // DFT of size 2^LOGB (at most 8) on x[OFF + i], natural order in, bit-reversed
@@ -142,8 +151,7 @@ struct PassArgs {
   const fr* premul;     // !LAST: optional factor per input element [(poly & pm_mask) << lgN | pos], pbd words of c R''
   const fr* tw;         // !LAST: pass twiddles (pbd words of w R' mod r), index j + S*k within the sub-problem
   const fr* inner;      // w_256^e (or w_256^-e), e < 256, stored form (small-size kernel)
-  const fr* inner29;    // the same as pbd words of w R' mod r (pass kernels)
-  const uint32_t* dft;  // rows29 tables of the in-register DFTs' factors (dft_dif)
+  const uint32_t* rows; // rows29 tables of the wave-uniform factors (pass kernels)
   uint64_t in_pstride;  // element stride between input polys (0: shared input)
   uint64_t nlines;      // lines (columns) in this launch
   uint32_t pm_mask;
@@ -159,32 +167,16 @@ struct PassArgs {
   fr scale29;           // pbd word of scale R' mod r (pass kernels)
 };
 
-// Tile geometry (compile-time; see the file header):
-//   PL_NTT_LGPER   log2 elements per lane (3: 8 elements, DFT_8 in registers)
-//   PL_NTT_LGTILE  log2 elements per workgroup tile (128 lanes x 8)
-//   PL_NTT_PHASES  LDS exchange rounds (9/PHASES limbs each)
-//   PL_NTT_WAVES   waves per SIMD the register allocation must allow
-// Passes have 2^m-point columns, m = PL_NTT_LGPER + LA, LA <= min(4, LGPER).
-#ifndef PL_NTT_LGTILE
-#define PL_NTT_LGTILE 10
-#endif
-#ifndef PL_NTT_LGPER
-#define PL_NTT_LGPER 3
-#endif
-constexpr int kLgPerT = PL_NTT_LGPER;
+// Tile geometry (see the file header): passes have 2^m-point columns,
+// m = kLgPerT + LA, LA <= kLgPerT.
+constexpr int kLgPerT = 3;           // log2 elements per lane
 constexpr int kPerT = 1 << kLgPerT;
-constexpr int kPmG = kPerT / 4;  // factor-table loads in flight per group (first pass of an LDE)
-#ifndef PL_NTT_PHASES
-#define PL_NTT_PHASES 3
-#endif
-#ifndef PL_NTT_WAVES
-#define PL_NTT_WAVES 4
-#endif
-constexpr int kLgTile = PL_NTT_LGTILE;
-constexpr int kTile = 1 << kLgTile;
-constexpr int kThreads = kTile / kPerT;
-constexpr int kPhases = PL_NTT_PHASES;
-constexpr int kW = 9 / kPhases;  // limbs per exchange round
+constexpr int kPmG = kPerT / 4;      // factor-table loads in flight per group (first pass of an LDE)
+constexpr int kLgLines = 6;          // log2 columns per workgroup, one per lane
+constexpr int kLines = 1 << kLgLines;
+constexpr int kWavesPerSimd = 4;     // that the register allocation must allow
+constexpr int kPhases = 3;           // LDS exchange rounds
+constexpr int kW = 9 / kPhases;      // limbs per exchange round
 static_assert(kW * kPhases == 9, "the exchange rounds cover the nine limbs");
 
 template <int W> struct lds_vec;
@@ -228,65 +220,104 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
   static_assert(!SCALE || LAST, "the scale factor is applied by the last pass");
   constexpr int A = 1 << LA;
   constexpr int m = LA + kLgPerT;
-  constexpr int LGC = kLgTile - m;  // log2 lines per tile
-  constexpr int C = 1 << LGC;
-  constexpr int F2 = kPerT / A;   // DFT_A groups per thread in sub-step 2
+  constexpr int F2 = kPerT / A;   // DFT_A groups per lane in sub-step 2
   typedef typename lds_vec<kW>::type vec;
-  __shared__ vec lds[kTile];  // kW limbs of every tile element
+  // kW limbs of every tile element (the exchange), and in the last pass first
+  // 16 bytes of every element (the loads)
+  constexpr size_t kLdsBytes = LAST ? (size_t)16 << (kLgLines + m) : LA > 0 ? sizeof(vec) << (kLgLines + m) : 16;
+  __shared__ uint4 lds_raw[kLdsBytes / 16];
+  vec* const lds = (vec*)lds_raw;
 
-  const int t = threadIdx.x;
-  const uint64_t line0 = blk << LGC;
+  const int lc = threadIdx.x & (kLines - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> kLgLines);
+  const uint64_t line_of = (blk << kLgLines) + lc;
   const uint32_t lgL = a.lgN - m;  // log2 lines per polynomial = log2(N / M')
+  const uwords rows = (uwords)a.rows;
 
   // ---- sub-step 1: kPerT points of one (line, rho1), DFT over rho2 ----------
-  // rho = rho1 + A*rho2.  Intermediate passes map lanes to adjacent columns
-  // (coalesced strided rows); the last pass reads contiguous sub-rows, so
-  // lanes take adjacent rho1.
-  int lc, rho1;
-  if (LAST) {
-    rho1 = t & (A - 1);
-    lc = t >> LA;
-  } else {
-    lc = t & (C - 1);
-    rho1 = t >> LGC;
-  }
-  const uint64_t line = line0 + lc;
+  // rho = rho1 + A*rho2
+  const int rho1 = wv;
   v9 x[kPerT];
-  if (line < a.nlines) {
-    uint64_t poly, pos0, estride;
-    if (LAST) {
-      uint64_t lp;
-      if (a.lgI) {
-        poly = line & ((1ull << a.lgI) - 1);
-        lp = line >> a.lgI;
-      } else {
-        poly = line >> lgL;
-        lp = line & ((1ull << lgL) - 1);
-      }
-      // the sub-problem whose outputs land at lp + (N/M')*k: undo the digit
-      // reversal lp = d1 + M1*(d2 + M2*(...)) -> r = (((d1)*M2 + d2)*M3 + ...)
-      uint64_t r = 0, q = lp;
-      for (uint32_t p = 0; p < a.ndig; p++) {
-        uint32_t lr = a.lgrad[p];
-        r = (r << lr) | (q & ((1ull << lr) - 1));
-        q >>= lr;
-      }
-      pos0 = r << m;
-      estride = 1;
+  // lanes beyond the launch's lines load its last line and store nothing
+  const uint64_t line = line_of < a.nlines ? line_of : a.nlines - 1;
+  if constexpr (LAST) {
+    uint64_t poly, lp;
+    if (a.lgI) {
+      poly = line & ((1ull << a.lgI) - 1);
+      lp = line >> a.lgI;
     } else {
       poly = line >> lgL;
-      uint64_t lp = line & ((1ull << lgL) - 1);
-      uint64_t j = lp & ((1ull << a.lgS) - 1);
-      uint64_t rr = lp >> a.lgS;
-      pos0 = (rr << a.lgMp) + j;
-      estride = 1ull << a.lgS;
+      lp = line & ((1ull << lgL) - 1);
     }
+    // the sub-problem whose outputs land at lp + (N/M')*k: undo the digit
+    // reversal lp = d1 + M1*(d2 + M2*(...)) -> r = (((d1)*M2 + d2)*M3 + ...)
+    uint64_t r = 0, q = lp;
+    for (uint32_t p = 0; p < a.ndig; p++) {
+      uint32_t lr = a.lgrad[p];
+      r = (r << lr) | (q & ((1ull << lr) - 1));
+      q >>= lr;
+    }
+    const uint64_t base = (uint64_t)(a.in + poly * a.in_pstride + (r << m));
+    // Adjacent lines are far-apart sub-rows (their first digit differs), so a
+    // lane reading its own line would touch 64 pages with every load.  The
+    // waves read whole sub-rows instead (lane = element, line uniform for
+    // A = 8) and the raw words change hands through LDS, one 16-byte half at a
+    // time (64 KiB for A = 8); the XOR keeps both sides free of bank
+    // conflicts.  Last pass of 2^24:
+    // 0.333 -> 0.291 ms.
+    uint4 raw[kPerT][2];
+    const int i1 = lc & ((1 << m) - 1);
+    static_for<0, kPerT>([&](auto q_) {
+      constexpr int q = decltype(q_)::value;
+      const int ll = LA == 3 ? wv * kPerT + q : (((wv * kPerT + q) << kLgLines) + lc) >> m;
+      uint32_t lo, hi;
+      if constexpr (LA == 3) {
+        lo = __builtin_amdgcn_readlane((uint32_t)base, ll);
+        hi = __builtin_amdgcn_readlane((uint32_t)(base >> 32), ll);
+      } else {
+        lo = __builtin_amdgcn_ds_bpermute(4 * ll, (uint32_t)base);
+        hi = __builtin_amdgcn_ds_bpermute(4 * ll, (uint32_t)(base >> 32));
+      }
+      const uint4* src = (const uint4*)(((uint64_t)hi << 32) | lo) + 2 * i1;
+      raw[q][0] = src[0];
+      raw[q][1] = src[1];
+    });
+    static_for<0, 2>([&](auto h_) {
+      constexpr int h = decltype(h_)::value;
+      if constexpr (h > 0) __syncthreads();
+      static_for<0, kPerT>([&](auto q_) {
+        constexpr int q = decltype(q_)::value;
+        const int ll = (((wv * kPerT + q) << kLgLines) + lc) >> m;
+        lds_raw[(i1 << kLgLines) + (ll ^ (i1 & (kLines - 1)))] = raw[q][h];
+      });
+      __syncthreads();
+      static_for<0, kPerT>([&](auto r2_) {
+        constexpr int r2 = decltype(r2_)::value;
+        const int i = rho1 + A * r2;
+        raw[r2][h] = lds_raw[(i << kLgLines) + (lc ^ (i & (kLines - 1)))];
+      });
+    });
+    if constexpr (LA > 0) __syncthreads();  // before the exchange below reuses the buffer
+    static_for<0, kPerT>([&](auto r2_) {
+      constexpr int r2 = decltype(r2_)::value;
+      const uint4 l = raw[r2][0], u = raw[r2][1];
+      const uint32_t w[8] = {l.x, l.y, l.z, l.w, u.x, u.y, u.z, u.w};
+      if (a.in_ext) unpack_ext(w, x[r2].l);
+      else pbd_unpack(w, x[r2].l);
+    });
+  } else {
+    const uint64_t poly = line >> lgL;
+    const uint64_t lp = line & ((1ull << lgL) - 1);
+    const uint64_t j = lp & ((1ull << a.lgS) - 1);
+    const uint64_t rr = lp >> a.lgS;
+    const uint64_t pos0 = (rr << a.lgMp) + j;
+    const uint64_t estride = 1ull << a.lgS;
     const fr* src = a.in + poly * a.in_pstride;
     // balanced digits: caller data is any 256-bit value (optionally times a
     // premultiplication factor), a previous pass's output is a pbd word.  Each
     // branch loads and unpacks on its own, so no loaded word lives across it.
     if (a.in_ext) {
-      if (!LAST && a.premul) {
+      if (a.premul) {
         const fr* pm = a.premul + ((uint64_t)(poly & a.pm_mask) << a.lgN) + pos0 + (uint64_t)rho1 * estride;
         const fr* sp = src + pos0 + (uint64_t)rho1 * estride;
         // factors are pbd words of c R' (the coset powers); the product with
@@ -335,76 +366,69 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
         pbd_unpack(raw.l, x[r2].l);
       });
     }
-  } else {
-    static_for<0, kPerT>([&](auto r2_) {
-#pragma unroll
-      for (int i = 0; i < 9; i++) x[decltype(r2_)::value].l[i] = 0;
-    });
   }
-  const uwords dft = (uwords)a.dft;
-  dft_dif<kLgPerT, 0>(x, dft);  // x[brev3(k2)] = sum_rho2 z[rho1 + A rho2] w8^(rho2 k2)
+  dft_dif<kLgPerT, 0>(x, rows);  // x[brev3(k2)] = sum_rho2 z[rho1 + A rho2] w8^(rho2 k2)
+  v9 (&y)[kPerT] = x;
   if constexpr (LA > 0) {
-    // k2 = 0 takes no twiddle: back to balanced digits of a small value, so
-    // that DFT_A again starts from balanced digits (the products' outputs
-    // below are balanced, mont29 BT)
-    {
+    // back to balanced digits of small values, so that DFT_A again starts from
+    // balanced digits: k2 = 0 and wave rho1 = 0 take no twiddle and are reduced
+    // (about 45 instructions), the others' products leave balanced digits (BT)
+    auto reduce = [&](v9& v) {
       v9 t0;
-      reduce_centered(x[0].l, t0.l);
-      x[0] = t0;
-    }
+      reduce_centered(v.l, t0.l);
+      v = t0;
+      pin9(v);
+    };
+    reduce(x[0]);
+    const uwords tw = rows + kRowWords * kInner;
+    const int step = (kRowWords * rho1) << (6 - m);  // w_M'^rho1
+    rows_cols g = rows29_open(tw + step, 0);
     static_for<1, kPerT>([&](auto k2_) {
       constexpr int k2 = decltype(k2_)::value;
-      const int e = rho1 * k2;  // < M'
-      pin9(x[brev(k2, kLgPerT)]);
-      uint32_t w[9];
-      pbd_unpack(fr_load(a.inner29 + (e << (8 - m))).l, w);
-      x[brev(k2, kLgPerT)] = v9_mul<false, false, true>(x[brev(k2, kLgPerT)], w);
+      v9& v = x[brev(k2, kLgPerT)];
+      pin9(v);
+      if (rho1 == 0) {
+        reduce(v);
+      } else {
+        v = v9_mul_rows<2, true>(v, tw + step * k2, g, tw + step * (k2 < kPerT - 1 ? k2 + 1 : k2));
+        pin9(v);
+      }
     });
-  }
-  // Exchange through LDS in kPhases rounds of kW limbs (3 rounds of 12 bytes
-  // = 12 KiB for a 1024-element tile, so eight workgroups = four waves per
-  // SIMD fit a CU).  LDS slot of W[line][rho1][k2]; consecutive lanes hit
-  // consecutive slots.  Each round's gathered limbs go back into the
-  // registers that round vacated: y lives in x (x[f*A + r1] afterwards).
-  // The line index is XOR-swizzled with rho1 so that both the line-major
-  // (intermediate passes) and the rho-major (last pass) write mappings and
-  // the line-major reads are free of LDS bank conflicts.
-  // a fresh copy of the thread index, so that sub-step 2's indices are not
-  // shared with sub-step 1's and kept live across it
-  int t2 = t;
-  asm volatile("" : "+v"(t2));
-  const int lc2 = t2 & (C - 1);
-  const int g = t2 >> LGC;
-  v9 (&y)[kPerT] = x;
-  static_for<0, kPhases>([&](auto h_) {
-    constexpr int h = decltype(h_)::value;
-    uint32_t hv[kPerT][kW];
-    static_for<0, kPerT>([&](auto k2_) {
-      constexpr int k2 = decltype(k2_)::value;
+    // Exchange through LDS in kPhases rounds of kW limbs (3 rounds of 12 bytes,
+    // 48 KiB for A = 8, so two workgroups = four waves per SIMD fit a CU).  A
+    // lane only meets its own column's elements; consecutive lanes hit
+    // consecutive slots.  Each round's gathered limbs go back into the
+    // registers that round vacated: y lives in x (x[f*A + r1] afterwards).
+    static_for<0, kPhases>([&](auto h_) {
+      constexpr int h = decltype(h_)::value;
+      uint32_t hv[kPerT][kW];
+      static_for<0, kPerT>([&](auto k2_) {
+        constexpr int k2 = decltype(k2_)::value;
 #pragma unroll
-      for (int w = 0; w < kW; w++) hv[k2][w] = x[brev(k2, kLgPerT)].l[kW * h + w];
-    });
-    if constexpr (h > 0) __syncthreads();  // previous round's reads done before overwrite
-    static_for<0, kPerT>([&](auto k2_) {
-      constexpr int k2 = decltype(k2_)::value;
-      const int slot = ((k2 * A + rho1) << LGC) + (lc ^ (rho1 & (C - 1)));
-      lds[slot] = pack_limbs<kW>(hv[k2]);
-    });
-    __syncthreads();
-    // sub-step 2 gathers: DFT_A over rho1 for F2 values of k2 of one line
-    static_for<0, F2>([&](auto f_) {
-      constexpr int f = decltype(f_)::value;
-      const int k2 = g * F2 + f;
-      static_for<0, A>([&](auto r1_) {
-        constexpr int r1 = decltype(r1_)::value;
-        const int slot = ((k2 * A + r1) << LGC) + (lc2 ^ (r1 & (C - 1)));
-        unpack_limbs<kW>(&y[f * A + r1].l[kW * h], lds[slot]);
+        for (int w = 0; w < kW; w++) hv[k2][w] = x[brev(k2, kLgPerT)].l[kW * h + w];
+      });
+      if constexpr (h > 0) __syncthreads();  // previous round's reads done before overwrite
+      static_for<0, kPerT>([&](auto k2_) {
+        constexpr int k2 = decltype(k2_)::value;
+        lds[((k2 * A + rho1) << kLgLines) + lc] = pack_limbs<kW>(hv[k2]);
+      });
+      __syncthreads();
+      // sub-step 2 gathers: DFT_A over rho1 for F2 values of k2 of one line
+      static_for<0, F2>([&](auto f_) {
+        constexpr int f = decltype(f_)::value;
+        static_for<0, A>([&](auto r1_) {
+          constexpr int r1 = decltype(r1_)::value;
+          unpack_limbs<kW>(&y[f * A + r1].l[kW * h], lds[(((wv * F2 + f) * A + r1) << kLgLines) + lc]);
+        });
       });
     });
-  });
+  }
   // no barrier follows: lanes of lines beyond the launch leave here
-  const uint64_t line2 = line0 + lc2;
-  if (line2 >= a.nlines) return;
+  if (line_of >= a.nlines) return;
+  // fresh copies of the lane's position, so that sub-step 2's indices are not
+  // shared with sub-step 1's and kept live across it
+  uint64_t line2 = line_of;
+  asm volatile("" : "+v"(line2));
   // last pass: the lane's output base, computed before DFT_A so that its
   // 64-bit temporaries are not live beside the eight results
   fr* base = nullptr;
@@ -423,9 +447,9 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
     asm volatile("" : "+v"(base));
   }
   if constexpr (LA > 0) {
-    static_for<0, F2>([&](auto f_) { dft_dif<LA, decltype(f_)::value * A>(y, dft); });
+    static_for<0, F2>([&](auto f_) { dft_dif<LA, decltype(f_)::value * A>(y, rows); });
   }
-  // y[f*A + brev_LA(k1)] = Z[k2 + kPerT*k1], k2 = g*F2 + f
+  // y[f*A + brev_LA(k1)] = Z[k2 + kPerT*k1], k2 = wv*F2 + f (A = 1: y[brev(f)])
 
   if (LAST) {
     if constexpr (SCALE) {
@@ -440,11 +464,11 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
     }
     static_for<0, F2>([&](auto f_) {
       constexpr int f = decltype(f_)::value;
-      const int k2 = g * F2 + f;
+      const int k2 = wv * F2 + f;
       static_for<0, A>([&](auto k1_) {
         constexpr int k1 = decltype(k1_)::value;
         const uint64_t k = (uint64_t)(k2 + kPerT * k1);
-        v9 v = y[f * A + brev(k1, LA)];
+        v9 v = y[LA > 0 ? f * A + brev(k1, LA) : brev(f, kLgPerT)];
         pin9(v);
         uint32_t tt[9];
         reduce_below_2r(v.l, tt);
@@ -468,11 +492,11 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
     const fr* tw = a.tw + j;
     static_for<0, F2>([&](auto f_) {
       constexpr int f = decltype(f_)::value;
-      const int k2 = g * F2 + f;
+      const int k2 = wv * F2 + f;
       static_for<0, A>([&](auto k1_) {
         constexpr int k1 = decltype(k1_)::value;
         const uint64_t k = (uint64_t)(k2 + kPerT * k1);
-        v9 v = y[f * A + brev(k1, LA)];
+        v9 v = y[LA > 0 ? f * A + brev(k1, LA) : brev(f, kLgPerT)];
         pin9(v);
         uint32_t w[9];
         pbd_unpack(fr_load(tw + (k << a.lgS)).l, w);
@@ -487,7 +511,7 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
 
 
 template <int LA, bool INV, bool LAST, bool SCALE>
-__global__ void __launch_bounds__(kThreads, PL_NTT_WAVES) ntt_pass_kernel(PassArgs a) {
+__global__ void __launch_bounds__(kLines << LA, kWavesPerSimd) ntt_pass_kernel(PassArgs a) {
   ntt_pass_body<LA, INV, LAST, SCALE>(a, blockIdx.x);
 }
 
@@ -496,7 +520,7 @@ __global__ void __launch_bounds__(kThreads, PL_NTT_WAVES) ntt_pass_kernel(PassAr
 // block, ascending; a block finds its segment by binary search (uniform
 // scalar loads, a few steps for the tens of segments of a batch).
 template <int LA, bool INV, bool LAST, bool SCALE>
-__global__ void __launch_bounds__(kThreads, PL_NTT_WAVES)
+__global__ void __launch_bounds__(kLines << LA, kWavesPerSimd)
     ntt_pass_ragged_kernel(const PassArgs* __restrict__ segs, const uint32_t* __restrict__ seg_block0,
                            uint32_t nsegs) {
   const uint32_t b = blockIdx.x;
@@ -515,15 +539,14 @@ __global__ void __launch_bounds__(kThreads, PL_NTT_WAVES)
 // Host launcher for one radix: LA = log2(column size) - kLgPerT.
 template <int LA, bool INV, bool LAST, bool SCALE = false>
 static void launch_pass(const PassArgs& a, hipStream_t s) {
-  constexpr int m = LA + kLgPerT;
-  uint64_t tiles = (a.nlines + (kTile >> m) - 1) >> (kLgTile - m);
-  hipLaunchKernelGGL((ntt_pass_kernel<LA, INV, LAST, SCALE>), dim3((unsigned)tiles), dim3(kThreads), 0, s, a);
+  const uint64_t tiles = (a.nlines + kLines - 1) >> kLgLines;
+  hipLaunchKernelGGL((ntt_pass_kernel<LA, INV, LAST, SCALE>), dim3((unsigned)tiles), dim3(kLines << LA), 0, s, a);
 }
 
 template <int LA, bool INV, bool LAST, bool SCALE = false>
 static void launch_pass_ragged(const PassArgs* segs, const uint32_t* seg_block0, uint32_t nsegs, uint32_t nblocks,
                                hipStream_t s) {
-  hipLaunchKernelGGL((ntt_pass_ragged_kernel<LA, INV, LAST, SCALE>), dim3(nblocks), dim3(kThreads), 0, s, segs,
+  hipLaunchKernelGGL((ntt_pass_ragged_kernel<LA, INV, LAST, SCALE>), dim3(nblocks), dim3(kLines << LA), 0, s, segs,
                      seg_block0, nsegs);
 }
 

@@ -44,13 +44,11 @@ struct Domain {
   fr* pw1 = nullptr;
   fr* inner_fwd = nullptr;         // omega_256^e, e < 256 (stored form; small-size kernel)
   fr* inner_inv = nullptr;
-  fr* inner29_fwd = nullptr;       // the same times 32 (pass kernels)
-  fr* inner29_inv = nullptr;
   // small transforms (ntt_lane.hip), null above kLaneMaxLg: w_N^e, e < N, and
   // the last step's factor pairs (forward, inverse), pbd words of w R'
   fr* lane_lin = nullptr;
   fr* lane_fin = nullptr;
-  uint32_t* dft = nullptr;         // rows29 tables of the in-register DFTs' factors, forward then inverse
+  uint32_t* rows = nullptr;        // rows29 tables of the pass kernels' wave-uniform factors, forward then inverse
   fr* block = nullptr;             // single allocation holding all tables
   size_t bytes = 0;
   host::fr64 n_inv;
@@ -91,14 +89,15 @@ struct NttCall {
   bool inverse = false;
 };
 
-// The one-element-per-lane form: whole transforms of 2^4 .. 2^kLaneMaxLg points
-// whose call has at most kLaneMaxElems elements in all; one launch up to
-// 2^kLaneOne points, where a column still fits one CU well (us per call, one
-// transform: 2^9 in one launch 9.2, 2^10 in one 16.4 and in two 10.3).  At
-// 2^19 elements in all it takes 85 us against the pass kernels' 95; above,
-// their eight elements per lane fill the chip and need half the instructions.
-constexpr int kLaneMaxLg = 19, kLaneOne = 9;
-constexpr uint64_t kLaneMaxElems = 1ull << 19;
+// The one-element-per-lane form: whole transforms of 2^4 .. 2^kLaneMaxLg
+// points, one launch up to 2^kLaneOne points, where a column still fits one CU
+// well (us per call, one transform: 2^9 in one launch 9.2, 2^10 in one 16.4
+// and in two 10.3).  lane_form's line lies where the pass kernels, with eight
+// elements per lane and half the instructions, have filled the chip (us per
+// call, lane form against passes): 2^18 elements in all, 2^12 points 28.8 /
+// 42.4, 2^15 36.1 / 51.5, 2^18 46.1 / 69.1; 2^19 elements, 2^12 points (two
+// passes) 47.5 / 47.2, 2^15 61.6 / 60.7, 2^18 79.7 / 74.0.
+constexpr int kLaneMaxLg = 18, kLaneOne = 9;
 constexpr int kLaneFin = 16;  // elements of the factor pairs
 hipError_t lane_tables(Domain& d, fr* fin, hipStream_t s);
 bool lane_form(const Domain& d, const NttCall& c);

@@ -142,10 +142,9 @@ hipError_t phase_plan(PhasePlan& ph, const std::vector<Item>& items, Bump& bump,
         ph.groups.push_back(g);
       }
       RaggedGroup& g = ph.groups[f->second];
-      const int lgc = kLgTile - d->plan.m[p];
       g.seg_block0.push_back(g.nblocks);
       g.segs.push_back(a);
-      g.nblocks += (uint32_t)((a.nlines + (1ull << lgc) - 1) >> lgc);
+      g.nblocks += (uint32_t)((a.nlines + kLines - 1) >> kLgLines);
     }
   }
   // launch order: every group of depth 0, then depth 1, ...
