@@ -108,7 +108,7 @@ __device__ __forceinline__ fr lds_get2(uint4 (*l)[kOpThreads], int t) {
 // the R'-view word of x / 32, so a level-0 output P(S(num), inverse of S(x)) =
 // 32 S(num / x), and without num the inverse alone is 1024 S(1 / x).  Every
 // output is linear in the one field inversion at the top, which absorbs that
-// factor (inv_single_kernel).
+// factor (inv_down_kernel's TOP).
 
 // R' mod r: the R'-view one
 __device__ __forceinline__ fr rp_one() {
@@ -139,56 +139,48 @@ __device__ __forceinline__ fr mul_pbd(const fr& a, const fr& b) {
   return o;
 }
 
-// Exclusive product over the 256 thread values (pbd words) of the threads
-// before t (suffix: after t), as a pbd word.  Work-efficient (up-sweep, then
-// down-sweep): 2 x 255 products per block instead of 8 per thread.  one: the
-// pbd word of the R'-view one.
-__device__ fr block_scan_excl(const fr& v, uint4 (*l)[kOpThreads], bool suffix, const fr& one) {
-  const int t = threadIdx.x;
-  const int slot = suffix ? kOpThreads - 1 - t : t;
-  lds_put2(l, slot, v);
-  for (int d = 1; d < kOpThreads; d <<= 1) {
-    __syncthreads();
-    const int i = (t + 1) * 2 * d - 1;
-    if (i < kOpThreads) lds_put2(l, i, mul_pbd(lds_get2(l, i - d), lds_get2(l, i)));
-  }
-  __syncthreads();
-  if (t == 0) lds_put2(l, kOpThreads - 1, one);
-  for (int d = kOpThreads / 2; d >= 1; d >>= 1) {
-    __syncthreads();
-    const int i = (t + 1) * 2 * d - 1;
-    if (i < kOpThreads) {
-      const fr left = lds_get2(l, i - d), right = lds_get2(l, i);
-      lds_put2(l, i - d, right);
-      lds_put2(l, i, mul_pbd(left, right));
-    }
-  }
-  __syncthreads();
-  const fr r = lds_get2(l, slot);
-  __syncthreads();
-  return r;
+__device__ __forceinline__ v9 shfl_xor9(const v9& v, int m) {
+  v9 o;
+#pragma unroll
+  for (int i = 0; i < 9; i++) o.l[i] = (uint32_t)__shfl_xor((int)v.l[i], m);
+  return o;
 }
 
-// The same exclusive product by Hillis-Steele steps: 8 levels of products
-// instead of 16 (more products in all, a shorter chain), for a single-block
-// top level where the latency is the cost.
-__device__ fr block_scan_excl_short(fr v, uint4 (*l)[kOpThreads], bool suffix, const fr one) {
-  const int t = threadIdx.x;
-  lds_put2(l, t, v);
-  __syncthreads();
-  for (int s = 1; s < kOpThreads; s <<= 1) {
-    const int o = suffix ? t + s : t - s;
-    const bool has = suffix ? o < kOpThreads : o >= 0;
-    const fr other = has ? lds_get2(l, o) : one;
-    __syncthreads();
-    if (has) v = mul_pbd(v, other);
-    lds_put2(l, t, v);
-    __syncthreads();
+// E = the product over the block's other threads of their P (balanced digits,
+// |value| < 1.08 r or a 256-bit word), and rest = that over the other waves.
+// A lane carries the product of its group of 2^k lanes and of the group less
+// itself, and takes its sibling group's: two products per step across the
+// wave, no barriers; the four wave products meet in LDS once.  14 products
+// per thread, a chain of 9, where an exclusive prefix and an exclusive suffix
+// by up- and down-sweep took a chain of 34 through 64 barriers (the
+// down-sweep of 2^21 quotients 157 -> 107 us, with the coalesced order below).
+__device__ __forceinline__ void block_others(v9& P, v9& E, v9& rest) {
+  __shared__ uint32_t wt[4][9];
+  const int t = threadIdx.x, w = t >> 6;
+  E = shfl_xor9(P, 1);
+  P = v9_mul<false, false, true>(P, E.l);
+#pragma unroll
+  for (int m = 2; m < 64; m <<= 1) {
+    const v9 sib = shfl_xor9(P, m);
+    E = v9_mul<false, false, true>(E, sib.l);
+    P = v9_mul<false, false, true>(P, sib.l);
   }
-  const int e = suffix ? t + 1 : t - 1;
-  const fr ex = (suffix ? e < kOpThreads : e >= 0) ? lds_get2(l, e) : one;
+  if ((t & 63) == 0) {
+#pragma unroll
+    for (int i = 0; i < 9; i++) wt[w][i] = P.l[i];
+  }
   __syncthreads();
-  return ex;
+  auto wave = [&](int k, v9& v) {
+#pragma unroll
+    for (int i = 0; i < 9; i++) v.l[i] = wt[(w + k) & 3][i];
+  };
+  v9 o;
+  wave(1, rest);
+  wave(2, o);
+  rest = v9_mul<false, false, true>(rest, o.l);
+  wave(3, o);
+  rest = v9_mul<false, false, true>(rest, o.l);
+  E = v9_mul<false, false, true>(E, rest.l);
 }
 
 // The exclusive prefix product of a and the exclusive suffix product of b
@@ -218,11 +210,8 @@ __device__ void block_scan2_short(fr& a, fr& b, uint4 (*la)[kOpThreads], uint4 (
 }
 
 // Phase 1: total[b] = product over block b of in[i] (zeros taken as one).
-// Blocks of 256 x 2^LG elements: LG = kOpLgPer in bulk levels; a single-block
-// top level takes the smallest LG that covers it.
-template <int LG>
 __global__ void __launch_bounds__(kOpThreads) inv_reduce_kernel(const fr* in, uint64_t n, fr* total) {
-  constexpr int kOpPer = 1 << LG, kOpLgPer = LG, kOpLgSeg = 8 + LG;
+  constexpr int kOpLgSeg = 8 + kOpLgPer;
   __shared__ uint4 l[2][kOpThreads];
   // order-free product: thread t takes elements b*kOpSeg + 256 k + t (coalesced)
   const uint64_t b0 = (uint64_t)blockIdx.x << kOpLgSeg;
@@ -236,27 +225,22 @@ __global__ void __launch_bounds__(kOpThreads) inv_reduce_kernel(const fr* in, ui
   // pairwise tree in registers: eight products of unpacked words, then the
   // products of products (all limbs normalized digits, so any pair is a valid
   // operand pair)
-  fr acc;
-  if constexpr (kOpPer == 1) {
-    acc = v[0];
-  } else {
-    v9 p[kOpPer / 2];
-    static_for<0, kOpPer / 2>([&](auto k_) {
+  v9 p[kOpPer / 2];
+  static_for<0, kOpPer / 2>([&](auto k_) {
+    constexpr int k = decltype(k_)::value;
+    v9 x, y;
+    unpack_ext(v[k].l, x.l);
+    unpack_ext(v[k + kOpPer / 2].l, y.l);
+    p[k] = v9_mul<false, false, false>(x, y.l);
+  });
+  static_for<0, kOpLgPer - 1>([&](auto s_) {
+    constexpr int h = kOpPer / 2 >> (decltype(s_)::value + 1);
+    static_for<0, h>([&](auto k_) {
       constexpr int k = decltype(k_)::value;
-      v9 x, y;
-      unpack_ext(v[k].l, x.l);
-      unpack_ext(v[k + kOpPer / 2].l, y.l);
-      p[k] = v9_mul<false, false, false>(x, y.l);
+      p[k] = v9_mul<false, false, false>(p[k], p[k + h].l);
     });
-    static_for<0, kOpLgPer - 1>([&](auto s_) {
-      constexpr int h = kOpPer / 2 >> (decltype(s_)::value + 1);
-      static_for<0, h>([&](auto k_) {
-        constexpr int k = decltype(k_)::value;
-        p[k] = v9_mul<false, false, false>(p[k], p[k + h].l);
-      });
-    });
-    acc = v9_canonical(p[0]);
-  }
+  });
+  fr acc = v9_canonical(p[0]);
   lds_put2(l, threadIdx.x, acc);
   __syncthreads();
   for (int s = kOpThreads / 2; s > 0; s >>= 1) {
@@ -271,16 +255,24 @@ __global__ void __launch_bounds__(kOpThreads) inv_reduce_kernel(const fr* in, ui
 
 // Phase 3: with binv[b] the inverse of block b's product, out[i] = num[i] /
 // in[i] (num == nullptr: one); zero inputs give zero.  out may equal in or num.
+// The products are order-free, so thread t takes elements b*kOpSeg + 256 k + t
+// (coalesced; a run of its own per thread fetched each line four times).
 // Local prefixes L_k are kept as pbd words (products with balanced digits; a
 // product of two values below 1.3 r lies in (-r, 0.03 r), inside a pbd word).
-// SHORT: Hillis-Steele thread scans (single-block top level)
-template <int LG, bool SHORT>
-__global__ void __launch_bounds__(kOpThreads) inv_down_kernel(const fr* in, const fr* num, fr* out, uint64_t n,
-                                                               const fr* binv) {
+// TOP: the only block, which also inverts its product: times 2^-5 (level-0
+// outputs with num) or 2^-10 (without), i.e. fr_inv_wave(W) times 32 or 1 (see
+// the batch-inversion notes above).
+template <int LG, bool TOP>
+__global__ void __launch_bounds__(kOpThreads) __attribute__((amdgpu_waves_per_eu(TOP ? 1 : 3)))
+inv_down_kernel(const fr* in, const fr* num, fr* out, uint64_t n, const fr* binv, int with_num) {
   constexpr int kOpPer = 1 << LG, kOpLgSeg = 8 + LG;
-  __shared__ uint4 l[2][kOpThreads];
   const int t = threadIdx.x;
-  const uint64_t base = ((uint64_t)blockIdx.x << kOpLgSeg) + (uint64_t)t * kOpPer;
+  // wave-uniform bases and 32-bit lane offsets: eight 64-bit indices per lane
+  // would spill
+  const uint64_t b0 = (uint64_t)blockIdx.x << kOpLgSeg;
+  const uint32_t rem = (uint32_t)(n - b0 < kOpThreads * kOpPer ? n - b0 : kOpThreads * kOpPer);
+  auto live = [&](int k) { return (uint32_t)(k * kOpThreads + t) < rem; };
+  auto load_in = [&](int k) { return live(k) ? fr_load(in + b0 + k * kOpThreads + t) : rp_one(); };
   fr e[kOpPer];
   uint32_t zmask = 0;
   // local prefix L_k = x_0 ... x_k (pbd words in e[]); the thread product is
@@ -288,16 +280,18 @@ __global__ void __launch_bounds__(kOpThreads) inv_down_kernel(const fr* in, cons
   v9 L;
   static_for<0, kOpPer>([&](auto k_) {
     constexpr int k = decltype(k_)::value;
-    fr v = base + k < n ? fr_load(in + base + k) : rp_one();
-    if (fr_is_zero(v)) {
+    e[k] = load_in(k);
+  });
+  static_for<0, kOpPer>([&](auto k_) {
+    constexpr int k = decltype(k_)::value;
+    if (fr_is_zero(e[k])) {
       zmask |= 1u << k;
-      v = rp_one();
+      e[k] = rp_one();
     }
     v9 x;
-    unpack_ext(v.l, x.l);
+    unpack_ext(e[k].l, x.l);
     if constexpr (k == 0) {
-      L = x;
-      e[0] = v;  // L_0 = x_0 as loaded (below 2^256, beyond a pbd word's range)
+      L = x;  // L_0 = x_0 as loaded (below 2^256, beyond a pbd word's range)
     } else {
       // |L_k| < 1.07 r: the product of a value below 1.07 r (or x_0 < 2^256) and
       // x_k < 2^256 lies in (-1.07 r, 0.07 r)
@@ -305,72 +299,70 @@ __global__ void __launch_bounds__(kOpThreads) inv_down_kernel(const fr* in, cons
       pbd_pack(L.l, e[k].l);
     }
   });
-  fr tp;
-  pbd_pack(L.l, tp.l);
-  fr one;
-  {
-    const fr o = rp_one();
-    to_pbd(o.l, one.l);
+  // inv(L_last) = binv * (the block product over everything outside this
+  // thread's elements)
+  v9 cur, E, rest;
+  block_others(L, E, rest);
+  fr b;
+  if constexpr (TOP) {
+    __shared__ fr cinv;
+    if (t < 64) {
+      fr z = fr_inv_wave(v9_canonical(v9_mul<false, false, false>(rest, L.l)));
+      if (with_num) {
+#pragma unroll
+        for (int d = 0; d < 5; d++) z = fr_add(z, z);
+      }
+      if (t == 0) cinv = z;
+    }
+    __syncthreads();
+    b = cinv;
+  } else {
+    b = fr_load(binv + blockIdx.x);
   }
-  const fr suf = SHORT ? block_scan_excl_short(tp, l, true, one) : block_scan_excl(tp, l, true, one);
-  const fr pre = SHORT ? block_scan_excl_short(tp, l, false, one) : block_scan_excl(tp, l, false, one);
-  // inv(L_last) = binv * suffix(> t) * prefix(< t): the block product over
-  // everything outside this thread's run, times the block's inverse
-  v9 cur;
-  {
-    v9 a, b, c;
-    unpack_ext(fr_load(binv + blockIdx.x).l, a.l);
-    pbd_unpack(suf.l, b.l);
-    pbd_unpack(pre.l, c.l);
-    cur = v9_mul<false, false, false>(v9_mul<false, false, false>(a, b.l), c.l);
-  }
+  unpack_ext(b.l, cur.l);
+  cur = v9_mul<false, false, false>(cur, E.l);
   // walk back: inv(x_k) = inv(L_k) L_{k-1} (inv(x_0) = inv(L_0));
-  // inv(L_{k-1}) = inv(L_k) x_k
+  // inv(L_{k-1}) = inv(L_k) x_k; each element and numerator is asked for one
+  // step ahead, before the result in between is stored
+  auto load_num = [&](int k) { return num && live(k) ? fr_load(num + b0 + k * kOpThreads + t) : rp_one(); };
+  fr xn = load_in(kOpPer - 1);
   static_for<0, kOpPer>([&](auto k_) {
     constexpr int k = kOpPer - 1 - decltype(k_)::value;
+    fr xk = xn;
+    const fr nk = load_num(k);
+    if constexpr (k > 0) xn = load_in(k - 1);
+    __builtin_amdgcn_sched_barrier(0x0002 | 0x0004 | 0x0080);
     v9 inv_k = cur;
     if constexpr (k > 0) {
       uint32_t Lp[9];
       if constexpr (k - 1 == 0) unpack_ext(e[0].l, Lp);
       else pbd_unpack(e[k > 1 ? k - 1 : 1].l, Lp);
       inv_k = v9_mul<false, false, false>(cur, Lp);
+      pin9(inv_k);  // one product at a time: fewer live temporaries
+      pin9(cur);
       // x_k from the original input (one again for zeros)
-      fr xk = base + k < n ? fr_load(in + base + k) : rp_one();
       if ((zmask >> k) & 1) xk = rp_one();
       uint32_t X[9];
       unpack_ext(xk.l, X);
       cur = v9_mul<false, false, false>(cur, X);
+      pin9(cur);
+      pin9(inv_k);
     }
-    if (base + k < n) {
+    if (live(k)) {
       fr r;
       if ((zmask >> k) & 1) {
         r = fr_zero();
       } else {
         if (num) {
           uint32_t N[9];
-          unpack_ext(fr_load(num + base + k).l, N);
+          unpack_ext(nk.l, N);
           inv_k = v9_mul<false, false, false>(inv_k, N);
         }
         r = v9_canonical(inv_k);
       }
-      fr_store(out + base + k, r);
+      fr_store(out + b0 + k * kOpThreads + t, r);
     }
   });
-}
-
-// single inversion at the top of the batch: *p <- the R'-view inverse of *p
-// times 2^-5 (level-0 outputs with num) or 2^-10 (without), i.e.
-// fr_inv_wave(W) times 32 or 1 (see the batch-inversion notes above); one
-// block of one wave
-__global__ void inv_single_kernel(fr* p, int with_num) {
-  if (threadIdx.x < 64 && blockIdx.x == 0) {
-    fr z = fr_inv_wave(fr_load(p));
-    if (with_num) {
-#pragma unroll
-      for (int d = 0; d < 5; d++) z = fr_add(z, z);
-    }
-    if (threadIdx.x == 0) fr_store(p, z);
-  }
 }
 
 static uint64_t inv_scratch_elems(uint64_t n) {
@@ -390,33 +382,23 @@ static hipError_t batch_inverse_level(const fr* in, const fr* num, fr* out, uint
   fr* tot = scratch;
   fr* tinv = scratch + nb;
   if (nb == 1) {
-    // one block: 256 x 2^LG with the smallest LG that covers n, short scans
+    // one block: 256 x 2^LG with the smallest LG that covers n (1024 values, in
+    // one launch instead of reduce, inversion and down-sweep: 72 -> 58 us, of
+    // which the inversion takes 31)
     const dim3 g(1), b(kOpThreads);
-    if (n <= 256) {
-      hipLaunchKernelGGL(inv_reduce_kernel<0>, g, b, 0, s, in, n, tot);
-      hipLaunchKernelGGL(inv_single_kernel, dim3(1), dim3(64), 0, s, tot, with_num);
-      hipLaunchKernelGGL((inv_down_kernel<0, true>), g, b, 0, s, in, num, out, n, (const fr*)tot);
-    } else if (n <= 512) {
-      hipLaunchKernelGGL(inv_reduce_kernel<1>, g, b, 0, s, in, n, tot);
-      hipLaunchKernelGGL(inv_single_kernel, dim3(1), dim3(64), 0, s, tot, with_num);
-      hipLaunchKernelGGL((inv_down_kernel<1, true>), g, b, 0, s, in, num, out, n, (const fr*)tot);
-    } else if (n <= 1024) {
-      hipLaunchKernelGGL(inv_reduce_kernel<2>, g, b, 0, s, in, n, tot);
-      hipLaunchKernelGGL(inv_single_kernel, dim3(1), dim3(64), 0, s, tot, with_num);
-      hipLaunchKernelGGL((inv_down_kernel<2, true>), g, b, 0, s, in, num, out, n, (const fr*)tot);
-    } else {
-      hipLaunchKernelGGL(inv_reduce_kernel<kOpLgPer>, g, b, 0, s, in, n, tot);
-      hipLaunchKernelGGL(inv_single_kernel, dim3(1), dim3(64), 0, s, tot, with_num);
-      hipLaunchKernelGGL((inv_down_kernel<kOpLgPer, true>), g, b, 0, s, in, num, out, n, (const fr*)tot);
-    }
+    const fr* none = nullptr;
+    if (n <= 256) hipLaunchKernelGGL((inv_down_kernel<0, true>), g, b, 0, s, in, num, out, n, none, with_num);
+    else if (n <= 512) hipLaunchKernelGGL((inv_down_kernel<1, true>), g, b, 0, s, in, num, out, n, none, with_num);
+    else if (n <= 1024) hipLaunchKernelGGL((inv_down_kernel<2, true>), g, b, 0, s, in, num, out, n, none, with_num);
+    else hipLaunchKernelGGL((inv_down_kernel<kOpLgPer, true>), g, b, 0, s, in, num, out, n, none, with_num);
     return hipGetLastError();
   }
-  hipLaunchKernelGGL(inv_reduce_kernel<kOpLgPer>, dim3((unsigned)nb), dim3(kOpThreads), 0, s, in, n, tot);
+  hipLaunchKernelGGL(inv_reduce_kernel, dim3((unsigned)nb), dim3(kOpThreads), 0, s, in, n, tot);
   // block totals are never zero (zeros were skipped): invert them as a batch
   hipError_t e = batch_inverse_level(tot, nullptr, tinv, nb, scratch + 2 * nb, with_num, s);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((inv_down_kernel<kOpLgPer, false>), dim3((unsigned)nb), dim3(kOpThreads), 0, s, in, num, out, n,
-                     (const fr*)tinv);
+                     (const fr*)tinv, with_num);
   return hipGetLastError();
 }
 

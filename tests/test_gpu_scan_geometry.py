@@ -1,0 +1,61 @@
+"""Grand product and batch inversion at the edges of their block geometries
+(256 threads x 1, 2, 4, 8, 16 elements; one and several blocks), against the
+oracle, with zeros, ones and r - 1 among the inputs."""
+import numpy as np
+import pytest
+
+import pyoracle as po
+
+pytestmark = pytest.mark.gpu
+
+MINUS_ONE_INT = [0xFFFFFFFF00000000, 0x53BDA402FFFE5BFE, 0x3339D80809A1D805, 0x73EDA753299D7D48]  # the word r - 1
+
+
+@pytest.fixture(scope="module")
+def pl():
+    import torch
+    assert torch.cuda.is_available(), "GPU tests need a HIP device"
+    import plffi
+    plffi.lib()
+    return plffi
+
+
+def inputs(n, seed):
+    x = po.uniform(n, seed)
+    x[::7] = MINUS_ONE_INT
+    x[3::11] = po.one()[0]
+    return x
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 2047, 2048, 2049,
+                               4096, 4111, 8193, 4096 * 256, 4096 * 257 + 1])
+def test_grand_product_edges(pl, n):
+    import torch
+    print("gp edge", n, flush=True)
+    x = inputs(n, po.seed(po.OP_GP, 1, n & 0xff))
+    exp = po.grand_product(x)
+    a = pl.to_dev(x)
+    incl = torch.zeros_like(a)
+    pl.grand_product(a, incl_out=incl)
+    np.testing.assert_array_equal(pl.to_host(a), exp)
+    gi = pl.to_host(incl)
+    np.testing.assert_array_equal(gi[:-1], exp[1:])
+    np.testing.assert_array_equal(gi[-1:], po.mul(exp[-1:], x[-1:]))
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 65, 255, 256, 257, 512, 513, 1024, 1025, 2047, 2048, 2049, 4097,
+                               2048 * 256 + 1, 2048 * 1025])
+def test_inverse_and_quotient_edges(pl, n):
+    print("inv edge", n, flush=True)
+    x, y = inputs(n, n), po.uniform(n, n + 1)
+    x[n // 2] = 0
+    x[-1 if n > 1 else 0] = 0
+    inv = np.zeros_like(x)
+    po.lib().or_vec_inv(po.P(inv), po.P(x), n)
+    xd, yd = pl.to_dev(x), pl.to_dev(y)
+    np.testing.assert_array_equal(pl.to_host(pl.vec_op("inv", xd)), inv)
+    np.testing.assert_array_equal(pl.to_host(pl.vec_op("div", yd, xd)), po.mul(y, inv))
+    # in place over the divisor and over the numerator
+    a, b = pl.to_dev(x), pl.to_dev(y)
+    np.testing.assert_array_equal(pl.to_host(pl.vec_op("div", b, a, out=a)), po.mul(y, inv))
+    np.testing.assert_array_equal(pl.to_host(pl.vec_op("div", b, xd, out=b)), po.mul(y, inv))
