@@ -42,106 +42,211 @@ __device__ __forceinline__ fr lds_get(uint4 (*l)[kScanThreads], int t) {
   return v;
 }
 
-// ---------------------------------------------------------------------------
-// multiplicative prefix scan
-// ---------------------------------------------------------------------------
-
-// thread-level exclusive prefix across the block (Hillis-Steele over 256
-// thread totals, multiplicative); returns the product of threads < t
-__device__ fr block_excl_prod(fr v, uint4 (*l)[kScanThreads], fr* block_total) {
-  const int t = threadIdx.x;
-  fr incl = v;
-  lds_put(l, t, incl);
-  __syncthreads();
-  for (int s = 1; s < kScanThreads; s <<= 1) {
-    fr other = t >= s ? lds_get(l, t - s) : fr_one();
-    __syncthreads();
-    if (t >= s) incl = fr_mul(incl, other);
-    lds_put(l, t, incl);
-    __syncthreads();
-  }
-  fr excl = t > 0 ? lds_get(l, t - 1) : fr_one();
-  if (block_total) *block_total = lds_get(l, kScanThreads - 1);
-  __syncthreads();
-  return excl;
+// R' mod r: the R'-form of one (R' = 2^261)
+__host__ __device__ constexpr uint32_t rp_one_limb(int i) {
+  return i == 0 ? 0xffffffbau : i == 1 ? 0x00000045u : i == 2 ? 0x0072d846u : i == 3 ? 0x1a25272eu
+       : i == 4 ? 0x5dbeee8bu : i == 5 ? 0xfe2eedcdu : i == 6 ? 0x9eefbe41u : 0x4d043f42u;
+}
+__device__ __forceinline__ fr rp_one_fr() {
+  fr o;
+#pragma unroll
+  for (int i = 0; i < 8; i++) o.l[i] = rp_one_limb(i);
+  return o;
 }
 
 // Block geometry of a scan kernel: 256 threads x 2^LG elements.  LG = kLgPer
-// for the bulk; LG = 0 for a top level of at most 256 values, where the
-// latency of the per-thread chains (2^LG dependent products) dominates.
+// for the bulk; a single-block level takes the smallest that covers it, where
+// the latency of the per-thread chains (2^LG dependent products) dominates.
 template <int LG>
 struct ScanGeom {
   static constexpr int kPer = 1 << LG;
   static constexpr int kLgSeg = 8 + LG;
 };
 
-// partial[b] = product of block b's elements.  The product is order-free,
-// so thread t takes elements b*kSeg + 256 k + t: every load is coalesced.
-template <int LG>
+// ---------------------------------------------------------------------------
+// multiplicative prefix scan
+// ---------------------------------------------------------------------------
+// The products run in signed radix-2^29 limbs (fr29.hpp): P(a, b) = a b / R',
+// R' = 2^261, about 205 VALU instructions against the saturated product's 290.
+// A stored word S(x) = x R shifted left by five bits is the integer 32 x R =
+// x R', the R'-form that P is closed under, and it fits nine 29-bit digits; so
+// P(S(a), 32 S(b)) = S(a b) with the shift taken in the digit split.  Level 0
+// (RF false) reads stored words: its running products stay in stored form,
+// its block products and everything a level above reads are in R'-form
+// (RF true).  At 2^21 the only block of the upper level took 37-54 us on
+// chains of 16 products and eight barrier-separated scan steps; with two
+// elements per thread and the scan inside the wave, 9-12 us.  Bounds: with w = 32 x R < 2^261 x / r a step maps |h| to at most
+// 0.453 |h| + r / 2 with centred Montgomery digits (BM), so |h| < 0.96 r from
+// h = S(x_0) < r; in R'-form a step of values within 1.1 r lies in (-1.02 r,
+// 0.02 r).  Both fit a pbd word (1.104 r).
+
+// nine 29-bit digits of 32 x (x any 256-bit word)
+__device__ __forceinline__ void split29_x32(const uint32_t* x, uint32_t* a) {
+  a[0] = (x[0] << 5) & kMask29;
+#pragma unroll
+  for (int i = 1; i < 8; i++) {
+    const int b = 29 * i - 5;
+    a[i] = funnel_r(x[(b >> 5) + 1], x[b >> 5], b & 31) & kMask29;
+  }
+  a[8] = x[7] >> 3;
+}
+
+// 32 v for balanced digits of a value within 1.1 r, again balanced
+__device__ __forceinline__ v9 v9_x32(const v9& v) {
+  v9 o;
+  int64_t acc = 0;
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    acc += (int64_t)(int32_t)v.l[i] * 32;
+    o.l[i] = sext29((uint32_t)acc);
+    acc = (acc - (int64_t)(int32_t)o.l[i]) >> 29;
+  }
+  o.l[8] = (uint32_t)(acc + (int64_t)(int32_t)v.l[8] * 32);
+  return o;
+}
+
+__device__ __forceinline__ v9 shfl_up9(const v9& v, int s) {
+  v9 o;
+#pragma unroll
+  for (int i = 0; i < 9; i++) o.l[i] = (uint32_t)__shfl_up((int)v.l[i], s);
+  return o;
+}
+
+// P closed in R'-form, balanced digits
+__device__ __forceinline__ v9 mul_r(const v9& a, const v9& b) { return v9_mul<false, false, true>(a, b.l); }
+
+// partial[b] = product of block b's elements (R'-form word).  The product is
+// order-free, so thread t takes elements b*kSeg + 256 k + t: every load is
+// coalesced.  Across the wave six exchange steps, then the four wave products.
+template <bool RF>
 __global__ void __launch_bounds__(kScanThreads) pfx_reduce_kernel(const fr* in, uint64_t n, fr* partial) {
-  constexpr int kPer = ScanGeom<LG>::kPer, kLgSeg = ScanGeom<LG>::kLgSeg, kLgPer = LG;
-  __shared__ uint4 l[2][kScanThreads];
+  __shared__ uint32_t wt[4][9];
+  const int t = threadIdx.x;
   const uint64_t b0 = (uint64_t)blockIdx.x << kLgSeg;
+  const uint32_t rem = (uint32_t)(n - b0 < kSeg ? n - b0 : kSeg);
   fr v[kPer];
   static_for<0, kPer>([&](auto k_) {
     constexpr int k = decltype(k_)::value;
-    const uint64_t i = b0 + (uint64_t)k * kScanThreads + threadIdx.x;
-    v[k] = i < n ? fr_load(in + i) : fr_one();
+    if ((uint32_t)(k * kScanThreads + t) < rem) v[k] = fr_load(in + b0 + k * kScanThreads + t);
   });
-  // pairwise tree in registers (independent products)
-  static_for<0, kLgPer>([&](auto s_) {
-    constexpr int h = kPer >> (decltype(s_)::value + 1);
-    static_for<0, h>([&](auto k_) {
-      constexpr int k = decltype(k_)::value;
-      v[k] = fr_mul(v[k], v[k + h]);
-    });
-  });
-  fr acc = v[0];
-  // tree product over the block
-  lds_put(l, threadIdx.x, acc);
-  __syncthreads();
-  for (int s = kScanThreads / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-      acc = fr_mul(acc, lds_get(l, threadIdx.x + s));
-      lds_put(l, threadIdx.x, acc);
+  v9 h;
+  unpack_ext(rp_one_fr().l, h.l);
+  static_for<0, kPer>([&](auto k_) {
+    constexpr int k = decltype(k_)::value;
+    // one element at a time, as its load arrives
+    if ((uint32_t)(k * kScanThreads + t) < rem) {
+      uint32_t w[9];
+      if constexpr (RF) unpack_ext(v[k].l, w);
+      else split29_x32(v[k].l, w);
+      h = v9_mul<false, !RF, true>(h, w);
     }
-    __syncthreads();
+  });
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) {
+    v9 o;
+#pragma unroll
+    for (int i = 0; i < 9; i++) o.l[i] = (uint32_t)__shfl_xor((int)h.l[i], m);
+    h = mul_r(h, o);
   }
-  if (threadIdx.x == 0) fr_store(partial + blockIdx.x, acc);
+  if ((t & 63) == 0) {
+#pragma unroll
+    for (int i = 0; i < 9; i++) wt[t >> 6][i] = h.l[i];
+  }
+  __syncthreads();
+  if (t >= 64) return;
+#pragma unroll
+  for (int w = 1; w < 4; w++) h = v9_mul<false, false, true>(h, wt[w]);
+  if (t == 0) fr_store(partial + blockIdx.x, v9_canonical(h));
 }
 
 // out_excl[i] = carry_b * prod_{block start <= j < i} in[j]; optional inclusive
-// output and block total (single-block use).  carry == nullptr means one.
-template <int LG>
-__global__ void __launch_bounds__(kScanThreads) pfx_down_kernel(const fr* in, fr* out_excl, fr* out_incl, uint64_t n,
-                                                                 const fr* carry, fr* total) {
+// output.  carry (R'-form words) == nullptr means one.  in may equal out_excl.
+template <int LG, bool RF>
+__global__ void __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(2)))
+pfx_down_kernel(const fr* in, fr* out_excl, fr* out_incl, uint64_t n, const fr* carry) {
   constexpr int kPer = ScanGeom<LG>::kPer, kLgSeg = ScanGeom<LG>::kLgSeg;
-  __shared__ uint4 l[2][kScanThreads];
-  const uint64_t base = ((uint64_t)blockIdx.x << kLgSeg) + (uint64_t)threadIdx.x * kPer;
+  __shared__ uint32_t wt[4][9];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const uint64_t b0 = (uint64_t)blockIdx.x << kLgSeg;
+  const int rem = (int)(n - b0 < kScanThreads * kPer ? n - b0 : kScanThreads * kPer) - t * kPer;
+  const fr* src = in + b0 + t * kPer;
   fr e[kPer];
   static_for<0, kPer>([&](auto k_) {
     constexpr int k = decltype(k_)::value;
-    e[k] = base + k < n ? fr_load(in + base + k) : fr_one();
+    e[k] = fr_zero();
+    if (k < rem) e[k] = fr_load(src + k);
   });
-  // local inclusive products in place: e[k] = in[base] * ... * in[base+k]
-  static_for<1, kPer>([&](auto k_) {
-    constexpr int k = decltype(k_)::value;
-    e[k] = fr_mul(e[k - 1], e[k]);
-  });
-  fr btot;
-  fr pre = block_excl_prod(e[kPer - 1], l, &btot);
-  if (carry) {
-    fr c = fr_load(carry + blockIdx.x);
-    pre = fr_mul(c, pre);
-    btot = fr_mul(c, btot);
-  }
-  if (total && blockIdx.x == 0 && threadIdx.x == 0) fr_store(total, btot);
+  v9 one;
+  unpack_ext(rp_one_fr().l, one.l);
+  // local inclusive products: e[k] = in[base] * ... * in[base+k], pbd words
+  // (level 0: stored form; an element beyond n counts as one)
+  v9 h;
   static_for<0, kPer>([&](auto k_) {
     constexpr int k = decltype(k_)::value;
-    if (base + k < n) {
-      fr ex = k == 0 ? pre : fr_mul(pre, e[k > 0 ? k - 1 : 0]);
-      if (out_incl) fr_store(out_incl + base + k, fr_mul(pre, e[k]));
-      fr_store(out_excl + base + k, ex);
+    if constexpr (k == 0) {
+      h = one;  // no element of this thread: R'-form one (never stored)
+      if (rem > 0) unpack_ext(e[0].l, h.l);
+    } else if (k < rem) {
+      uint32_t w[9];
+      if constexpr (RF) unpack_ext(e[k].l, w);
+      else split29_x32(e[k].l, w);
+      h = v9_mul<false, !RF, true>(h, w);
+    }
+    pbd_pack(h.l, e[k].l);  // canonical words and products fit
+  });
+  // thread products in R'-form, their exclusive prefix across the block
+  v9 p = RF || rem <= 0 ? h : v9_x32(h);
+#pragma unroll
+  for (int s = 1; s < 64; s <<= 1) {
+    const v9 o = shfl_up9(p, s);
+    const v9 q = mul_r(p, o);
+    if (lane >= s) p = q;
+  }
+  if (lane == 63) {
+#pragma unroll
+    for (int i = 0; i < 9; i++) wt[wave][i] = p.l[i];
+  }
+  __syncthreads();
+  v9 pre = shfl_up9(p, 1);
+  if (lane == 0) pre = one;
+#pragma unroll
+  for (int w = 0; w < 3; w++)
+    if (w < wave) pre = v9_mul<false, false, true>(pre, wt[w]);
+  if (carry) {
+    uint32_t c[9];
+    unpack_ext(fr_load(carry + blockIdx.x).l, c);
+    pre = v9_mul<false, false, true>(pre, c);
+  }
+  fr* dst = out_excl + b0 + t * kPer;
+  static_for<0, kPer>([&](auto k_) {
+    constexpr int k = decltype(k_)::value;
+    if (k < rem) {
+      fr ex;
+      if constexpr (k == 0) {
+        if constexpr (RF) {
+          ex = v9_canonical(pre);
+        } else {
+          uint32_t w[9];
+          unpack_ext(fr_one().l, w);
+          ex = v9_canonical(v9_mul<false, false, false>(pre, w));
+        }
+      } else {
+        uint32_t w[9];
+        pbd_unpack(e[k > 0 ? k - 1 : 0].l, w);
+        ex = v9_canonical(v9_mul<false, false, false>(pre, w));
+      }
+      fr_store(dst + k, ex);
+      if constexpr (!RF) {
+        // an inclusive output is the next element's exclusive one
+        if (out_incl) {
+          if constexpr (k > 0) fr_store(out_incl + b0 + t * kPer + k - 1, ex);
+          if (k == kPer - 1 || k == rem - 1) {
+            uint32_t w[9];
+            pbd_unpack(e[k].l, w);
+            fr_store(out_incl + b0 + t * kPer + k, v9_canonical(v9_mul<false, false, false>(pre, w)));
+          }
+        }
+      }
     }
   });
 }
@@ -156,26 +261,32 @@ static uint64_t pfx_scratch_elems(uint64_t n) {
   return tot + 1;
 }
 
-static hipError_t prefix_product(const fr* in, fr* out_excl, fr* out_incl, uint64_t n, fr* total, fr* scratch,
-                                 hipStream_t s) {
-  if (n <= (uint64_t)kScanThreads) {
-    hipLaunchKernelGGL(pfx_down_kernel<0>, dim3(1), dim3(kScanThreads), 0, s, in, out_excl, out_incl, n,
-                       (const fr*)nullptr, total);
-    return hipGetLastError();
-  }
+// the only block of a level: the smallest geometry that covers it
+template <bool RF>
+static void pfx_one_block(const fr* in, fr* out_excl, fr* out_incl, uint64_t n, hipStream_t s) {
+  const dim3 g(1), b(kScanThreads);
+  const fr* none = nullptr;
+  if (n <= 256) hipLaunchKernelGGL((pfx_down_kernel<0, RF>), g, b, 0, s, in, out_excl, out_incl, n, none);
+  else if (n <= 512) hipLaunchKernelGGL((pfx_down_kernel<1, RF>), g, b, 0, s, in, out_excl, out_incl, n, none);
+  else if (n <= 1024) hipLaunchKernelGGL((pfx_down_kernel<2, RF>), g, b, 0, s, in, out_excl, out_incl, n, none);
+  else if (n <= 2048) hipLaunchKernelGGL((pfx_down_kernel<3, RF>), g, b, 0, s, in, out_excl, out_incl, n, none);
+  else hipLaunchKernelGGL((pfx_down_kernel<kLgPer, RF>), g, b, 0, s, in, out_excl, out_incl, n, none);
+}
+
+template <bool RF>
+static hipError_t prefix_product(const fr* in, fr* out_excl, fr* out_incl, uint64_t n, fr* scratch, hipStream_t s) {
   if (n <= (uint64_t)kSeg) {
-    hipLaunchKernelGGL(pfx_down_kernel<kLgPer>, dim3(1), dim3(kScanThreads), 0, s, in, out_excl, out_incl, n,
-                       (const fr*)nullptr, total);
+    pfx_one_block<RF>(in, out_excl, out_incl, n, s);
     return hipGetLastError();
   }
   const uint64_t nb = (n + kSeg - 1) / kSeg;
   fr* part = scratch;
   fr* part_excl = scratch + nb;
-  hipLaunchKernelGGL(pfx_reduce_kernel<kLgPer>, dim3(sgrid(n)), dim3(kScanThreads), 0, s, in, n, part);
-  hipError_t e = prefix_product(part, part_excl, nullptr, nb, total, scratch + 2 * nb, s);
+  hipLaunchKernelGGL(pfx_reduce_kernel<RF>, dim3(sgrid(n)), dim3(kScanThreads), 0, s, in, n, part);
+  hipError_t e = prefix_product<true>(part, part_excl, nullptr, nb, scratch + 2 * nb, s);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(pfx_down_kernel<kLgPer>, dim3(sgrid(n)), dim3(kScanThreads), 0, s, in, out_excl, out_incl, n,
-                     (const fr*)part_excl, (fr*)nullptr);
+  hipLaunchKernelGGL((pfx_down_kernel<kLgPer, RF>), dim3(sgrid(n)), dim3(kScanThreads), 0, s, in, out_excl, out_incl,
+                     n, (const fr*)part_excl);
   return hipGetLastError();
 }
 
@@ -189,12 +300,6 @@ static hipError_t prefix_product(const fr* in, fr* out_excl, fr* out_incl, uint6
 
 // a * w R' / R' = a w (stored form), canonical
 __device__ __forceinline__ fr mulp(const fr& a, const fr& w) { return fr_reduce_once(fr_mul29(a, w)); }
-// R' mod r: the R'-form of one
-__host__ __device__ constexpr uint32_t rp_one_limb(int i) {
-  return i == 0 ? 0xffffffbau : i == 1 ? 0x00000045u : i == 2 ? 0x0072d846u : i == 3 ? 0x1a25272eu
-       : i == 4 ? 0x5dbeee8bu : i == 5 ? 0xfe2eedcdu : i == 6 ? 0x9eefbe41u : 0x4d043f42u;
-}
-
 // block suffix combine: V_t <- V_t + m^(2^LG * 2^s) V_{t+2^s}; returns the
 // suffix value starting at thread t (the block's carry folded in by the caller)
 template <int LG>
@@ -540,12 +645,6 @@ constexpr uint32_t kLatMaxG = 255;
 // division the upper-half Horner values H (256 G)
 constexpr uint64_t kWsA = 0, kWsB = 256, kWsP = 512, kWsPw = 768, kWsHalf = 784, kWsL = 800;
 
-__device__ __forceinline__ fr rp_one_fr() {
-  fr o;
-#pragma unroll
-  for (int i = 0; i < 8; i++) o.l[i] = rp_one_limb(i);
-  return o;
-}
 __device__ __forceinline__ fr to_rp(fr v) {  // x R (stored) -> x R' (five doublings)
   for (int d = 0; d < 5; d++) v = fr_add(v, v);
   return v;
@@ -846,7 +945,7 @@ uint64_t scan_scratch_elems(uint64_t n) {
 uint64_t grand_product_scratch_elems(uint64_t n) { return pfx_scratch_elems(n); }
 
 hipError_t grand_product(fr* inout, fr* incl_out, uint64_t n, fr* scratch, hipStream_t s) {
-  return prefix_product(inout, inout, incl_out, n, nullptr, scratch, s);
+  return prefix_product<false>(inout, inout, incl_out, n, scratch, s);
 }
 
 hipError_t div_linear(fr* inout, uint64_t n, const fr* c, fr* rem, fr* scratch, hipStream_t s) {
