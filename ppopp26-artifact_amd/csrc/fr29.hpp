@@ -472,6 +472,33 @@ __device__ __forceinline__ v9 v9_mul_rows(const v9& x, uwords w, rows_cols& g, u
   return t;
 }
 
+// 2^(29 (i + 2) + 5) mod r, balanced digits: lane i's factor in rows29_make
+static __constant__ const uint32_t kRowShift[9][9] = {
+    {0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u},
+    {0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u},
+    {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u},
+    {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u, 0x00000000u, 0x00000000u},
+    {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u, 0x00000000u},
+    {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u},
+    {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u},
+    {0xfffff72bu, 0x000046a8u, 0xff5f3540u, 0x0ce3021du, 0xf18f3661u, 0x008176ccu, 0x054e487cu, 0xf02e8190u, 0x001e092fu},
+    {0xf7b58901u, 0x0253af23u, 0x0135066au, 0x03f86fa7u, 0x00a56cd7u, 0xf391cf69u, 0x007feb85u, 0xf69dc586u, 0x0032509cu}};
+
+// The rows29 table (D = 2) of a factor known only on the device: m is x R
+// (any 256-bit word of the class) on every lane; lane i < 9 returns row W_i =
+// x 2^(29 (i + 2)) as balanced digits in (-1.04 r, 0.04 r), one product.  Beside
+// the centred rows of rows29_row the bound on T grows to 1.04 X / 2^58 r, which
+// D = 2 still makes (-1.001 r, 0.001 r).
+__device__ __forceinline__ v9 rows29_make(const fr& m) {
+  const int lane = threadIdx.x & 63;
+  uint32_t c[9];
+#pragma unroll
+  for (int j = 0; j < 9; j++) c[j] = kRowShift[lane < 9 ? lane : 0][j];
+  v9 x;
+  unpack_ext(m.l, x.l);
+  return v9_mul<false, false, true>(x, c);
+}
+
 // the canonical value in [0, r) of v (|v_i| < 2^31)
 __device__ __forceinline__ fr v9_canonical(const v9& v) {
   uint32_t t[9];

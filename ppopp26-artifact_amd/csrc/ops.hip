@@ -126,19 +126,6 @@ __device__ __forceinline__ fr mul_rp(const fr& a, const fr& b) {
   return v9_canonical(v9_mul<false, false, false>(x, y.l));
 }
 
-// P of two pbd words (values within 1.07 r), as a pbd word: the product lies
-// in (-1.02 r, 0.02 r) and its balanced digits fit
-__device__ __forceinline__ fr mul_pbd(const fr& a, const fr& b) {
-  v9 x;
-  uint32_t y[9];
-  pbd_unpack(a.l, x.l);
-  pbd_unpack(b.l, y);
-  const v9 t = v9_mul<false, false, true>(x, y);
-  fr o;
-  pbd_pack(t.l, o.l);
-  return o;
-}
-
 __device__ __forceinline__ v9 shfl_xor9(const v9& v, int m) {
   v9 o;
 #pragma unroll
@@ -184,29 +171,50 @@ __device__ __forceinline__ void block_others(v9& P, v9& E, v9& rest) {
 }
 
 // The exclusive prefix product of a and the exclusive suffix product of b
-// over the 256 thread values (pbd words), by Hillis-Steele steps with the two
-// scans interleaved: 8 levels of two independent products, every thread busy
-// (a missing partner multiplies by one).
-__device__ void block_scan2_short(fr& a, fr& b, uint4 (*la)[kOpThreads], uint4 (*lb)[kOpThreads], const fr one) {
-  const int t = threadIdx.x;
-  lds_put2(la, t, a);
-  lds_put2(lb, t, b);
-  __syncthreads();
-  for (int s = 1; s < kOpThreads; s <<= 1) {
-    const fr oa = t >= s ? lds_get2(la, t - s) : one;
-    const fr ob = t + s < kOpThreads ? lds_get2(lb, t + s) : one;
-    __syncthreads();
-    a = mul_pbd(a, oa);
-    b = mul_pbd(b, ob);
-    lds_put2(la, t, a);
-    lds_put2(lb, t, b);
-    __syncthreads();
+// over the 256 thread values (balanced digits, |value| < 1.1 r): six shuffle
+// steps inside the wave, two independent products each, then the wave products
+// of the waves before and after.  waves: how many waves hold values other than
+// one (a single-block level of at most 64 threads' values skips the meeting).
+__device__ __forceinline__ void block_scan2(v9& a, v9& b, const v9& one, int waves) {
+  __shared__ uint32_t wa[4][9], wb[4][9];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+#pragma unroll
+  for (int s = 1; s < 64; s <<= 1) {
+    v9 oa, ob;
+#pragma unroll
+    for (int i = 0; i < 9; i++) {
+      oa.l[i] = (uint32_t)__shfl_up((int)a.l[i], s);
+      ob.l[i] = (uint32_t)__shfl_down((int)b.l[i], s);
+    }
+    oa = v9_mul<false, false, true>(a, oa.l);
+    ob = v9_mul<false, false, true>(b, ob.l);
+    if (lane >= s) a = oa;
+    if (lane + s < 64) b = ob;
   }
-  const fr ea = t > 0 ? lds_get2(la, t - 1) : one;
-  const fr eb = t + 1 < kOpThreads ? lds_get2(lb, t + 1) : one;
+  if (waves > 1) {
+    if (lane == 63) {
+#pragma unroll
+      for (int i = 0; i < 9; i++) wa[w][i] = a.l[i];
+    }
+    if (lane == 0) {
+#pragma unroll
+      for (int i = 0; i < 9; i++) wb[w][i] = b.l[i];
+    }
+  }
   __syncthreads();
-  a = ea;
-  b = eb;
+#pragma unroll
+  for (int i = 0; i < 9; i++) {
+    const uint32_t ua = (uint32_t)__shfl_up((int)a.l[i], 1), ub = (uint32_t)__shfl_down((int)b.l[i], 1);
+    a.l[i] = lane > 0 ? ua : one.l[i];
+    b.l[i] = lane < 63 ? ub : one.l[i];
+  }
+  if (waves > 1) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      if (k < w) a = v9_mul<false, false, true>(a, wa[k]);
+      if (k > w) b = v9_mul<false, false, true>(b, wb[k]);
+    }
+  }
 }
 
 // Phase 1: total[b] = product over block b of in[i] (zeros taken as one).
@@ -415,6 +423,7 @@ struct RatioArgs {
   const fr* w0;  // w^i = w0[i & 16383] * w1[i >> 14]
   const fr* w1;
   fr* tab;       // [3][tstride] pbd words of (beta k_j w0[lo]) R' (perm_table_kernel)
+  uint32_t* brows;  // rows29 table of beta (perm_table_kernel)
   uint32_t tstride;  // min(n, 16384): the low-window entries in use
   fr k[3];
   fr k29[3];  // pbd words of (32 k_j) R' = 1024 k_j R mod r
@@ -429,40 +438,37 @@ struct RatioArgs {
 //   P(., (32 k) R')   = (beta k w0) R'            (host constant, pbd word)
 //     -- once per call for the 16384 low-window entries (perm_table_kernel) --
 //   P((beta k w0) R', S(w1)) = S(beta k w^i)      (w^i = w0[lo] w1[hi])
-//   P(S(s_j), beta R') = S(beta s_j)
+//   rows29(S(s_j), beta) = S(beta s_j)              (beta: the same for all lanes)
 // so n_j = S(w_j + gamma + beta k_j w^i) and d_j = S(w_j + gamma + beta s_j)
 // exactly, and the two products of three terms each carry 2^-10:
 // num = S(n_0 n_1 n_2 / 1024), den = S(d_0 d_1 d_2 / 1024), whose ratio is the
 // permutation ratio.  Limbs: the inputs are balanced digits (<= 2^28); the
 // three-term sums <= 3 2^28 (products with balanced outputs), so a product of
 // two of them stays below 81 2^56 + 2^61 < 2^62.8 per column.
-// per-thread constants of the terms: B = beta R' (= 32 S(beta)), g = gamma
-struct TermConsts {
-  uint32_t B[9];
-  v9 g;
-};
-__device__ __forceinline__ TermConsts term_consts(const RatioArgs& a) {
-  TermConsts c;
-  fr b32 = fr_load(a.beta);
-#pragma unroll
-  for (int d = 0; d < 5; d++) b32 = fr_add(b32, b32);
-  unpack_ext(b32.l, c.B);
-  unpack_ext(fr_load(a.gamma).l, c.g.l);
-  return c;
-}
-
 constexpr int kWin = 16384;  // entries of the low window table
-static uint64_t perm_table_elems(uint64_t n) { return 3 * std::min<uint64_t>(n, kWin); }
+constexpr uint64_t kBRows = (81 * sizeof(uint32_t) + sizeof(fr) - 1) / sizeof(fr);  // beta's rows29 table
+static uint64_t perm_table_elems(uint64_t n) { return 3 * std::min<uint64_t>(n, kWin) + kBRows; }
 
 // tab[j][lo] = P(P(S(w0[lo]), beta R'), (32 k_j) R') = (beta k_j w0[lo]) R', so
 // that P(tab[j][lo], S(w1[hi])) = S(beta k_j w^i)
 __global__ void __launch_bounds__(256) perm_table_kernel(RatioArgs a, uint32_t count) {
   const uint32_t lo = blockIdx.x * blockDim.x + threadIdx.x;
+  if (blockIdx.x == 0 && threadIdx.x < 64) {
+    const v9 r = rows29_make(fr_load(a.beta));
+    if (threadIdx.x < 9) {
+#pragma unroll
+      for (int j = 0; j < 9; j++) a.brows[9 * j + threadIdx.x] = r.l[j];
+    }
+  }
   if (lo >= count) return;
-  const TermConsts c = term_consts(a);
+  fr b32 = fr_load(a.beta);  // beta R' = 32 S(beta)
+#pragma unroll
+  for (int d = 0; d < 5; d++) b32 = fr_add(b32, b32);
+  uint32_t b[9];
+  unpack_ext(b32.l, b);
   v9 w;
   unpack_ext(fr_load(a.w0 + lo).l, w.l);
-  const v9 bw = v9_mul<false, false, false>(w, c.B);
+  const v9 bw = v9_mul<false, false, false>(w, b);
 #pragma unroll
   for (int j = 0; j < 3; j++) {
     uint32_t K[9];
@@ -491,9 +497,15 @@ __device__ __forceinline__ void v9_carry_balanced(v9& v) {
 // (|t_i| <= 2^28), so 7 t_i fits a signed limb; carried back to balanced
 // digits, 7 t plus 6 t fits again (13 t = 7 t + 6 t); each carried value is
 // the same integer, so n_j = w_j + gamma + k_j t keeps the three-term bound.
+// beta s_j takes beta as a wave-uniform factor (rows29): 117 VALU instructions
+// of about 205, and beta's digits leave the vector registers (131 -> 95,
+// five waves per SIMD instead of three; 2^20 rows 104 -> 95 us).
 template <bool SK>
-__device__ __forceinline__ void perm_terms_at(const RatioArgs& a, const TermConsts& c, uint64_t i, v9& num,
-                                              v9& den) {
+__device__ __forceinline__ void perm_terms_at(const RatioArgs& a, uint64_t i, v9& num, v9& den) {
+  const uwords B = (uwords)a.brows;
+  rows_cols g0 = rows29_open(B, 0);
+  v9 gam;
+  unpack_ext(fr_load(a.gamma).l, gam.l);
   v9 w1;
   unpack_ext(fr_load(a.w1 + (i >> 14)).l, w1.l);
   v9 t1, t7;  // SK: beta w^i, then 7 beta w^i (balanced digits)
@@ -501,7 +513,7 @@ __device__ __forceinline__ void perm_terms_at(const RatioArgs& a, const TermCons
   for (int j = 0; j < 3; j++) {
     v9 wj, sj;
     unpack_ext(fr_load(a.w[j] + i).l, wj.l);
-    const v9 wg = v9_add(wj, c.g);
+    const v9 wg = v9_add(wj, gam);
     v9 kt;
     if (!SK || j == 0) {
       uint32_t K[9];
@@ -520,7 +532,7 @@ __device__ __forceinline__ void perm_terms_at(const RatioArgs& a, const TermCons
     }
     const v9 nj = v9_add(wg, kt);
     unpack_ext(fr_load(a.s[j] + i).l, sj.l);
-    const v9 dj = v9_add(wg, v9_mul<false, false, true>(sj, c.B));
+    const v9 dj = v9_add(wg, v9_mul_rows<2, true>(sj, B, g0, B));
     num = j == 0 ? nj : v9_mul<false, false, false>(num, nj.l);  // the first factor needs no product
     den = j == 0 ? dj : v9_mul<false, false, false>(den, dj.l);
   }
@@ -537,17 +549,15 @@ __global__ void __launch_bounds__(256) perm_terms_kernel(RatioArgs a, fr* rn, fr
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if constexpr (!ZERO_DEN) {
     if (i >= a.n) return;
-    const TermConsts c = term_consts(a);
     v9 num, den;
-    perm_terms_at<SK>(a, c, i, num, den);
+    perm_terms_at<SK>(a, i, num, den);
     fr_store(a.num + i, v9_canonical(num));
     fr_store(a.den + i, v9_canonical(den));
   } else {
     fr nw = rp_one(), dw = rp_one();
     if (i < a.n) {
-      const TermConsts c = term_consts(a);
       v9 num, den;
-      perm_terms_at<SK>(a, c, i, num, den);
+      perm_terms_at<SK>(a, i, num, den);
       nw = v9_canonical(num);
       dw = v9_canonical(den);
       if (fr_is_zero(dw)) {
@@ -602,44 +612,39 @@ __global__ void __launch_bounds__(256) perm_terms_kernel(RatioArgs a, fr* rn, fr
 
 // Up-sweep over one level: thread products of num and den over each
 // thread's 8 consecutive elements (tn, td: one per thread of every block, for
-// the down-sweep) and the block products (bn, bd).
-__global__ void __launch_bounds__(kOpThreads) gp_up_kernel(const fr* nv, const fr* dv, uint64_t n, fr* tn, fr* td,
-                                                            fr* bn, fr* bd) {
-  __shared__ uint4 ln[2][kOpThreads], ld[2][kOpThreads];
-  const int t = threadIdx.x;
+// the down-sweep) and the block products (bn, bd).  Half the block's 512
+// threads take num and half den: at 2^20 the level is 64 blocks, one wave per
+// SIMD and both chains in turn with 256 threads (27.6 us), two waves and half
+// the chain with 512 (18.8 us).
+constexpr int kUpThreads = 2 * kOpThreads;
+__global__ void __launch_bounds__(kUpThreads) gp_up_kernel(const fr* nv, const fr* dv, uint64_t n, fr* tn, fr* td,
+                                                           fr* bn, fr* bd) {
+  __shared__ uint32_t wt[kUpThreads / 64][9];
+  const int t = threadIdx.x & (kOpThreads - 1), w = threadIdx.x >> 6;
+  const bool den = w >= 4;
   const uint64_t tid = (uint64_t)blockIdx.x * kOpThreads + t;
   const uint64_t base = tid * kOpPer;
-  v9 pn, pd;
+  const fr* src = den ? dv : nv;
+  v9 p;
   static_for<0, kOpPer>([&](auto k_) {
     constexpr int k = decltype(k_)::value;
-    const bool live = base + k < n;
-    const fr nw = live ? fr_load(nv + base + k) : rp_one();
-    const fr dw = live ? fr_load(dv + base + k) : rp_one();
-    v9 x, y;
-    unpack_ext(nw.l, x.l);
-    unpack_ext(dw.l, y.l);
-    pn = k == 0 ? x : v9_mul<false, false, false>(pn, x.l);
-    pd = k == 0 ? y : v9_mul<false, false, false>(pd, y.l);
+    const fr v = base + k < n ? fr_load(src + base + k) : rp_one();
+    v9 x;
+    unpack_ext(v.l, x.l);
+    p = k == 0 ? x : v9_mul<false, false, true>(p, x.l);
   });
-  fr cn = v9_canonical(pn), cd = v9_canonical(pd);
-  fr_store(tn + tid, cn);
-  fr_store(td + tid, cd);
-  lds_put2(ln, t, cn);
-  lds_put2(ld, t, cd);
+  fr_store((den ? td : tn) + tid, v9_canonical(p));
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) p = v9_mul<false, false, true>(p, shfl_xor9(p, m).l);
+  if ((t & 63) == 0) {
+#pragma unroll
+    for (int i = 0; i < 9; i++) wt[w][i] = p.l[i];
+  }
   __syncthreads();
-  for (int s = kOpThreads / 2; s > 0; s >>= 1) {
-    if (t < s) {
-      cn = mul_rp(cn, lds_get2(ln, t + s));
-      cd = mul_rp(cd, lds_get2(ld, t + s));
-      lds_put2(ln, t, cn);
-      lds_put2(ld, t, cd);
-    }
-    __syncthreads();
-  }
-  if (t == 0) {
-    fr_store(bn + blockIdx.x, cn);
-    fr_store(bd + blockIdx.x, cd);
-  }
+  if (t >= 64) return;  // wave 0 folds num, wave 4 den
+#pragma unroll
+  for (int k = 1; k < 4; k++) p = v9_mul<false, false, true>(p, wt[w + k]);
+  if (t == 0) fr_store((den ? bd : bn) + blockIdx.x, v9_canonical(p));
 }
 
 // 32 fr_inv_wave(total): the R'-view word of 1 / (32 total / R'); by a whole
@@ -664,16 +669,12 @@ __device__ __forceinline__ void gp_down_body(const fr* nv, const fr* dv, const f
                                              const fr* carry, fr* out, fr* tot,
                                              uint32_t blk) {
   constexpr int kPer = 1 << LG;
-  __shared__ uint4 l[2][kOpThreads], l2[2][kOpThreads];
   __shared__ uint32_t cinv[8];
   const int t = threadIdx.x;
   const uint64_t tid = (uint64_t)blk * kOpThreads + t;
   const uint64_t base = tid * kPer;
-  fr one;
-  {
-    const fr o = rp_one();
-    to_pbd(o.l, one.l);
-  }
+  v9 one;
+  unpack_ext(rp_one().l, one.l);
   // local den suffixes S[k] (pbd words; a product of a value below 1.07 r and
   // one below r lies in (-1.07 r, 0.07 r))
   fr S[kPer];
@@ -688,7 +689,7 @@ __device__ __forceinline__ void gp_down_body(const fr* nv, const fr* dv, const f
       pbd_pack(acc.l, S[k].l);
     } else {
       if constexpr (k == kPer - 1) {
-        S[k] = one;
+        pbd_pack(one.l, S[k].l);
         acc = y;
       } else {
         pbd_pack(acc.l, S[k].l);
@@ -696,41 +697,29 @@ __device__ __forceinline__ void gp_down_body(const fr* nv, const fr* dv, const f
       }
     }
   });
-  // acc: the thread's den product
-  fr tnw, tdw;
+  // acc: the thread's den product; num's likewise
+  v9 pre, suf;
   if constexpr (TOP) {
-    v9 pn;
     static_for<0, kPer>([&](auto k_) {
       constexpr int k = decltype(k_)::value;
       const fr nw = base + k < n ? fr_load(nv + base + k) : rp_one();
       v9 x;
       unpack_ext(nw.l, x.l);
-      pn = k == 0 ? x : v9_mul<false, false, false>(pn, x.l);
+      pre = k == 0 ? x : v9_mul<false, false, true>(pre, x.l);
     });
-    pbd_pack(acc.l, tdw.l);
-    if constexpr (kPer == 1) {
-      pbd_pack(pn.l, tnw.l);  // balanced digits of a canonical value
-    } else {
-      uint32_t b[9];
-      reduce_centered(pn.l, b);
-      pbd_pack(b, tnw.l);
-    }
+    suf = acc;
   } else {
-    to_pbd(fr_load(tn + tid).l, tnw.l);
-    to_pbd(fr_load(td + tid).l, tdw.l);
+    unpack_ext(fr_load(tn + tid).l, pre.l);
+    unpack_ext(fr_load(td + tid).l, suf.l);
   }
-  fr pre = tnw, suf = tdw;
-  block_scan2_short(pre, suf, l, l2, one);
+  const v9 mine = suf;
+  block_scan2(pre, suf, one, TOP ? (int)((n + 64 * kPer - 1) / (64 * kPer)) : 4);
   fr cw;
   if constexpr (TOP) {
     if (t < 64) {
       // total den product = suf_0 x (thread 0's product): lane 0's value
       // (wave 0 runs it whole for the wave-wide inversion)
-      v9 a;
-      uint32_t b[9];
-      pbd_unpack(suf.l, a.l);
-      pbd_unpack(tdw.l, b);
-      const fr total = v9_canonical(v9_mul<false, false, false>(a, b));
+      const fr total = v9_canonical(v9_mul<false, false, false>(suf, mine.l));
       fr z;
       if (tot) {
         if (t == 0) fr_store(tot, total);  // inverted by gp_inverse beside the next sweep
@@ -752,11 +741,8 @@ __device__ __forceinline__ void gp_down_body(const fr* nv, const fr* dv, const f
   v9 cur;
   {
     v9 a;
-    uint32_t b[9], c[9];
     unpack_ext(cw.l, a.l);
-    pbd_unpack(pre.l, b);
-    pbd_unpack(suf.l, c);
-    cur = v9_mul<false, false, false>(v9_mul<false, false, false>(a, b), c);
+    cur = v9_mul<false, false, false>(v9_mul<false, false, false>(a, pre.l), suf.l);
   }
   static_for<0, kPer>([&](auto k_) {
     constexpr int k = decltype(k_)::value;
@@ -993,6 +979,7 @@ static RatioArgs ratio_args(const fr* const w[3], const fr* const sg[3], const f
   a.w0 = w0;
   a.w1 = w1;
   a.tab = nullptr;
+  a.brows = nullptr;
   a.tstride = 0;
   a.num = nullptr;
   a.den = nullptr;
@@ -1019,6 +1006,7 @@ static void perm_tables(RatioArgs& a, fr*& scratch, hipStream_t s) {
   a.tab = scratch;
   a.tstride = count;
   scratch += perm_table_elems(a.n);
+  a.brows = (uint32_t*)(scratch - kBRows);
   hipLaunchKernelGGL(perm_table_kernel, dim3((count + 255) / 256), dim3(256), 0, s, a, count);
 }
 
@@ -1072,7 +1060,7 @@ hipError_t perm_grand_product(const fr* const w[3], const fr* const sg[3], const
     fr* bn = p;
     fr* bd = p + nb;
     p += 2 * nb;
-    hipLaunchKernelGGL(gp_up_kernel, dim3((unsigned)nb), dim3(kOpThreads), 0, s, (const fr*)c.nv, (const fr*)c.dv,
+    hipLaunchKernelGGL(gp_up_kernel, dim3((unsigned)nb), dim3(kUpThreads), 0, s, (const fr*)c.nv, (const fr*)c.dv,
                        c.n, c.tn, c.td, bn, bd);
     lv[++top] = {bn, bd, nullptr, nullptr, nb};
   }
