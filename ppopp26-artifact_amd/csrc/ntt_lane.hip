@@ -42,6 +42,7 @@ struct LaneArgs {
   const fr* premul;     // optional factor per input element [(poly & pm_mask) << lgN | pos], pbd words of c R'
   const fr* lin;        // w_N^e, e < N, pbd words of w R'
   const fr* fin;        // (s, s i^k), k < 4: s = 1, or 1/N for the inverse (pbd words times R')
+  const fr* post;       // LAST: such pairs per output index instead (NttCall::post), or null
   uint64_t in_pstride;  // element stride between input polys (0: shared input)
   uint64_t nlines;
   uint32_t pm_mask;
@@ -151,8 +152,9 @@ __global__ void __launch_bounds__(lane_threads(m), 4) ntt_lane_kernel(LaneArgs a
       twiddle(std::integral_constant<int, s + 1>(), w1, w2);
     } else if constexpr (s + 1 < NS) {
       if constexpr (LAST) {
-        w1 = fr_load(a.fin + 2 * (tau & 3));
-        w2 = fr_load(a.fin + 2 * (tau & 3) + 1);
+        const fr* f = a.post ? a.post + 2 * (lp + (kappa << lgL)) : a.fin + 2 * (tau & 3);
+        w1 = fr_load(f);
+        w2 = fr_load(f + 1);
       } else {
         // w_N^(J kappa), and times i^k
         w1 = lin(lp * kappa);
@@ -252,6 +254,28 @@ hipError_t lane_tables(Domain& d, fr* fin, hipStream_t s) {
   return hipGetLastError();
 }
 
+// one thread per output index i; its last digit k is i's top two bits
+__global__ void __launch_bounds__(256) lane_post_kernel(const fr* f, fr* post, const fr* w256i, fr n_inv32, uint32_t lg) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >> lg) return;
+  const fr s = fr_mul(fr_load(f + i), n_inv32);
+  const fr v = fr_mul(s, fr_load(w256i + 64 * (i >> (lg - 2))));
+  fr o;
+  to_pbd(s.l, o.l);
+  fr_store(post + 2 * i, o);
+  to_pbd(v.l, o.l);
+  fr_store(post + 2 * i + 1, o);
+}
+
+hipError_t lane_post_table(const Domain& d, const fr* f, fr* post, hipStream_t s) {
+  fr n_inv32;
+  const host::fr64 h = host::mul(d.n_inv, host::from_u64(32));
+  memcpy(n_inv32.l, h.l, 32);
+  hipLaunchKernelGGL(lane_post_kernel, dim3(((1u << d.lg) + 255) / 256), dim3(256), 0, s, f, post,
+                     (const fr*)d.inner_inv, n_inv32, (uint32_t)d.lg);
+  return hipGetLastError();
+}
+
 bool lane_form(const Domain& d, const NttCall& c) {
   const uint64_t n = (uint64_t)c.npoly << d.lg;
   return d.lane_lin && (n <= 1ull << 18 || (d.lg > 12 && n < 1ull << 19));
@@ -285,6 +309,7 @@ hipError_t lane_launch(const Domain& d, const NttCall& c, hipStream_t s) {
     a.in_ext = 0;
   }
   a.out = c.out;
+  a.post = c.post;
   a.nlines = one ? c.npoly : (uint64_t)c.npoly << (lg - m1);
   launch_lane_m(one ? m0 : m1, true, a, s);
   return hipGetLastError();

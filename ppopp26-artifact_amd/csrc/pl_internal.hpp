@@ -87,6 +87,9 @@ struct NttCall {
   uint32_t pm_mask = 0;
   uint32_t lgI = 0;            // output interleave: out[(pos << lgI) + (poly & (2^lgI-1))]
   bool inverse = false;
+  // lane form, inverse: factor pairs of the last step per output index in place
+  // of the domain's (lane_post_table), or null
+  const fr* post = nullptr;
 };
 
 // The one-element-per-lane form: whole transforms of 2^4 .. 2^kLaneMaxLg
@@ -101,6 +104,9 @@ constexpr int kLaneMaxLg = 18, kLaneOne = 9;
 constexpr int kLaneFin = 16;  // elements of the factor pairs
 hipError_t lane_tables(Domain& d, fr* fin, hipStream_t s);
 bool lane_form(const Domain& d, const NttCall& c);
+// post[2 i], post[2 i + 1] = the inverse transform's last factor pair of output
+// i times f[i] (stored form), i < N: the transform then leaves f[i] x_i
+hipError_t lane_post_table(const Domain& d, const fr* f, fr* post, hipStream_t s);
 hipError_t lane_launch(const Domain& d, const NttCall& c, hipStream_t s);
 
 hipError_t ntt_launch(const Domain& d, const NttCall& c, hipStream_t s);

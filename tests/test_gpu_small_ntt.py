@@ -63,3 +63,18 @@ def test_any_256_bit_words(pl):
         for inverse in (False, True):
             np.testing.assert_array_equal(pl.to_host(pl.ntt(pl.to_dev(x), dom, inverse=inverse)),
                                           po.ntt(y, lg, inverse=inverse))
+
+
+@pytest.mark.parametrize("lg", [4, 5, 8, 9, 10, 11, 14, 17, 18])
+def test_coset_inverse(pl, lg):
+    # the coset powers ride on the last step's factors
+    for shift in (None, po.uniform(1, 99)):
+        dom = pl.CosetDomain(lg, shift)
+        g = po.from_u64(7) if shift is None else shift
+        x = po.uniform(1 << lg, po.seed(po.OP_INTT, lg, 3))
+        print("lane form inverse coset", lg, flush=True)
+        xd = pl.to_dev(x)
+        ref = po.coset_intt(x, lg, g)
+        np.testing.assert_array_equal(pl.to_host(pl.coset_ntt(xd, dom, inverse=True)), ref)
+        pl.coset_ntt(xd, dom, inverse=True, out=xd)
+        np.testing.assert_array_equal(pl.to_host(xd), ref)
