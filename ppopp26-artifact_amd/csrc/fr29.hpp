@@ -472,31 +472,80 @@ __device__ __forceinline__ v9 v9_mul_rows(const v9& x, uwords w, rows_cols& g, u
   return t;
 }
 
-// 2^(29 (i + 2) + 5) mod r, balanced digits: lane i's factor in rows29_make
-static __constant__ const uint32_t kRowShift[9][9] = {
-    {0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u},
-    {0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u},
-    {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u},
-    {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u, 0x00000000u, 0x00000000u},
-    {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u, 0x00000000u},
-    {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u},
-    {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u},
-    {0xfffff72bu, 0x000046a8u, 0xff5f3540u, 0x0ce3021du, 0xf18f3661u, 0x008176ccu, 0x054e487cu, 0xf02e8190u, 0x001e092fu},
-    {0xf7b58901u, 0x0253af23u, 0x0135066au, 0x03f86fa7u, 0x00a56cd7u, 0xf391cf69u, 0x007feb85u, 0xf69dc586u, 0x0032509cu}};
+// 2^(29 (i + 2) + 5) and 2^(29 (i + 2)) mod r, balanced digits: lane i's factor
+// in rows29_make
+static __constant__ const uint32_t kRowShift[2][9][9] = {
+    {
+     {0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u},
+     {0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u},
+     {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u},
+     {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u, 0x00000000u, 0x00000000u},
+     {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u, 0x00000000u},
+     {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u, 0x00000000u},
+     {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000020u},
+     {0xfffff72bu, 0x000046a8u, 0xff5f3540u, 0x0ce3021du, 0xf18f3661u, 0x008176ccu, 0x054e487cu, 0xf02e8190u, 0x001e092fu},
+     {0xf7b58901u, 0x0253af23u, 0x0135066au, 0x03f86fa7u, 0x00a56cd7u, 0xf391cf69u, 0x007feb85u, 0xf69dc586u, 0x0032509cu}},
+    {
+     {0x00000000u, 0x00000000u, 0x00000001u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u},
+     {0x00000000u, 0x00000000u, 0x00000000u, 0x00000001u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u},
+     {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000001u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u},
+     {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000001u, 0x00000000u, 0x00000000u, 0x00000000u},
+     {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000001u, 0x00000000u, 0x00000000u},
+     {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000001u, 0x00000000u},
+     {0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000000u, 0x00000001u},
+     {0xffffffb9u, 0x00000238u, 0xfd1f11c0u, 0x0f065601u, 0xf1685c66u, 0x0ae2aa0fu, 0x03e72bd4u, 0xfdeeaa48u, 0xffd91698u},
+     {0x0abdac48u, 0x0a129d79u, 0x070cf035u, 0xfb45834du, 0xf81928bdu, 0xfd3c6e55u, 0xf65af8f5u, 0xf461c48fu, 0xfffdf318u}}};
 
-// The rows29 table (D = 2) of a factor known only on the device: m is x R
-// (any 256-bit word of the class) on every lane; lane i < 9 returns row W_i =
-// x 2^(29 (i + 2)) as balanced digits in (-1.04 r, 0.04 r), one product.  Beside
-// the centred rows of rows29_row the bound on T grows to 1.04 X / 2^58 r, which
+// The rows29 table (D = 2) of a factor known only on the device, one product:
+// m is the word of x in stored form (RP false: x R) or R'-form (RP true: x R'),
+// any 256-bit word of the class, the same on every lane; lane i < 9 returns row
+// W_i = x 2^(29 (i + 2)) as balanced digits in (-1.04 r, 0.04 r).  Beside the
+// centred rows of rows29_row the bound on T grows to 1.04 X / 2^58 r, which
 // D = 2 still makes (-1.001 r, 0.001 r).
+template <bool RP>
 __device__ __forceinline__ v9 rows29_make(const fr& m) {
   const int lane = threadIdx.x & 63;
   uint32_t c[9];
 #pragma unroll
-  for (int j = 0; j < 9; j++) c[j] = kRowShift[lane < 9 ? lane : 0][j];
+  for (int j = 0; j < 9; j++) c[j] = kRowShift[RP ? 1 : 0][lane < 9 ? lane : 0][j];
   v9 x;
   unpack_ext(m.l, x.l);
   return v9_mul<false, false, true>(x, c);
+}
+
+// all 81 words of a factor in SGPRs, for a loop that multiplies by nothing else
+struct rows_all {
+  uint32_t w[81];
+};
+// from rows29_make's lanes
+__device__ __forceinline__ rows_all rows29_spread(const v9& r) {
+  rows_all a;
+#pragma unroll
+  for (int i = 0; i < 9; i++)
+#pragma unroll
+    for (int j = 0; j < 9; j++) a.w[9 * j + i] = (uint32_t)__builtin_amdgcn_readlane((int)r.l[j], i);
+  return a;
+}
+// x w (rows29, D = 2) for the factor held whole
+template <bool BT>
+__device__ __forceinline__ v9 v9_mul_all(const v9& x, const rows_all& a) {
+  constexpr int D = 2;
+  v9 t;
+  uint32_t m[D];
+  uint64_t acc[9 + D];
+  static_for<0, 8 + D>([&](auto k_) {
+    constexpr int k = decltype(k_)::value;
+    constexpr bool RND = BT && k - 1 >= D;
+    Rows29Col<k, D, RND>::run(acc[k], k ? acc[k ? k - 1 : 0] : 0, x.l, a.w + (k <= 8 ? 9 * k : 0), m);
+    const uint32_t lo = (uint32_t)acc[k];
+    if constexpr (k < D)
+      m[k] = lo & kMask29;
+    else
+      t.l[k - D] = BT ? sext29(lo) : (lo & kMask29);
+  });
+  Rows29Col<8 + D, D, BT>::run(acc[8 + D], acc[7 + D], x.l, a.w, m);
+  t.l[8] = (uint32_t)acc[8 + D];
+  return t;
 }
 
 // the canonical value in [0, r) of v (|v_i| < 2^31)

@@ -454,7 +454,7 @@ static uint64_t perm_table_elems(uint64_t n) { return 3 * std::min<uint64_t>(n, 
 __global__ void __launch_bounds__(256) perm_table_kernel(RatioArgs a, uint32_t count) {
   const uint32_t lo = blockIdx.x * blockDim.x + threadIdx.x;
   if (blockIdx.x == 0 && threadIdx.x < 64) {
-    const v9 r = rows29_make(fr_load(a.beta));
+    const v9 r = rows29_make<false>(fr_load(a.beta));
     if (threadIdx.x < 9) {
 #pragma unroll
       for (int j = 0; j < 9; j++) a.brows[9 * j + threadIdx.x] = r.l[j];

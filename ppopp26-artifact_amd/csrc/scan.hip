@@ -319,19 +319,24 @@ __device__ fr block_suffix(fr v, uint4 (*l)[kScanThreads], const fr* pw) {
   return v;
 }
 
-// sum_k v_k w^k by Horner in signed limbs (fr29.hpp): h <- P(h, w R') + v_k,
-// limb-wise sums of a product (digits in [0, 2^29)) and balanced digits, so
-// every limb stays below 2^30 and the value within (-r, 1.02 r); canonical
-// once at the end.  w9: balanced digits of w R'.
+// the factor of the word w R' for a whole kernel's Horner steps
+__device__ __forceinline__ rows_all rp_rows(const fr* w) { return rows29_spread(rows29_make<true>(fr_load(w))); }
+
+// sum_k v_k w^k by Horner in signed limbs (fr29.hpp): h <- h w + v_k with the
+// wave-uniform w held as rows in SGPRs (about 150 VALU instructions per step,
+// 225 with w per lane; evaluation of 2^24 176 -> 154 us, of 2^20 24.9 -> 22.3,
+// division 598 -> 565 and 52.7 -> 48.7), limb-wise sums of a product (digits in [0, 2^29)) and
+// balanced digits, so every limb stays below 2^30 and the product within
+// (-1.001 r, 0.001 r); canonical once at the end.
 template <int K>
-__device__ __forceinline__ fr horner29(const fr (&v)[K], const uint32_t (&w9)[9]) {
+__device__ __forceinline__ fr horner29(const fr (&v)[K], const rows_all& w) {
   v9 h;
   unpack_ext(v[K - 1].l, h.l);
   static_for<0, K - 1>([&](auto k_) {
     constexpr int k = K - 2 - decltype(k_)::value;
     v9 x;
     unpack_ext(v[k].l, x.l);
-    h = v9_add(v9_mul<false, false, false>(h, w9), x);
+    h = v9_add(v9_mul_all<false>(h, w), x);
   });
   return v9_canonical(h);
 }
@@ -371,8 +376,7 @@ __global__ void __launch_bounds__(kScanThreads) sfx_reduce_kernel(const fr* a, u
     blk--;
   }
   const uint64_t b0 = (uint64_t)blk << kLgSeg;
-  uint32_t M[9];
-  unpack_ext(fr_load(pw + 8).l, M);  // m^256, balanced digits
+  const rows_all M = rp_rows(pw + 8);  // m^256
   fr v[kPer];
   static_for<0, kPer>([&](auto k_) {
     constexpr int k = decltype(k_)::value;
@@ -424,8 +428,7 @@ __global__ void __launch_bounds__(kScanThreads) sfx_run_reduce_kernel(const fr* 
   }
   const uint64_t tid = (uint64_t)blk * kScanThreads + t;
   const uint64_t base = tid * kPer;
-  uint32_t m[9];
-  unpack_ext(fr_load(pw).l, m);  // balanced digits
+  const rows_all m = rp_rows(pw);
   fr e[kPer];
   static_for<0, kPer>([&](auto k_) {
     constexpr int k = decltype(k_)::value;
@@ -449,8 +452,7 @@ __global__ void __launch_bounds__(kScanThreads) sfx_down_kernel(const fr* a, fr*
   __shared__ uint4 l[2][kScanThreads];
   const int t = threadIdx.x;
   const uint64_t base = ((uint64_t)blockIdx.x << kLgSeg) + (uint64_t)t * kPer;
-  uint32_t m[9];
-  unpack_ext(fr_load(pw).l, m);  // balanced digits
+  const v9 row = rows29_make<true>(fr_load(pw));  // m's rows, spread where they are used
   // local Horner: L = sum_k e_k m^k
   fr h;
   if constexpr (LT) {
@@ -461,7 +463,7 @@ __global__ void __launch_bounds__(kScanThreads) sfx_down_kernel(const fr* a, fr*
       constexpr int k = decltype(k_)::value;
       e[k] = base + k < n ? fr_load(a + base + k) : fr_zero();
     });
-    h = horner29<kPer>(e, m);
+    h = horner29<kPer>(e, rows29_spread(row));
   }
   // fold the block carry into the last thread: s(start of thread 255) = L + m^kPer K
   fr K = carry ? fr_load(carry + blockIdx.x) : fr_zero();
@@ -474,6 +476,7 @@ __global__ void __launch_bounds__(kScanThreads) sfx_down_kernel(const fr* a, fr*
   // canonical where stored); out may equal a: each half's elements are read
   // before its outputs are written, and the low half's outputs only overwrite
   // elements already read
+  const rows_all m = rows29_spread(row);
   v9 sn;
   unpack_ext(cin.l, sn.l);
   constexpr int G = kPer > 1 ? 2 : 1, Q = kPer / G;
@@ -490,7 +493,7 @@ __global__ void __launch_bounds__(kScanThreads) sfx_down_kernel(const fr* a, fr*
       if constexpr (k > 0) {
         v9 x;
         unpack_ext(e[top - k].l, x.l);
-        sn = v9_add(v9_mul<false, false, false>(sn, m), x);
+        sn = v9_add(v9_mul_all<false>(sn, m), x);
       }
     });
   });
@@ -620,8 +623,7 @@ static hipError_t suffix_scan(const fr* a, fr* out, uint64_t n, const fr* pw, fr
 //             Horner value L = sum_k a_k m^k, which needs m alone;
 //             table block 0 (on a CU of its own: G + 1 <= 256 blocks) raises
 //             m: mu = m^K, its squares mu^(2^s), A_j = mu^j (j < 256) and
-//             B_b = mu^(256 b) (b < G), by doubling steps that follow the
-//             squaring chain;
+//             B_b = mu^(256 b) (b < G), multiplied up as the squares appear;
 //   evaluation (m = x)
 //   launch 2  block b: P_b = B_b sum_t L_(256 b + t) A_t;
 //   launch 3  y = sum_b P_b;
@@ -645,15 +647,17 @@ constexpr uint32_t kLatMaxG = 255;
 // division the upper-half Horner values H (256 G)
 constexpr uint64_t kWsA = 0, kWsB = 256, kWsP = 512, kWsPw = 768, kWsHalf = 784, kWsL = 800;
 
-__device__ __forceinline__ fr to_rp(fr v) {  // x R (stored) -> x R' (five doublings)
-  for (int d = 0; d < 5; d++) v = fr_add(v, v);
-  return v;
-}
-// the multiplier m R' of a scan: x, or -c for a division by X + c
+// the multiplier of a scan in stored form: x, or -c for a division by X + c
 __device__ __forceinline__ fr load_m(const fr* x, int neg) {
-  fr m = fr_load(x);
-  if (neg) m = fr_neg(m);
-  return to_rp(m);
+  const fr m = fr_load(x);
+  return neg ? fr_neg(m) : m;
+}
+// m R' as balanced digits within (-0.51 r, 0.51 r)
+__device__ __forceinline__ v9 m_rp(const fr& m) {
+  v9 a, b;
+  split29_x32(m.l, a.l);
+  reduce_centered(a.l, b.l);
+  return b;
 }
 
 // Horner over a run held in registers, each element's digit split ordered
@@ -662,7 +666,7 @@ __device__ __forceinline__ fr load_m(const fr* x, int neg) {
 // them instead of all at once
 // *upper (if not null): the value after the upper half, sum_(k >= K/2) a_k m^(k - K/2)
 template <int K>
-__device__ __forceinline__ fr horner29_inorder(fr (&v)[K], const uint32_t (&w9)[9], fr* upper) {
+__device__ __forceinline__ fr horner29_inorder(fr (&v)[K], const rows_all& w, fr* upper) {
   v9 h;
   unpack_ext(v[K - 1].l, h.l);
   static_for<0, K - 1>([&](auto k_) {
@@ -672,7 +676,7 @@ __device__ __forceinline__ fr horner29_inorder(fr (&v)[K], const uint32_t (&w9)[
                  "+v"(e.l[6]), "+v"(e.l[7]) : "v"(h.l[0]));
     v9 xv;
     unpack_ext(e.l, xv.l);
-    h = v9_add(v9_mul<false, false, false>(h, w9), xv);
+    h = v9_add(v9_mul_all<false>(h, w), xv);
     if constexpr (k == K / 2) {
       if (upper) *upper = v9_canonical(h);
     }
@@ -697,7 +701,7 @@ __device__ __forceinline__ void load_run(const fr* a, uint64_t n, uint64_t base,
   }
 }
 
-// launch 1; steps: doubling steps of the table block (8 for A, then B's);
+// launch 1; steps: squares of mu the table block raises (8 for A, then B's);
 // halves (division): also the upper-half Horner value of every run and m^(K/2)
 template <int K>
 __global__ void __launch_bounds__(kScanThreads) lat_runs_kernel(const fr* a, uint64_t n, const fr* x, int neg,
@@ -705,60 +709,103 @@ __global__ void __launch_bounds__(kScanThreads) lat_runs_kernel(const fr* a, uin
   static_assert(K % 2 == 0, "runs split in two halves");
   const int t = threadIdx.x;
   if (blockIdx.x == 0) {
-    // ---- table block: wave 0 squares mu, waves 1..3 extend A, then B ----
-    __shared__ fr pw_s[16];
-    __shared__ fr tab[2][256];
-    const int w = t >> 6;
-    if (w == 0) {
-      const fr xp = load_m(x, neg);
-      fr mu = xp;  // m^K R', left to right; K is even, so m^(K/2) precedes the last squaring
-      for (int bit = 30 - __builtin_clz(K); bit >= 0; bit--) {
-        if (bit == 0 && t == 0) fr_store(ws + kWsHalf, mu);
-        mu = mulp(mu, mu);
-        if ((K >> bit) & 1) mu = mulp(mu, xp);
-      }
-      if (t == 0) pw_s[0] = mu;
-    }
-    tab[0][t] = rp_one_fr();
-    tab[1][t] = rp_one_fr();
+    // ---- table block: wave 0 raises mu, mu^2, mu^4, ... and publishes each;
+    // a lane of the other waves multiplies up its own entries from the bits of
+    // their index as the squares appear (wave 1: A_l, A_(l+64), ...; waves 2
+    // and 3: B).  No step waits for another's table, so the chain is the
+    // squarings and one product, about 21 at K = 20.
+    __shared__ uint32_t pw_s[16][9];
+    __shared__ int ready;
+    const int w = t >> 6, l = t & 63;
+    if (t == 0) ready = 0;
     __syncthreads();
-    // step s: entries [2^s', 2^(s'+1)) of A (s < 8) or of B (s >= 8),
-    // s' = s mod 8, at most 128 per step, over the 192 lanes of waves 1..3
-    for (int s = 0; s < steps; s++) {
-      const fr p = pw_s[s];  // mu^(2^s) R'
-      if (w == 0) {
-        if (s + 1 < steps) {
-          const fr q = mulp(p, p);
-          if (t == 0) pw_s[s + 1] = q;
+    if (w == 0) {
+      const v9 xp = m_rp(load_m(x, neg));
+      v9 mu = xp;  // m^K R', left to right; K is even, so m^(K/2) precedes the last squaring
+      for (int bit = 30 - __builtin_clz(K); bit >= 0; bit--) {
+        if (bit == 0 && t == 0) {
+          fr o;
+          pbd_pack(mu.l, o.l);
+          fr_store(ws + kWsHalf, o);
         }
-      } else {
-        const int tb = s < 8 ? 0 : 1, ss = s & 7;
-        const int j = (1 << ss) + t - 64;
-        if (t - 64 < (1 << ss) && (tb == 0 || j < (int)G)) tab[tb][j] = mulp(tab[tb][j - (1 << ss)], p);
+        mu = mul_r(mu, mu);
+        if ((K >> bit) & 1) mu = mul_r(mu, xp);
       }
-      __syncthreads();
+      for (int s = 0; s < steps; s++) {
+        if (t == 0) {
+#pragma unroll
+          for (int i = 0; i < 9; i++) pw_s[s][i] = mu.l[i];
+          __hip_atomic_store(&ready, s + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+          fr o;
+          pbd_pack(mu.l, o.l);
+          fr_store(ws + kWsPw + s, o);
+        }
+        if (s + 1 < steps) mu = mul_r(mu, mu);
+      }
+      return;
     }
-    fr_store(ws + kWsA + t, tab[0][t]);
-    if (t < (int)G) fr_store(ws + kWsB + t, tab[1][t]);
-    if (t < steps) fr_store(ws + kWsPw + t, pw_s[t]);
+    const int from = w == 1 ? 0 : 8, nb = w == 1 ? 8 : steps - 8;  // index bits of this table
+    const uint64_t tab = w == 1 ? kWsA : kWsB;
+    const int cnt = w == 1 ? kScanThreads : (int)G;
+    auto square = [&](int s) {  // mu^(2^(from + s)) once wave 0 has it
+      while (__hip_atomic_load(&ready, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) <= from + s)
+        __builtin_amdgcn_s_sleep(1);
+      v9 p;
+#pragma unroll
+      for (int i = 0; i < 9; i++) p.l[i] = pw_s[from + s][i];
+      return p;
+    };
+    auto put = [&](int j, const v9& v) {
+      if (j >= cnt) return;
+      fr o;
+      pbd_pack(v.l, o.l);
+      fr_store(ws + tab + j, o);
+    };
+    v9 e0;
+    unpack_ext(rp_one_fr().l, e0.l);
+    for (int s = 0; s < 6 && s < nb; s++) {
+      const v9 p = square(s), q = mul_r(e0, p);
+      if ((l >> s) & 1) e0 = q;
+    }
+    if (w != 3) put(l, e0);
+    if (nb > 6) {
+      v9 e1;
+      if (w != 3) {
+        e1 = mul_r(e0, square(6));
+        put(l + 64, e1);
+      }
+      if (nb > 7) {
+        const v9 p = square(7);
+        if (w != 2) put(l + 128, mul_r(e0, p));
+        if (w != 3) put(l + 192, mul_r(e1, p));
+      }
+    }
     return;
   }
   // ---- data block b: the Horner value of each thread's run ----
   const uint32_t b = blockIdx.x - 1;
-  uint32_t w9[9];
-  unpack_ext(load_m(x, neg).l, w9);  // balanced digits of m R'
+  v9 row = rows29_make<false>(load_m(x, neg));
   const uint64_t base = ((uint64_t)b * kScanThreads + t) * K;
   const bool full = (uint64_t)(b + 1) * kScanThreads * K <= n;
   fr v[K];
   load_run<K>(a, n, base, full, v);
-  // the Horner chain starts after every load is issued (w9 passes through)
-  asm volatile("" : "+v"(w9[0]), "+v"(w9[1]), "+v"(w9[2]), "+v"(w9[3]), "+v"(w9[4]), "+v"(w9[5]), "+v"(w9[6]),
-               "+v"(w9[7]), "+v"(w9[8])::"memory");
+  // the Horner chain starts after every load is issued (its rows pass through)
+  asm volatile("" : "+v"(row.l[0]), "+v"(row.l[1]), "+v"(row.l[2]), "+v"(row.l[3]), "+v"(row.l[4]), "+v"(row.l[5]),
+               "+v"(row.l[6]), "+v"(row.l[7]), "+v"(row.l[8])::"memory");
   fr upper;
-  const fr L = horner29_inorder<K>(v, w9, halves ? &upper : nullptr);
+  const fr L = horner29_inorder<K>(v, rows29_spread(row), halves ? &upper : nullptr);
   const uint64_t r = (uint64_t)b * kScanThreads + t;
   fr_store(ws + kWsL + r, L);
   if (halves) fr_store(ws + kWsL + (uint64_t)kScanThreads * G + r, upper);
+}
+
+// a word (stored form) times a pbd word in R'-form, canonical
+__device__ __forceinline__ fr mul_word_pbd(const fr& a, const fr& w) {
+  v9 x;
+  uint32_t f[9];
+  unpack_ext(a.l, x.l);
+  pbd_unpack(w.l, f);
+  return v9_canonical(v9_mul<false, false, false>(x, f));
 }
 
 // evaluation, launch 2: P_b = B_b sum_t L_(256 b + t) A_t
@@ -766,7 +813,7 @@ __global__ void __launch_bounds__(kScanThreads) lat_combine_kernel(fr* ws) {
   __shared__ uint4 l[2][kScanThreads];
   const int t = threadIdx.x;
   const uint32_t b = blockIdx.x;
-  fr c = mulp(fr_load(ws + kWsL + (uint64_t)b * kScanThreads + t), fr_load(ws + kWsA + t));
+  fr c = mul_word_pbd(fr_load(ws + kWsL + (uint64_t)b * kScanThreads + t), fr_load(ws + kWsA + t));
   lds_put(l, t, c);
   __syncthreads();
   for (int s = kScanThreads / 2; s > 0; s >>= 1) {
@@ -776,7 +823,7 @@ __global__ void __launch_bounds__(kScanThreads) lat_combine_kernel(fr* ws) {
     }
     __syncthreads();
   }
-  if (t == 0) fr_store(ws + kWsP + b, mulp(c, fr_load(ws + kWsB + b)));
+  if (t == 0) fr_store(ws + kWsP + b, mul_word_pbd(c, fr_load(ws + kWsB + b)));
 }
 
 // evaluation, launch 3: y = sum of the G block values
@@ -798,27 +845,54 @@ __global__ void __launch_bounds__(kScanThreads) eval_lat_sum_kernel(const fr* ws
 
 // division, launch 2: the run suffixes of block b, S_t = sum_(t' >= t) L_t' mu^(t' - t)
 // (S_t replaces L_t), and the block value P_b = S_0
+// Six exchange steps inside the wave, then the sum over the waves after: with
+// D_w = s at the end of wave w, S_t += mu^(64 - lane) D_w.  The running value
+// is signed limbs: products with balanced digits (2^28) summed seven times.
 __global__ void __launch_bounds__(kScanThreads) div_lat_suffix_kernel(fr* ws) {
-  __shared__ uint4 l[2][kScanThreads];
-  const int t = threadIdx.x;
+  __shared__ uint32_t wt[4][9];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const uint64_t r = (uint64_t)blockIdx.x * kScanThreads + t;
-  fr v = fr_load(ws + kWsL + r);
-  fr pw[8];  // mu^(2^s), loaded once before the levels
+  fr pw[7];  // mu^(2^s), loaded once before the steps
 #pragma unroll
-  for (int s = 0; s < 8; s++) pw[s] = fr_load(ws + kWsPw + s);
-  lds_put(l, t, v);
-  __syncthreads();
+  for (int s = 0; s < 7; s++) pw[s] = fr_load(ws + kWsPw + s);
+  uint32_t f[9];
+  pbd_unpack(fr_load(ws + kWsA + 64 - lane).l, f);  // mu^(64 - lane)
+  v9 v;
+  unpack_ext(fr_load(ws + kWsL + r).l, v.l);
 #pragma unroll
-  for (int s = 0; s < 8; s++) {
-    const int o = 1 << s;
-    const fr other = t + o < kScanThreads ? lds_get(l, t + o) : fr_zero();
-    __syncthreads();
-    if (t + o < kScanThreads) v = fr_add(v, mulp(other, pw[s]));
-    lds_put(l, t, v);
-    __syncthreads();
+  for (int s = 0; s < 6; s++) {
+    v9 o;
+#pragma unroll
+    for (int i = 0; i < 9; i++) o.l[i] = (uint32_t)__shfl_down((int)v.l[i], 1 << s);
+    uint32_t p[9];
+    pbd_unpack(pw[s].l, p);
+    o = v9_mul<false, false, true>(o, p);
+    if (lane + (1 << s) < 64) v = v9_add(v, o);
   }
-  fr_store(ws + kWsL + r, v);
-  if (t == 0) fr_store(ws + kWsP + blockIdx.x, v);
+  if (lane == 0) {
+    const fr c = v9_canonical(v);
+    v9 b;
+    unpack_ext(c.l, b.l);
+#pragma unroll
+    for (int i = 0; i < 9; i++) wt[w][i] = b.l[i];
+  }
+  __syncthreads();
+  if (w < 3) {
+    v9 d;  // D_w: the later waves' values by Horner in mu^64
+    uint32_t p[9];
+    pbd_unpack(pw[6].l, p);
+#pragma unroll
+    for (int i = 0; i < 9; i++) d.l[i] = wt[3][i];
+    for (int k = 2; k > w; k--) {
+      d = v9_mul<false, false, true>(d, p);
+#pragma unroll
+      for (int i = 0; i < 9; i++) d.l[i] += wt[k][i];
+    }
+    v = v9_add(v, v9_mul<false, false, true>(d, f));
+  }
+  const fr S = v9_canonical(v);
+  fr_store(ws + kWsL + r, S);
+  if (t == 0) fr_store(ws + kWsP + blockIdx.x, S);
 }
 
 // division, launch 3: two threads per run, each rescanning half of it in
@@ -842,7 +916,8 @@ __global__ void __launch_bounds__(kScanThreads) div_lat_down_kernel(const fr* a,
   const uint64_t base = r * K + (upper ? H : 0);
   fr v[H];
   load_run<H>(a, n, base, (uint64_t)(b + 1) * kScanThreads * K <= n, v);
-  fr cb = b + 1 + tid < G ? mulp(fr_load(ws + kWsP + b + 1 + tid), fr_load(ws + kWsB + tid)) : fr_zero();
+  v9 row = rows29_make<false>(load_m(c, 1));
+  fr cb = b + 1 + tid < G ? mul_word_pbd(fr_load(ws + kWsP + b + 1 + tid), fr_load(ws + kWsB + tid)) : fr_zero();
   lds_put(l, tid, cb);
   __syncthreads();
   for (int s = kScanThreads / 2; s > 0; s >>= 1) {
@@ -855,13 +930,13 @@ __global__ void __launch_bounds__(kScanThreads) div_lat_down_kernel(const fr* a,
   cb = lds_get(l, 0);
   if (blockIdx.x == 0 && tid == 0 && rem) {
     const fr p0 = fr_load(ws + kWsP);
-    fr_store(rem, G > 1 ? fr_add(p0, mulp(cb, fr_load(ws + kWsB + 1))) : p0);
+    fr_store(rem, G > 1 ? fr_add(p0, mul_word_pbd(cb, fr_load(ws + kWsB + 1))) : p0);
   }
-  fr cin = mulp(cb, fr_load(ws + kWsA + (kScanThreads - 1 - t)));
+  fr cin = mul_word_pbd(cb, fr_load(ws + kWsA + (kScanThreads - 1 - t)));
   if (t + 1 < kScanThreads) cin = fr_add(cin, fr_load(ws + kWsL + r + 1));
-  if (!upper) cin = fr_add(fr_load(ws + kWsL + (uint64_t)kScanThreads * G + r), mulp(cin, fr_load(ws + kWsHalf)));
-  uint32_t w9[9];
-  unpack_ext(load_m(c, 1).l, w9);
+  if (!upper)
+    cin = fr_add(fr_load(ws + kWsL + (uint64_t)kScanThreads * G + r), mul_word_pbd(cin, fr_load(ws + kWsHalf)));
+  const rows_all m = rows29_spread(row);
   v9 sn;
   unpack_ext(cin.l, sn.l);
   static_for<0, H>([&](auto j_) {
@@ -870,7 +945,7 @@ __global__ void __launch_bounds__(kScanThreads) div_lat_down_kernel(const fr* a,
     if constexpr (k > 0) {
       v9 xv;
       unpack_ext(v[k].l, xv.l);
-      sn = v9_add(v9_mul<false, false, false>(sn, w9), xv);
+      sn = v9_add(v9_mul_all<false>(sn, m), xv);
     }
   });
 }
@@ -911,7 +986,7 @@ struct LatDown {
   }
 };
 
-// B and A need 8 + ceil(log2 G) doubling steps
+// B and A need 8 + ceil(log2 G) squares
 static int lat_steps(uint32_t G) { return 8 + (G > 1 ? 32 - __builtin_clz(G - 1) : 0); }
 
 static hipError_t evaluate_lat(const fr* a, uint64_t n, const fr* x, fr* y, fr* ws, hipStream_t s) {
