@@ -365,51 +365,56 @@ __device__ __forceinline__ void dual29_dev(const uint32_t* a, const uint32_t* w,
   t[8] = (uint32_t)acc[17];
 }
 
-// Three columns (27 words) of a rows29 factor, in SGPRs.  rows29_open's loads
-// are issued where it stands: the scheduling barrier lets vector and LDS
-// instructions pass but neither the scalar loads nor the column blocks, so
-// they are in flight while the blocks before their use run.
-struct rows_cols {
-  uint32_t w[27];
+// The first five or the last four columns of a rows29 factor, in SGPRs.
+// rows29_open's loads are issued where it stands: the scheduling barrier lets
+// vector and LDS instructions pass but neither the scalar loads nor the column
+// blocks, so they are in flight while the blocks before their use run.
+constexpr int kRowsA = 5, kRowsB = 4;
+template <int C>
+struct rows_part {
+  uint32_t w[9 * C];
 };
-__device__ __forceinline__ rows_cols rows29_open(uwords w, int group) {
-  rows_cols g;
+typedef rows_part<kRowsA> rows_cols;
+template <int C>
+__device__ __forceinline__ rows_part<C> rows29_open_part(uwords w, int col) {
+  rows_part<C> g;
   asm volatile("" : "+s"(w));  // a fresh load: no rows held from product to product
 #pragma unroll
-  for (int i = 0; i < 27; i++) g.w[i] = w[27 * group + i];
+  for (int i = 0; i < 9 * C; i++) g.w[i] = w[9 * col + i];
   __builtin_amdgcn_sched_barrier(0x0002 | 0x0004 | 0x0010 | 0x0080);
   return g;
 }
+__device__ __forceinline__ rows_cols rows29_open(uwords w) { return rows29_open_part<kRowsA>(w, 0); }
 
 // rows29 on the device: x w for the wave-uniform factor whose rows are at w.
-// The 81 words come in three groups of three columns, each opened a group
-// (two columns, about 90 issue cycles) ahead of its use: all at once beside the kernel's
-// own they would not fit the scalar registers (180-230 spilled), and loaded
-// where they are used a lone wave waits for each group.  g holds the first group;
-// `next`, the factor of the product that follows, leaves its first group there.
+// The 81 words come in two parts, each opened about 45 VALU instructions ahead
+// of its use: two factors beside the kernel's own would not fit the scalar
+// registers (180-230 spilled), and loaded where they are used a lone wave waits
+// for each part.  g holds the first part; `next`, the factor of the product
+// that follows, leaves its first part there.
 template <int D, bool BT>
 __device__ __forceinline__ void rows29_dev(const uint32_t* x, uwords w, rows_cols& g, uint32_t* t, uwords next) {
   uint32_t m[D];
   uint64_t acc[9 + D];
-  rows_cols g1, g2, gn;
+  rows_part<kRowsB> b;
+  rows_cols gn;
   static_for<0, 8 + D>([&](auto k_) {
     constexpr int k = decltype(k_)::value;
-    // after the group's first column: scalar loads return in any order, so
-    // its wait would be for the new group's loads too
-    if constexpr (k == 1) g1 = rows29_open(w, 1);
-    if constexpr (k == 4) g2 = rows29_open(w, 2);
-    if constexpr (k == 7) gn = rows29_open(next, 0);
+    // after the part's first column: scalar loads return in any order, so
+    // its wait would be for the new part's loads too
+    if constexpr (k == 1) b = rows29_open_part<kRowsB>(w, kRowsA);
+    if constexpr (k == kRowsA + 1) gn = rows29_open(next);
     // block k closes column k - 1, an output column (balanced if BT) from D on
     constexpr bool RND = BT && k - 1 >= D;
-    Rows29Col<k, D, RND>::run(acc[k], k ? acc[k ? k - 1 : 0] : 0, x, (k < 3 ? g : k < 6 ? g1 : g2).w + 9 * (k % 3),
-                              m);
+    const uint32_t* c = k < kRowsA ? g.w + 9 * (k < kRowsA ? k : 0) : b.w + 9 * (k < 9 && k >= kRowsA ? k - kRowsA : 0);
+    Rows29Col<k, D, RND>::run(acc[k], k ? acc[k ? k - 1 : 0] : 0, x, c, m);
     const uint32_t lo = (uint32_t)acc[k];
     if constexpr (k < D)
       m[k] = lo & kMask29;
     else
       t[k - D] = BT ? sext29(lo) : (lo & kMask29);
   });
-  Rows29Col<8 + D, D, BT>::run(acc[8 + D], acc[7 + D], x, g2.w, m);
+  Rows29Col<8 + D, D, BT>::run(acc[8 + D], acc[7 + D], x, b.w, m);
   t[8] = (uint32_t)acc[8 + D];
   g = gn;
 }

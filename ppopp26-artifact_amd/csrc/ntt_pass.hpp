@@ -119,7 +119,7 @@ __device__ __forceinline__ void dft_dif(v9 (&x)[NX], uwords f) {
   };
   // x times factor e; n is the next product's
   rows_cols g;
-  if constexpr (LOGB >= 2) g = rows29_open(f + kRowWords * kDftI, 0);
+  if constexpr (LOGB >= 2) g = rows29_open(f + kRowWords * kDftI);
   auto mul = [&](v9& a, int e, int n) {
     a = v9_mul_rows<1, false>(a, f + kRowWords * e, g, f + kRowWords * n);
     pin9(a);
@@ -386,7 +386,7 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
     reduce(x[0]);
     const uwords tw = rows + kRowWords * kInner;
     const int step = (kRowWords * rho1) << (6 - m);  // w_M'^rho1
-    rows_cols g = rows29_open(tw + step, 0);
+    rows_cols g = rows29_open(tw + step);
     static_for<1, kPerT>([&](auto k2_) {
       constexpr int k2 = decltype(k2_)::value;
       v9& v = x[brev(k2, kLgPerT)];

@@ -503,7 +503,7 @@ __device__ __forceinline__ void v9_carry_balanced(v9& v) {
 template <bool SK>
 __device__ __forceinline__ void perm_terms_at(const RatioArgs& a, uint64_t i, v9& num, v9& den) {
   const uwords B = (uwords)a.brows;
-  rows_cols g0 = rows29_open(B, 0);
+  rows_cols g0 = rows29_open(B);
   v9 gam;
   unpack_ext(fr_load(a.gamma).l, gam.l);
   v9 w1;
