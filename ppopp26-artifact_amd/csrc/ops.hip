@@ -118,11 +118,16 @@ __device__ __forceinline__ fr rp_one() {
   return r;
 }
 
+// A word enters a product as plain 29-bit digits (split29, 17 VALU instructions
+// against unpack_ext's 33 for balanced ones): with the other operand's digits
+// below 2^30 a column stays below 9 * 2^59 + 8 * 2^58 + 2^35 < 2^62.8.  Only a
+// word that is packed or summed as it is takes balanced digits.
+
 // P(a, b) of two words, canonical
 __device__ __forceinline__ fr mul_rp(const fr& a, const fr& b) {
   v9 x, y;
-  unpack_ext(a.l, x.l);
-  unpack_ext(b.l, y.l);
+  split29(a.l, x.l);
+  split29(b.l, y.l);
   return v9_canonical(v9_mul<false, false, false>(x, y.l));
 }
 
@@ -237,8 +242,8 @@ __global__ void __launch_bounds__(kOpThreads) inv_reduce_kernel(const fr* in, ui
   static_for<0, kOpPer / 2>([&](auto k_) {
     constexpr int k = decltype(k_)::value;
     v9 x, y;
-    unpack_ext(v[k].l, x.l);
-    unpack_ext(v[k + kOpPer / 2].l, y.l);
+    split29(v[k].l, x.l);
+    split29(v[k + kOpPer / 2].l, y.l);
     p[k] = v9_mul<false, false, false>(x, y.l);
   });
   static_for<0, kOpLgPer - 1>([&](auto s_) {
@@ -297,7 +302,7 @@ inv_down_kernel(const fr* in, const fr* num, fr* out, uint64_t n, const fr* binv
       e[k] = rp_one();
     }
     v9 x;
-    unpack_ext(e[k].l, x.l);
+    split29(e[k].l, x.l);
     if constexpr (k == 0) {
       L = x;  // L_0 = x_0 as loaded (below 2^256, beyond a pbd word's range)
     } else {
@@ -327,7 +332,7 @@ inv_down_kernel(const fr* in, const fr* num, fr* out, uint64_t n, const fr* binv
   } else {
     b = fr_load(binv + blockIdx.x);
   }
-  unpack_ext(b.l, cur.l);
+  split29(b.l, cur.l);
   cur = v9_mul<false, false, false>(cur, E.l);
   // walk back: inv(x_k) = inv(L_k) L_{k-1} (inv(x_0) = inv(L_0));
   // inv(L_{k-1}) = inv(L_k) x_k; each element and numerator is asked for one
@@ -343,7 +348,7 @@ inv_down_kernel(const fr* in, const fr* num, fr* out, uint64_t n, const fr* binv
     v9 inv_k = cur;
     if constexpr (k > 0) {
       uint32_t Lp[9];
-      if constexpr (k - 1 == 0) unpack_ext(e[0].l, Lp);
+      if constexpr (k - 1 == 0) split29(e[0].l, Lp);
       else pbd_unpack(e[k > 1 ? k - 1 : 1].l, Lp);
       inv_k = v9_mul<false, false, false>(cur, Lp);
       pin9(inv_k);  // one product at a time: fewer live temporaries
@@ -351,7 +356,7 @@ inv_down_kernel(const fr* in, const fr* num, fr* out, uint64_t n, const fr* binv
       // x_k from the original input (one again for zeros)
       if ((zmask >> k) & 1) xk = rp_one();
       uint32_t X[9];
-      unpack_ext(xk.l, X);
+      split29(xk.l, X);
       cur = v9_mul<false, false, false>(cur, X);
       pin9(cur);
       pin9(inv_k);
@@ -363,7 +368,7 @@ inv_down_kernel(const fr* in, const fr* num, fr* out, uint64_t n, const fr* binv
       } else {
         if (num) {
           uint32_t N[9];
-          unpack_ext(nk.l, N);
+          split29(nk.l, N);
           inv_k = v9_mul<false, false, false>(inv_k, N);
         }
         r = v9_canonical(inv_k);
@@ -465,9 +470,9 @@ __global__ void __launch_bounds__(256) perm_table_kernel(RatioArgs a, uint32_t c
 #pragma unroll
   for (int d = 0; d < 5; d++) b32 = fr_add(b32, b32);
   uint32_t b[9];
-  unpack_ext(b32.l, b);
+  split29(b32.l, b);
   v9 w;
-  unpack_ext(fr_load(a.w0 + lo).l, w.l);
+  split29(fr_load(a.w0 + lo).l, w.l);
   const v9 bw = v9_mul<false, false, false>(w, b);
 #pragma unroll
   for (int j = 0; j < 3; j++) {
@@ -507,7 +512,7 @@ __device__ __forceinline__ void perm_terms_at(const RatioArgs& a, uint64_t i, v9
   v9 gam;
   unpack_ext(fr_load(a.gamma).l, gam.l);
   v9 w1;
-  unpack_ext(fr_load(a.w1 + (i >> 14)).l, w1.l);
+  split29(fr_load(a.w1 + (i >> 14)).l, w1.l);
   v9 t1, t7;  // SK: beta w^i, then 7 beta w^i (balanced digits)
 #pragma unroll
   for (int j = 0; j < 3; j++) {
@@ -531,7 +536,7 @@ __device__ __forceinline__ void perm_terms_at(const RatioArgs& a, uint64_t i, v9
       v9_carry_balanced(kt);
     }
     const v9 nj = v9_add(wg, kt);
-    unpack_ext(fr_load(a.s[j] + i).l, sj.l);
+    split29(fr_load(a.s[j] + i).l, sj.l);
     const v9 dj = v9_add(wg, v9_mul_rows<2, true>(sj, B, g0, B));
     num = j == 0 ? nj : v9_mul<false, false, false>(num, nj.l);  // the first factor needs no product
     den = j == 0 ? dj : v9_mul<false, false, false>(den, dj.l);
@@ -572,12 +577,12 @@ __global__ void __launch_bounds__(256) perm_terms_kernel(RatioArgs a, fr* rn, fr
     {
       const fr send = (lane & 1) ? nw : dw;
       v9 mine;
-      unpack_ext(((lane & 1) ? dw : nw).l, mine.l);
+      split29(((lane & 1) ? dw : nw).l, mine.l);
       fr o;
 #pragma unroll
       for (int j = 0; j < 8; j++) o.l[j] = (uint32_t)__shfl_xor((int)send.l[j], 1);
       uint32_t other[9];
-      unpack_ext(o.l, other);
+      split29(o.l, other);
       p = v9_mul<false, false, false>(mine, other);
     }
 #pragma unroll
@@ -630,7 +635,7 @@ __global__ void __launch_bounds__(kUpThreads) gp_up_kernel(const fr* nv, const f
     constexpr int k = decltype(k_)::value;
     const fr v = base + k < n ? fr_load(src + base + k) : rp_one();
     v9 x;
-    unpack_ext(v.l, x.l);
+    split29(v.l, x.l);
     p = k == 0 ? x : v9_mul<false, false, true>(p, x.l);
   });
   fr_store((den ? td : tn) + tid, v9_canonical(p));
@@ -683,7 +688,8 @@ __device__ __forceinline__ void gp_down_body(const fr* nv, const fr* dv, const f
     constexpr int k = kPer - 1 - decltype(k_)::value;
     const fr dw = base + k < n ? fr_load(dv + base + k) : rp_one();
     v9 y;
-    unpack_ext(dw.l, y.l);
+    if constexpr (k == kPer - 1) unpack_ext(dw.l, y.l);  // packed as it is: balanced digits
+    else split29(dw.l, y.l);
     if constexpr (INCL) {
       acc = k == kPer - 1 ? y : v9_mul<false, false, true>(acc, y.l);
       pbd_pack(acc.l, S[k].l);
@@ -741,7 +747,7 @@ __device__ __forceinline__ void gp_down_body(const fr* nv, const fr* dv, const f
   v9 cur;
   {
     v9 a;
-    unpack_ext(cw.l, a.l);
+    split29(cw.l, a.l);
     cur = v9_mul<false, false, false>(v9_mul<false, false, false>(a, pre.l), suf.l);
   }
   static_for<0, kPer>([&](auto k_) {
@@ -755,7 +761,7 @@ __device__ __forceinline__ void gp_down_body(const fr* nv, const fr* dv, const f
     }
     if constexpr (k < kPer - 1) {
       uint32_t x[9];
-      unpack_ext(nw.l, x);
+      split29(nw.l, x);
       cur = v9_mul<false, false, false>(cur, x);
     }
   });
@@ -808,15 +814,16 @@ __global__ void __launch_bounds__(256) gp_run_down_kernel(const fr* nv, const fr
     constexpr int k = kOpPer - 1 - decltype(k_)::value;
     const fr dw = base + k < n ? fr_load(dv + base + k) : rp_one();
     v9 y;
-    unpack_ext(dw.l, y.l);
+    if constexpr (k == kOpPer - 1) unpack_ext(dw.l, y.l);  // packed as it is: balanced digits
+    else split29(dw.l, y.l);
     acc = k == kOpPer - 1 ? y : v9_mul<false, false, true>(acc, y.l);
     pbd_pack(acc.l, S[k].l);
   });
   v9 cur;
-  unpack_ext(fr_load(carry + run).l, cur.l);
+  split29(fr_load(carry + run).l, cur.l);
   if (inv) {
     uint32_t w[9];
-    unpack_ext(fr_load(inv).l, w);
+    split29(fr_load(inv).l, w);
     cur = v9_mul<false, false, false>(cur, w);
   }
   // four quarters: each quarter's num values are loaded before its outputs
@@ -839,7 +846,7 @@ __global__ void __launch_bounds__(256) gp_run_down_kernel(const fr* nv, const fr
       }
       if constexpr (k < kOpPer - 1) {
         uint32_t x[9];
-        unpack_ext(nw[j].l, x);
+        split29(nw[j].l, x);
         cur = v9_mul<false, false, false>(cur, x);
       }
     });

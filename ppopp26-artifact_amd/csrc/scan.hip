@@ -136,7 +136,7 @@ __global__ void __launch_bounds__(kScanThreads) pfx_reduce_kernel(const fr* in, 
     // one element at a time, as its load arrives
     if ((uint32_t)(k * kScanThreads + t) < rem) {
       uint32_t w[9];
-      if constexpr (RF) unpack_ext(v[k].l, w);
+      if constexpr (RF) split29(v[k].l, w);
       else split29_x32(v[k].l, w);
       h = v9_mul<false, !RF, true>(h, w);
     }
@@ -188,7 +188,7 @@ pfx_down_kernel(const fr* in, fr* out_excl, fr* out_incl, uint64_t n, const fr* 
       if (rem > 0) unpack_ext(e[0].l, h.l);
     } else if (k < rem) {
       uint32_t w[9];
-      if constexpr (RF) unpack_ext(e[k].l, w);
+      if constexpr (RF) split29(e[k].l, w);
       else split29_x32(e[k].l, w);
       h = v9_mul<false, !RF, true>(h, w);
     }
@@ -214,7 +214,7 @@ pfx_down_kernel(const fr* in, fr* out_excl, fr* out_incl, uint64_t n, const fr* 
     if (w < wave) pre = v9_mul<false, false, true>(pre, wt[w]);
   if (carry) {
     uint32_t c[9];
-    unpack_ext(fr_load(carry + blockIdx.x).l, c);
+    split29(fr_load(carry + blockIdx.x).l, c);
     pre = v9_mul<false, false, true>(pre, c);
   }
   fr* dst = out_excl + b0 + t * kPer;
@@ -227,7 +227,7 @@ pfx_down_kernel(const fr* in, fr* out_excl, fr* out_incl, uint64_t n, const fr* 
           ex = v9_canonical(pre);
         } else {
           uint32_t w[9];
-          unpack_ext(fr_one().l, w);
+          split29(fr_one().l, w);
           ex = v9_canonical(v9_mul<false, false, false>(pre, w));
         }
       } else {
@@ -325,17 +325,17 @@ __device__ __forceinline__ rows_all rp_rows(const fr* w) { return rows29_spread(
 // sum_k v_k w^k by Horner in signed limbs (fr29.hpp): h <- h w + v_k with the
 // wave-uniform w held as rows in SGPRs (about 150 VALU instructions per step,
 // 225 with w per lane; evaluation of 2^24 176 -> 154 us, of 2^20 24.9 -> 22.3,
-// division 598 -> 565 and 52.7 -> 48.7), limb-wise sums of a product (digits in [0, 2^29)) and
-// balanced digits, so every limb stays below 2^30 and the product within
+// division 598 -> 565 and 52.7 -> 48.7), limb-wise sums of a product and a word
+// (digits in [0, 2^29) both), so every limb stays below 2^30 and the product within
 // (-1.001 r, 0.001 r); canonical once at the end.
 template <int K>
 __device__ __forceinline__ fr horner29(const fr (&v)[K], const rows_all& w) {
   v9 h;
-  unpack_ext(v[K - 1].l, h.l);
+  split29(v[K - 1].l, h.l);
   static_for<0, K - 1>([&](auto k_) {
     constexpr int k = K - 2 - decltype(k_)::value;
     v9 x;
-    unpack_ext(v[k].l, x.l);
+    split29(v[k].l, x.l);
     h = v9_add(v9_mul_all<false>(h, w), x);
   });
   return v9_canonical(h);
@@ -478,7 +478,7 @@ __global__ void __launch_bounds__(kScanThreads) sfx_down_kernel(const fr* a, fr*
   // elements already read
   const rows_all m = rows29_spread(row);
   v9 sn;
-  unpack_ext(cin.l, sn.l);
+  split29(cin.l, sn.l);
   constexpr int G = kPer > 1 ? 2 : 1, Q = kPer / G;
   static_for<0, G>([&](auto g_) {
     constexpr int top = kPer - 1 - decltype(g_)::value * Q;  // highest index of this half
@@ -492,7 +492,7 @@ __global__ void __launch_bounds__(kScanThreads) sfx_down_kernel(const fr* a, fr*
       if (base + k < n) fr_store(out + base + k, k == kPer - 1 ? cin : v9_canonical(sn));
       if constexpr (k > 0) {
         v9 x;
-        unpack_ext(e[top - k].l, x.l);
+        split29(e[top - k].l, x.l);
         sn = v9_add(v9_mul_all<false>(sn, m), x);
       }
     });
@@ -668,14 +668,14 @@ __device__ __forceinline__ v9 m_rp(const fr& m) {
 template <int K>
 __device__ __forceinline__ fr horner29_inorder(fr (&v)[K], const rows_all& w, fr* upper) {
   v9 h;
-  unpack_ext(v[K - 1].l, h.l);
+  split29(v[K - 1].l, h.l);
   static_for<0, K - 1>([&](auto k_) {
     constexpr int k = K - 2 - decltype(k_)::value;
     fr e = v[k];
     asm volatile("" : "+v"(e.l[0]), "+v"(e.l[1]), "+v"(e.l[2]), "+v"(e.l[3]), "+v"(e.l[4]), "+v"(e.l[5]),
                  "+v"(e.l[6]), "+v"(e.l[7]) : "v"(h.l[0]));
     v9 xv;
-    unpack_ext(e.l, xv.l);
+    split29(e.l, xv.l);
     h = v9_add(v9_mul_all<false>(h, w), xv);
     if constexpr (k == K / 2) {
       if (upper) *upper = v9_canonical(h);
@@ -803,7 +803,7 @@ __global__ void __launch_bounds__(kScanThreads) lat_runs_kernel(const fr* a, uin
 __device__ __forceinline__ fr mul_word_pbd(const fr& a, const fr& w) {
   v9 x;
   uint32_t f[9];
-  unpack_ext(a.l, x.l);
+  split29(a.l, x.l);
   pbd_unpack(w.l, f);
   return v9_canonical(v9_mul<false, false, false>(x, f));
 }
@@ -938,13 +938,13 @@ __global__ void __launch_bounds__(kScanThreads) div_lat_down_kernel(const fr* a,
     cin = fr_add(fr_load(ws + kWsL + (uint64_t)kScanThreads * G + r), mul_word_pbd(cin, fr_load(ws + kWsHalf)));
   const rows_all m = rows29_spread(row);
   v9 sn;
-  unpack_ext(cin.l, sn.l);
+  split29(cin.l, sn.l);
   static_for<0, H>([&](auto j_) {
     constexpr int k = H - 1 - decltype(j_)::value;
     if (base + k < n) fr_store(q + base + k, k == H - 1 ? cin : v9_canonical(sn));
     if constexpr (k > 0) {
       v9 xv;
-      unpack_ext(v[k].l, xv.l);
+      split29(v[k].l, xv.l);
       sn = v9_add(v9_mul_all<false>(sn, m), xv);
     }
   });
