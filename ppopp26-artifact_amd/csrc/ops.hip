@@ -545,10 +545,14 @@ __device__ __forceinline__ void perm_terms_at(const RatioArgs& a, uint64_t i, v9
 
 // ZERO_DEN (grand product): a zero den is stored as num = 0, den = R' mod r,
 // and the products of num and den over each run of 8 consecutive elements go
-// to rn/rd: three butterfly steps across the run's lanes, each one product
-// per lane (step 1 pairs num on even lanes with den on odd lanes; after steps
-// 2 and 3, lane 8g holds the run's num product and lane 8g + 1 its den
-// product).  Lanes past n carry R' mod r.
+// to rn/rd, in three steps of a tree over the block: the first pairs
+// neighbouring lanes (num on the even one, den on the odd one), the next two
+// take their pairs through LDS into the block's first two waves and then the
+// first, so that every lane of a wave that still runs holds a product of its
+// own: 7 products of a wave per block.  As butterflies across the run's lanes
+// all four waves take all three steps, 12, with a quarter of the lanes useful
+// in the last (perm of 2^20 rows, whole call 203 us; so 196: the kernel is
+// bound by its products).  Lanes past n carry R' mod r.
 template <bool ZERO_DEN, bool SK>
 __global__ void __launch_bounds__(256) perm_terms_kernel(RatioArgs a, fr* rn, fr* rd) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -572,7 +576,7 @@ __global__ void __launch_bounds__(256) perm_terms_kernel(RatioArgs a, fr* rn, fr
       fr_store(a.num + i, nw);
       fr_store(a.den + i, dw);
     }
-    const int lane = threadIdx.x & 7;
+    const int lane = threadIdx.x & 1;
     v9 p;
     {
       const fr send = (lane & 1) ? nw : dw;
@@ -585,14 +589,28 @@ __global__ void __launch_bounds__(256) perm_terms_kernel(RatioArgs a, fr* rn, fr
       split29(o.l, other);
       p = v9_mul<false, false, false>(mine, other);
     }
+    __shared__ uint32_t wp[2][9][256];
+    static_for<0, 2>([&](auto s_) {
+      constexpr int s = decltype(s_)::value;
+      const int u = threadIdx.x;
+      if (u < (256 >> s)) {
 #pragma unroll
-    for (int m = 2; m <= 4; m <<= 1) {
-      uint32_t q[9];
+        for (int j = 0; j < 9; j++) wp[s][j][u] = p.l[j];
+      }
+      __syncthreads();
+      if (u < (128 >> s)) {
+        const int from = 4 * (u >> 1) + (u & 1);
+        uint32_t q[9];
 #pragma unroll
-      for (int j = 0; j < 9; j++) q[j] = (uint32_t)__shfl_xor((int)p.l[j], m);
-      p = v9_mul<false, false, false>(p, q);
-    }
-    if ((i & ~(uint64_t)7) < a.n && lane < 2) fr_store((lane ? rd : rn) + (i >> 3), v9_canonical(p));
+        for (int j = 0; j < 9; j++) {
+          p.l[j] = wp[s][j][from];
+          q[j] = wp[s][j][from + 2];
+        }
+        p = v9_mul<false, false, false>(p, q);
+      }
+    });
+    const uint64_t run = (uint64_t)blockIdx.x * 32 + (threadIdx.x >> 1);
+    if (threadIdx.x < 64 && run * 8 < a.n) fr_store((threadIdx.x & 1 ? rd : rn) + run, v9_canonical(p));
   }
 }
 
