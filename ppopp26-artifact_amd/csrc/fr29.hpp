@@ -135,6 +135,35 @@ PL_HD29 void mont29(const uint32_t* a, const uint32_t* w, uint32_t* t) {
   t[8] = (uint32_t)acc;
 }
 
+// The same in (a w / 2^261 + r/2, a w / 2^261 + 3r/2), plain digits: for
+// |a w| / 2^261 < r/2 a positive value below 2^256, so that the digits join to a
+// 256-bit word.  The last of the digits m alone is taken in
+// [-2^28 - 2^29, 2^28 - 2^29), which centres m and adds r; its column closes as
+// (acc + 2^28 + 2^29) >> 29.  Against mont29<true, true> this saves the seven
+// other balanced digits of m, the eight of t and their columns' roundings: each
+// a multiply-add and a three-operand bit-field extract (1.9 ns per wave and
+// SIMD at four waves) for a two-operand and (1.1 ns).
+PL_HD29 void mont29_word(const uint32_t* a, const uint32_t* w, uint32_t* t) {
+  uint32_t m[9];
+  int64_t acc = 0;
+#pragma unroll
+  for (int k = 0; k < 17; k++) {
+    const int lo = k > 8 ? k - 8 : 0, hi = k < 8 ? k : 8;
+#pragma unroll
+    for (int i = lo; i <= hi; i++) acc += (int64_t)(int32_t)a[i] * (int64_t)(int32_t)w[k - i];
+#pragma unroll
+    for (int i = lo; i <= hi; i++)
+      if (i < k) acc -= (int64_t)(int32_t)m[i] * (int64_t)r29(k - i);
+    const uint32_t dig = k == 8 ? sext29((uint32_t)acc) - (1u << 29) : ((uint32_t)acc & kMask29);
+    if (k <= 8)
+      m[k] = dig;
+    else
+      t[k - 9] = dig;
+    acc = (acc - (int64_t)(int32_t)dig) >> 29;  // exact
+  }
+  t[8] = (uint32_t)acc;
+}
+
 // t = x w for a fixed factor w given as nine pre-reduced rows: rows[9 j + i]
 // holds digit j of W_i = w 2^(29 (i + D)) mod r, W_i in (-0.51 r, 0.51 r) with
 // balanced digits (rows29_entry builds them).  V = sum_i x_i W_i is congruent
@@ -192,8 +221,8 @@ PL_HD29 void add_r256(uint32_t* x) {
 // [29 i, 29 i + 29), i < 8, hold digits b_i in [-2^28, 2^28) as 29-bit two's
 // complement and whose bits [232, 256) hold b_8 in [-2^23, 2^23) as 24-bit two's
 // complement; its value is sum b_i 2^(29 i).  Pass twiddle tables hold their
-// factors this way, and the pass kernels hand intermediate results from pass
-// to pass in it.
+// factors this way, and the one-element-per-lane kernels hand intermediate
+// results from launch to launch in it.
 
 // the nine signed limbs of a pbd word
 PL_HD29 void pbd_unpack(const uint32_t* x, uint32_t* b) {
@@ -342,6 +371,27 @@ __device__ __forceinline__ void mont29_dev(const uint32_t* x, const uint32_t* w,
 // wave-uniform read-only words (loaded to SGPRs)
 typedef const __attribute__((address_space(4))) uint32_t* uwords;
 
+// mont29_word on the device
+__device__ __forceinline__ void mont29_word_dev(const uint32_t* x, const uint32_t* w, uint32_t* t) {
+  uint32_t m[9];
+  uint64_t acc[18];
+  static_for<0, 17>([&](auto k_) {
+    constexpr int k = decltype(k_)::value;
+    uint64_t prev = k ? acc[k ? k - 1 : 0] : 0;
+    if constexpr (k == 9) prev += 3u << 28;
+    Mont29Col<k, false, false>::run(acc[k], prev, x, w, m);
+    const uint32_t lo = (uint32_t)acc[k];
+    if constexpr (k < 8)
+      m[k] = lo & kMask29;
+    else if constexpr (k == 8)
+      m[k] = sext29(lo) - (1u << 29);
+    else
+      t[k - 9] = lo & kMask29;
+  });
+  Mont29Col<17, false, false>::run(acc[17], acc[16], x, w, m);
+  t[8] = (uint32_t)acc[17];
+}
+
 // (a w + b v) / 2^261 mod r: two per-lane products with one reduction, 234
 // multiply-adds where two mont29 take 306.  For |a_i|, |b_i| <= 2^29 and
 // balanced factor digits a column stays below 18 * 2^57 + 8 * 2^58 + 2^34 <
@@ -467,6 +517,15 @@ __device__ __forceinline__ v9 v9_mul(const v9& x, const uint32_t (&w)[9]) {
   v9 t;
   mont29_dev<UB, BM, BT>(x.l, w, t.l);
   return t;
+}
+
+// x w / 2^261 + r as plain digits that join to a 256-bit word (mont29_word)
+__device__ __forceinline__ fr v9_mul_word(const v9& x, const uint32_t (&w)[9]) {
+  uint32_t t[9];
+  mont29_word_dev(x.l, w, t);
+  fr o;
+  join29(t, o.l);
+  return o;
 }
 
 // x w for the wave-uniform factor whose rows are at w (rows29_dev)

@@ -398,7 +398,6 @@ static void fill_pass_args(const Domain& d, const NttCall& c, int p, const fr* i
     const fr sc = to_dev(host::mul(d.n_inv, host::from_u64(32)));
     to_pbd(sc.l, a.scale29.l);
   }
-  a.in_ext = (P.P == 0 || p == 0) ? 1 : 0;
   a.in = in;
   a.out = out;
   a.in_pstride = in_pstride;

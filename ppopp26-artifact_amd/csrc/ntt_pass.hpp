@@ -30,12 +30,21 @@
 // 2^20: 2.98 -> 2.64 ms; the per-lane twiddles of a 16-column tile of two
 // waves before).  Longer tiles leave two workgroups of eight waves on a CU,
 // so loads and stores hide less behind the other's products than with eight
-// of two: 2^24, a middle pass, 534 VALU instructions per element (0.28 ms
-// at the multiply-add probe's rate) in 0.33 ms, where 757 took 0.42.
-// Global accesses move 64 * 32 contiguous bytes, except the last pass's
-// loads, where a lane reads its own sub-row and the waves of a workgroup use
-// up each line between them.  Between passes the data is held as pbd words
-// (fr29.hpp), not reduced; the last pass writes canonical values in [0, r).
+// of two: 2^24, a middle pass, 0.42 -> 0.33 ms with 757 -> 534 VALU
+// instructions per element.  Loading the next tile's words into the registers
+// that the results leave (a workgroup looping over 2 .. 16 tiles) was slower
+// (2^24: 1.32 -> 1.42 ms): the passes wait for VALU issue and for memory, not
+// for single loads.
+// Global accesses move 64 * 32 contiguous bytes, the last pass's loads whole
+// sub-rows.  Between passes the data is held as 256-bit words of the class
+// mod r, not reduced; the last pass writes canonical values in [0, r).
+//
+// Elements are plain digits in [0, 2^29) (a signed top) from load to
+// exchange to store, factors balanced ones: a digit taken plain is a
+// two-operand and (1.1 ns per wave and SIMD at four waves), taken balanced a
+// three-operand bit-field extract (1.9) and a multiply-add that rounds its
+// column (2.0).  2^24: 1.317 -> 1.281 ms, 2^22: 0.340 -> 0.327, 2^20: 102.6 ->
+// 97.2 us with balanced digits before.
 #pragma once
 #include <type_traits>
 
@@ -96,13 +105,14 @@ constexpr int kRowWords = 81;
 // Montgomery digit: about 107 VALU instructions against mont29's 196.
 // NTT 2^24: 1.64 -> 1.43 ms; 2^16: 46 -> 43.7 us (a lone wave per SIMD).
 //
-// Bounds, with input limbs balanced digits (|l| <= 2^28) of values within V:
-// d = x_i - x_(i+4) has |l| <= 2^29, the products' inputs |l| <= 2^30, and the
-// products' limbs lie in [0, 2^29).  y0, y4 = sums of eight digits, first sign
-// plus, so within [-2^31, 2^31); e0 +- i e1 within 2^30 + 2^29; f = d0 +- i d2
-// within [-2^29, 2^30), so y1 = f + A + B within [-2^29, 2^31) and the others
-// smaller.  Values: i d2 within 5.6 r, i e1, A, B within 10.2 r, so every
-// output is within max(8 V, 2 V + 26 r).
+// Bounds, with input limbs plain digits in [0, 2^29) (the top one signed and
+// small) of values within V: sums of four lie in [0, 2^31) and differences of
+// such within 2^31, so only y0, a sum of eight, leaves 32 bits (zero_bias
+// brings it back); d = x_i - x_(i+4) has |l| < 2^29, e0, e1, d1 +- d3 < 2^30,
+// the products' inputs; the products' limbs lie in [0, 2^29).  e0 +- i e1
+// within 2^30 + 2^29; f = d0 +- i d2 within (-2^30, 2^30), so y1 = f + A + B
+// within [-2^30, 2^31) and the others smaller.  Values: i d2 within 5.6 r,
+// i e1, A, B within 10.2 r, so every output is within max(8 V, 2 V + 26 r).
 template <int LOGB, int OFF, int NX>
 __device__ __forceinline__ void dft_dif(v9 (&x)[NX], uwords f) {
   static_assert(LOGB <= 3, "limb growth: at most three butterfly levels");
@@ -116,6 +126,16 @@ __device__ __forceinline__ void dft_dif(v9 (&x)[NX], uwords f) {
     a = s;
     pin9(a);
     pin9(b);
+  };
+  // y0 back into signed limbs: a sum of eight plain digits lies in [0, 2^32),
+  // and adding -2^31 to limb 0, 4 - 2^31 to the middle ones and 4 to limb 8
+  // adds nothing (2^31 at limb i is 4 at limb i + 1)
+  auto zero_bias = [](v9& a) {
+    a.l[0] ^= 1u << 31;
+#pragma unroll
+    for (int i = 1; i < 8; i++) a.l[i] += 4u - (1u << 31);
+    a.l[8] += 4;
+    pin9(a);
   };
   // x times factor e; n is the next product's
   rows_cols g;
@@ -137,6 +157,7 @@ __device__ __forceinline__ void dft_dif(v9 (&x)[NX], uwords f) {
     bfly(x[OFF], x[OFF + 2]);      // b0, e0
     bfly(x[OFF + 1], x[OFF + 3]);  // b1, e1
     bfly(x[OFF], x[OFF + 1]);      // y0, y4
+    zero_bias(x[OFF]);
     mul(x[OFF + 3], kDftI, kDftI);  // i e1
     bfly(x[OFF + 2], x[OFF + 3]);  // y2, y6
     mul(x[OFF + 6], kDftI, kDftC1);  // i d2
@@ -166,7 +187,6 @@ struct PassArgs {
   uint32_t lgI;         // LAST: output interleave
   uint32_t ndig;        // LAST: number of earlier passes
   uint32_t do_scale;    // multiply every output by `scale` (single-pass transforms)
-  uint32_t in_ext;      // the input is caller data (any 256-bit values), not a previous pass's pbd words
   uint32_t lgrad[PL_MAX_PASSES];  // LAST: log2 radices of the earlier passes, pass 1 first
   fr scale;             // stored form (small-size kernel)
   fr scale29;           // pbd word of scale R' mod r (pass kernels)
@@ -206,17 +226,16 @@ __device__ __forceinline__ void unpack_limbs(uint32_t* v, const typename lds_vec
 
 // One pass over columns of M' = 8*A points, A = 2^LA; blk = tile index.
 //
-// Arithmetic: the lane's elements are signed-limb values (v9).  The input is
-// unpacked to balanced digits (caller data: any 256-bit value; later passes:
-// the previous pass's pbd words), so each in-register DFT starts from
-// balanced digits and its limbs stay within 32 bits; every product takes
-// such limbs.  Value bounds (V = input magnitude, at most 2^256 < 2.21 r): a
-// DFT_8 output is below 8 V = 17.7 r; an inner-twiddle product of it lies in
-// (-1.25 r, 0.25 r) (x w / 2^261 < 0.0142 x for w < r); element k2 = 0, which
-// has no inner twiddle, is reduced into (-0.51 r, 0.51 r); so a DFT_A output
-// is below 10 r, and the pass twiddle product with centred digits
-// (mont29 BM) lies in (-0.65 r, 0.65 r): its balanced digits fit a pbd word
-// (top digit below 2^23).  The last pass reduces its outputs to [0, r).
+// Arithmetic: the lane's elements are signed-limb values (v9).  The input,
+// any 256-bit words (below 2.21 r), is split into plain digits, so each
+// in-register DFT starts from such digits and its limbs stay within 32 bits;
+// every product takes such limbs.  Value bounds: the first DFT's outputs are
+// within 2 * 2.21 r + 26 r = 30.4 r; an inner-twiddle product lies in
+// (-1.001 r, 0.001 r), and elements k2 = 0 and rho1 = 0, which have no inner
+// twiddle, are reduced into [0, 1.01 r); so DFT_A's outputs are within
+// 28.1 r, or 30.4 r without one.  The pass twiddle multiplies by at most
+// r / 2^261 < 0.0142, so that mont29_word's product is a word in
+// (0.06 r, 1.94 r).  The last pass reduces its outputs to [0, r).
 // SCALE: multiply every output by a.scale29 (single-pass inverse transforms;
 // a separate instance, so the other last-pass kernels keep no registers for it)
 template <int LA, bool INV, bool LAST, bool SCALE>
@@ -306,8 +325,7 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
       constexpr int r2 = decltype(r2_)::value;
       const uint4 l = raw[r2][0], u = raw[r2][1];
       const uint32_t w[8] = {l.x, l.y, l.z, l.w, u.x, u.y, u.z, u.w};
-      if (a.in_ext) unpack_ext(w, x[r2].l);
-      else pbd_unpack(w, x[r2].l);
+      split29(w, x[r2].l);
     });
   } else {
     const uint64_t poly = line >> lgL;
@@ -317,69 +335,60 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
     const uint64_t pos0 = (rr << a.lgMp) + j;
     const uint64_t estride = 1ull << a.lgS;
     const fr* src = a.in + poly * a.in_pstride;
-    // balanced digits: caller data is any 256-bit value (optionally times a
-    // premultiplication factor), a previous pass's output is a pbd word.  Each
-    // branch loads and unpacks on its own, so no loaded word lives across it.
-    if (a.in_ext) {
-      if (a.premul) {
-        const fr* pm = a.premul + ((uint64_t)(poly & a.pm_mask) << a.lgN) + pos0 + (uint64_t)rho1 * estride;
-        const fr* sp = src + pos0 + (uint64_t)rho1 * estride;
-        // factors are pbd words of c R' (the coset powers); the product with
-        // balanced output digits lies in (-r, 0.03 r) and leaves balanced
-        // digits, as the DFT wants.  Elements and factors are asked for two
-        // products ahead, one once half the lane's results are held: their
-        // loads hide behind those products; addresses are opaque bases plus
-        // wave-uniform offsets
-        fr f[kPerT], v[kPerT];
-        auto load = [&](auto k_) {
-          constexpr int k = decltype(k_)::value;
-          const fr* q = pm;
-          const fr* d = sp;
-          asm volatile("" : "+v"(q), "+v"(d));
-          v[k] = fr_load(d + (uint64_t)(A * k) * estride);
-          f[k] = fr_load(q + (uint64_t)(A * k) * estride);
-          mem_here();
-        };
-        static_for<0, 2>(load);
-        static_for<0, kPerT>([&](auto k_) {
-          constexpr int k = decltype(k_)::value;
-          constexpr int n = k < kPerT / 2 - 1 ? k + 2 : k + 1;
-          if constexpr (n < kPerT && k != kPerT / 2 - 1) load(std::integral_constant<int, n>());
-          v9 xx;
-          unpack_ext(v[k].l, xx.l);
-          uint32_t w[9];
-          pbd_unpack(f[k].l, w);
-          x[k] = v9_mul<false, false, true>(xx, w);
-          pin9(x[k]);
-        });
-      } else {
-        fr raw[kPerT];
-        static_for<0, kPerT>([&](auto r2_) {
-          constexpr int r2 = decltype(r2_)::value;
-          raw[r2] = fr_load(src + pos0 + (uint64_t)(rho1 + A * r2) * estride);
-        });
-        static_for<0, kPerT>([&](auto r2_) {
-          constexpr int r2 = decltype(r2_)::value;
-          unpack_ext(raw[r2].l, x[r2].l);
-        });
-      }
+    // plain digits of any 256-bit words: caller data (optionally times a
+    // premultiplication factor) or a previous pass's
+    if (a.premul) {
+      const fr* pm = a.premul + ((uint64_t)(poly & a.pm_mask) << a.lgN) + pos0 + (uint64_t)rho1 * estride;
+      const fr* sp = src + pos0 + (uint64_t)rho1 * estride;
+      // factors are pbd words of c R' (the coset powers); the product with
+      // plain output digits lies in (-r, 0.03 r) and leaves such
+      // digits, as the DFT wants.  Elements and factors are asked for two
+      // products ahead, one once half the lane's results are held: their
+      // loads hide behind those products; addresses are opaque bases plus
+      // wave-uniform offsets
+      fr f[kPerT], v[kPerT];
+      auto load = [&](auto k_) {
+        constexpr int k = decltype(k_)::value;
+        const fr* q = pm;
+        const fr* d = sp;
+        asm volatile("" : "+v"(q), "+v"(d));
+        v[k] = fr_load(d + (uint64_t)(A * k) * estride);
+        f[k] = fr_load(q + (uint64_t)(A * k) * estride);
+        mem_here();
+      };
+      static_for<0, 2>(load);
+      static_for<0, kPerT>([&](auto k_) {
+        constexpr int k = decltype(k_)::value;
+        constexpr int n = k < kPerT / 2 - 1 ? k + 2 : k + 1;
+        if constexpr (n < kPerT && k != kPerT / 2 - 1) load(std::integral_constant<int, n>());
+        v9 xx;
+        split29(v[k].l, xx.l);
+        uint32_t w[9];
+        pbd_unpack(f[k].l, w);
+        x[k] = v9_mul<false, false, false>(xx, w);
+        pin9(x[k]);
+      });
     } else {
+      fr raw[kPerT];
       static_for<0, kPerT>([&](auto r2_) {
         constexpr int r2 = decltype(r2_)::value;
-        const fr raw = fr_load(src + pos0 + (uint64_t)(rho1 + A * r2) * estride);
-        pbd_unpack(raw.l, x[r2].l);
+        raw[r2] = fr_load(src + pos0 + (uint64_t)(rho1 + A * r2) * estride);
+      });
+      static_for<0, kPerT>([&](auto r2_) {
+        constexpr int r2 = decltype(r2_)::value;
+        split29(raw[r2].l, x[r2].l);
       });
     }
   }
   dft_dif<kLgPerT, 0>(x, rows);  // x[brev3(k2)] = sum_rho2 z[rho1 + A rho2] w8^(rho2 k2)
   v9 (&y)[kPerT] = x;
   if constexpr (LA > 0) {
-    // back to balanced digits of small values, so that DFT_A again starts from
-    // balanced digits: k2 = 0 and wave rho1 = 0 take no twiddle and are reduced
-    // (about 45 instructions), the others' products leave balanced digits (BT)
+    // back to plain digits of small values, so that DFT_A again starts from
+    // such: k2 = 0 and wave rho1 = 0 take no twiddle and are reduced (about 45
+    // instructions)
     auto reduce = [&](v9& v) {
       v9 t0;
-      reduce_centered(v.l, t0.l);
+      reduce_below_2r(v.l, t0.l);
       v = t0;
       pin9(v);
     };
@@ -394,7 +403,7 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
       if (rho1 == 0) {
         reduce(v);
       } else {
-        v = v9_mul_rows<2, true>(v, tw + step * k2, g, tw + step * (k2 < kPerT - 1 ? k2 + 1 : k2));
+        v = v9_mul_rows<2, false>(v, tw + step * k2, g, tw + step * (k2 < kPerT - 1 ? k2 + 1 : k2));
         pin9(v);
       }
     });
@@ -513,10 +522,7 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
       pin9(v);
       uint32_t w[9];
       pbd_unpack(cur.l, w);
-      v = v9_mul<false, true, true>(v, w);
-      fr o;
-      pbd_pack(v.l, o.l);
-      fr_store(dst + row(i), o);
+      fr_store(dst + row(i), v9_mul_word(v, w));
     });
   }
 }
