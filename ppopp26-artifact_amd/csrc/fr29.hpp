@@ -221,8 +221,7 @@ PL_HD29 void add_r256(uint32_t* x) {
 // [29 i, 29 i + 29), i < 8, hold digits b_i in [-2^28, 2^28) as 29-bit two's
 // complement and whose bits [232, 256) hold b_8 in [-2^23, 2^23) as 24-bit two's
 // complement; its value is sum b_i 2^(29 i).  Pass twiddle tables hold their
-// factors this way, and the one-element-per-lane kernels hand intermediate
-// results from launch to launch in it.
+// factors this way.
 
 // the nine signed limbs of a pbd word
 PL_HD29 void pbd_unpack(const uint32_t* x, uint32_t* b) {
@@ -393,25 +392,30 @@ __device__ __forceinline__ void mont29_word_dev(const uint32_t* x, const uint32_
 }
 
 // (a w + b v) / 2^261 mod r: two per-lane products with one reduction, 234
-// multiply-adds where two mont29 take 306.  For |a_i|, |b_i| <= 2^29 and
-// balanced factor digits a column stays below 18 * 2^57 + 8 * 2^58 + 2^34 <
-// 2^62; the value is within (T - r, T], T = (a w + b v) / 2^261.  Output digits
-// balanced.
+// multiply-adds where two mont29 take 306.  For |a_i|, |b_i| < 2^30 and
+// balanced factor digits a column stays below 18 * 2^58 + 8 * 2^58 + 2^35 <
+// 2^62.8; output digits plain.  With T = (a w + b v) / 2^261 the value lies in
+// (T - r, T], or with WORD in (T + r/2, T + 3r/2) as in mont29_word.
+template <bool WORD>
 __device__ __forceinline__ void dual29_dev(const uint32_t* a, const uint32_t* w, const uint32_t* b,
                                            const uint32_t* v, uint32_t* t) {
   uint32_t m[9];
   uint64_t acc[18];
   static_for<0, 17>([&](auto k_) {
     constexpr int k = decltype(k_)::value;
-    Mont29Col<k, false, (k >= 10)>::run(acc[k], k ? acc[k ? k - 1 : 0] : 0, a, w, m);
+    uint64_t prev = k ? acc[k ? k - 1 : 0] : 0;
+    if constexpr (WORD && k == 9) prev += 3u << 28;
+    Mont29Col<k, false, false>::run(acc[k], prev, a, w, m);
     Mac29Col<k>::run(acc[k], b, v);
     const uint32_t lo = (uint32_t)acc[k];
-    if constexpr (k <= 8)
+    if constexpr (WORD && k == 8)
+      m[k] = sext29(lo) - (1u << 29);
+    else if constexpr (k <= 8)
       m[k] = lo & kMask29;
     else
-      t[k - 9] = sext29(lo);
+      t[k - 9] = lo & kMask29;
   });
-  Mont29Col<17, false, true>::run(acc[17], acc[16], a, w, m);
+  Mont29Col<17, false, false>::run(acc[17], acc[16], a, w, m);
   t[8] = (uint32_t)acc[17];
 }
 

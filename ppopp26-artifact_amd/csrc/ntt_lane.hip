@@ -20,16 +20,18 @@
 // own four pairs, which carry 2^-lg for the inverse.
 //
 // lg <= kLaneOne: one launch.  Above: two, M'0 = 2^ceil(lg/2) columns at stride
-// N / M'0 into the caller's scratch as pbd words with the twiddle w_N^(J kappa),
+// N / M'0 into the caller's scratch as 256-bit words (not reduced; the step's
+// product centres its last Montgomery digit and adds r, mont29_word) with the
+// twiddle w_N^(J kappa),
 // then contiguous rows in natural order.  Against the pass kernels, one forward
 // transform: 2^9 24.6 -> 9.2 us, 2^12 30.3 -> 10.5, 2^14 42.0 -> 11.5, 2^16
 // 46.0 -> 14.5, 2^18 57.4 -> 43.2 (the caller's own launches take 7.4 of it).
 //
-// Bounds: inputs are balanced digits (|l| <= 2^28), so the sums have |l| <= 2^29;
+// Bounds: inputs are plain digits in [0, 2^29), so the sums have |l| < 2^30;
 // values: a caller's 2^256 < 2.21 r makes the first sums 4.42 r each and the
-// step's result within (-1.126 r, 0.126 r), later steps within (-1.065 r,
-// 0.065 r) (x w / 2^261 < 0.01415 |x| for w < r), which fits a pbd word
-// (1.104 r).
+// step's result within (-1.126 r, 0.126 r), later steps within (-1.07 r,
+// 0.07 r) (x w / 2^261 < 0.01415 |x| for w < r), a stored word in (0.43 r,
+// 1.57 r).
 #include <type_traits>
 
 #include "ntt_pass.hpp"
@@ -49,7 +51,6 @@ struct LaneArgs {
   uint32_t lgN;
   uint32_t lgI;         // LAST: output interleave
   uint32_t inverse;
-  uint32_t in_ext;      // caller data (any 256-bit values), not pbd words
 };
 
 // the limb of lane CTRL's choice within the quad
@@ -117,15 +118,11 @@ __global__ void __launch_bounds__(lane_threads(m), 4) ntt_lane_kernel(LaneArgs a
     const uint32_t pos = lane_pos(tau, lane_mu(m, 0), lane_lr(m, 0));
     const uint32_t at = LAST ? (lp << m) + pos : lp + (pos << lgL);
     const fr raw = fr_load(a.in + poly * a.in_pstride + at);
-    if (a.in_ext) {
-      unpack_ext(raw.l, x.l);
-      if (!LAST && a.premul) {
-        uint32_t w[9];
-        pbd_unpack(fr_load(a.premul + (((poly & a.pm_mask) << lg) + at)).l, w);
-        x = v9_mul<false, false, true>(x, w);
-      }
-    } else {
-      pbd_unpack(raw.l, x.l);
+    split29(raw.l, x.l);
+    if (!LAST && a.premul) {
+      uint32_t w[9];
+      pbd_unpack(fr_load(a.premul + (((poly & a.pm_mask) << lg) + at)).l, w);
+      x = v9_mul<false, false, false>(x, w);
     }
   }
   // kappa, the output index of this lane's last element: its position's
@@ -144,6 +141,7 @@ __global__ void __launch_bounds__(lane_threads(m), 4) ntt_lane_kernel(LaneArgs a
   }
   static_for<0, NS>([&](auto s_) {
     constexpr int s = decltype(s_)::value, lr = lane_lr(m, s);
+    constexpr bool word = !LAST && s + 1 == NS;  // this step's result is stored between launches
     uint32_t f1[9], f2[9];
     pbd_unpack(w1.l, f1);
     if constexpr (lr == 2) pbd_unpack(w2.l, f2);
@@ -166,7 +164,8 @@ __global__ void __launch_bounds__(lane_threads(m), 4) ntt_lane_kernel(LaneArgs a
       const uint32_t neg = 0u - (tau & 1);
 #pragma unroll
       for (int i = 0; i < 9; i++) u.l[i] = quad<0, 0, 2, 2>(x.l[i]) + ((quad<1, 1, 3, 3>(x.l[i]) ^ neg) - neg);
-      x = v9_mul<false, false, true>(u, f1);
+      if constexpr (word) mont29_word_dev(u.l, f1, x.l);
+      else x = v9_mul<false, false, false>(u, f1);
     } else {
       // lanes 0, 1: x_q + x_(q+2); lanes 2, 3: x_(q-2) - x_q
       const uint32_t neg = 0u - ((tau >> 1) & 1);
@@ -178,7 +177,7 @@ __global__ void __launch_bounds__(lane_threads(m), 4) ntt_lane_kernel(LaneArgs a
         u.l[i] = quad<0, 2, 0, 2>(p[i]);
         v.l[i] = quad<1, 3, 1, 3>(p[i]);
       }
-      dual29_dev(u.l, f1, v.l, f2, x.l);
+      dual29_dev<word>(u.l, f1, v.l, f2, x.l);
     }
     if constexpr (s + 1 < NS) {
       const uint32_t wr = (c << m) + lane_pos(tau, lane_mu(m, s), lr);
@@ -204,7 +203,7 @@ __global__ void __launch_bounds__(lane_threads(m), 4) ntt_lane_kernel(LaneArgs a
     fr_store(dst + ((uint64_t)(lp + (kappa << lgL)) << lgI), v9_canonical(x));
   } else {
     fr o;
-    pbd_pack(x.l, o.l);
+    join29(x.l, o.l);
     fr_store(a.out + (poly << lg) + lp + (kappa << lgL), o);
   }
 }
@@ -294,7 +293,6 @@ hipError_t lane_launch(const Domain& d, const NttCall& c, hipStream_t s) {
   a.inverse = c.inverse;
   a.in = c.in;
   a.in_pstride = c.in_pstride;
-  a.in_ext = 1;
   a.pm_mask = c.pm_mask;
   const int m0 = one ? lg : (lg + 1) / 2, m1 = lg - m0;
   if (!one) {
@@ -306,7 +304,6 @@ hipError_t lane_launch(const Domain& d, const NttCall& c, hipStream_t s) {
     a.premul = nullptr;
     a.in = c.tmp;
     a.in_pstride = 1ull << lg;
-    a.in_ext = 0;
   }
   a.out = c.out;
   a.post = c.post;
