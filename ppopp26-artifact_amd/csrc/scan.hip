@@ -16,6 +16,7 @@
 // carry.  About 3 mulmods per element in total, three memory sweeps.
 #include "fr29.hpp"
 #include "pl_internal.hpp"
+#include "run_stage.hpp"
 
 namespace pl {
 
@@ -27,6 +28,10 @@ constexpr int kLgPer = PL_SCAN_LGPER;        // elements per thread: 2^kLgPer
 constexpr int kPer = 1 << kLgPer;
 constexpr int kSeg = kScanThreads * kPer;    // elements per block
 constexpr int kLgSeg = 8 + kLgPer;
+
+// the bulk kernels move their runs in chunks of four elements (run_stage.hpp)
+constexpr int kChunk = 4;
+typedef RunStage<kChunk> Stage;
 
 static inline unsigned sgrid(uint64_t n) { return (unsigned)((n + kSeg - 1) / kSeg); }
 
@@ -319,6 +324,48 @@ __device__ fr block_suffix(fr v, uint4 (*l)[kScanThreads], const fr* pw) {
   return v;
 }
 
+// Run suffixes of a block, S_t = sum_(t' >= t) v_t' mu^(t' - t): six exchange
+// steps inside the wave, then the sum over the waves after: with D_w = s at the
+// end of wave w, S_t += mu^(64 - lane) D_w (f: that power's digits).  The
+// running value is signed limbs: products with balanced digits (2^28) summed
+// seven times.  pw(s, p): the balanced digits of mu^(2^s) R', s < 7.
+template <class Pw>
+__device__ __forceinline__ fr run_suffix(v9 v, const uint32_t (&f)[9], uint32_t (*wt)[9], Pw pw) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int s = 0; s < 6; s++) {
+    v9 o;
+#pragma unroll
+    for (int i = 0; i < 9; i++) o.l[i] = (uint32_t)__shfl_down((int)v.l[i], 1 << s);
+    uint32_t p[9];
+    pw(s, p);
+    o = v9_mul<false, false, true>(o, p);
+    if (lane + (1 << s) < 64) v = v9_add(v, o);
+  }
+  if (lane == 0) {
+    const fr c = v9_canonical(v);
+    v9 b;
+    unpack_ext(c.l, b.l);
+#pragma unroll
+    for (int i = 0; i < 9; i++) wt[w][i] = b.l[i];
+  }
+  __syncthreads();
+  if (w < 3) {
+    v9 d;  // D_w: the later waves' values by Horner in mu^64
+    uint32_t p[9];
+    pw(6, p);
+#pragma unroll
+    for (int i = 0; i < 9; i++) d.l[i] = wt[3][i];
+    for (int k = 2; k > w; k--) {
+      d = v9_mul<false, false, true>(d, p);
+#pragma unroll
+      for (int i = 0; i < 9; i++) d.l[i] += wt[k][i];
+    }
+    v = v9_add(v, v9_mul<false, false, true>(d, f));
+  }
+  return v9_canonical(v);
+}
+
 // the factor of the word w R' for a whole kernel's Horner steps
 __device__ __forceinline__ rows_all rp_rows(const fr* w) { return rows29_spread(rows29_make<true>(fr_load(w))); }
 
@@ -411,12 +458,22 @@ __global__ void __launch_bounds__(kScanThreads) sfx_reduce_kernel(const fr* a, u
 }
 
 // partial[b] as sfx_reduce_kernel computes it, from contiguous runs (thread t
-// owns the kPer elements the down-sweep gives it): the local Horner value L_t
-// goes to lt for the down-sweep (which then skips its own), then the block
-// suffix over the L_t gives the block's value at thread 0.
+// owns the kPer elements the down-sweep gives it).  lt takes what the
+// down-sweep needs of each run, so that it starts at its rescan.  TAB, the
+// level that holds the data: the suffix S_t of the block's runs (run_suffix,
+// with mu = m^kPer and its powers in mutab), and the block's value is S_0.
+// Otherwise the run's Horner value L_t, scanned again below with the carry.
+// The runs come as 128-byte chunks through LDS (run_stage.hpp).
+// Division of 2^24: this kernel 230 -> 200 us, bound by its products; the
+// down-sweep 331 -> 195, a copy's time; with the chunks alone, the scans as
+// before, 200 and 266.  Opening 841 -> 784 us, of 2^22 290 -> 263.
+template <bool TAB>
 __global__ void __launch_bounds__(kScanThreads) sfx_run_reduce_kernel(const fr* a, uint64_t n, const fr* pw,
-                                                                      fr* partial, fr* lt, PwExt ext) {
-  __shared__ uint4 l[2][kScanThreads];
+                                                                      fr* partial, fr* lt, PwExt ext,
+                                                                      const fr* mutab) {
+  __shared__ uint4 l[2][TAB ? 1 : kScanThreads];
+  __shared__ uint32_t wt[4][9];
+  __shared__ uint4 stage[Stage::kSlots * kScanThreads / 64];
   const int t = threadIdx.x;
   uint32_t blk = blockIdx.x;
   if (ext.count) {
@@ -427,51 +484,95 @@ __global__ void __launch_bounds__(kScanThreads) sfx_run_reduce_kernel(const fr* 
     blk--;
   }
   const uint64_t tid = (uint64_t)blk * kScanThreads + t;
-  const uint64_t base = tid * kPer;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const uint64_t w0 = ((uint64_t)blk * kScanThreads + 64 * wave) * kPer;  // the wave's first element
+  const bool all = w0 + 64 * kPer <= n;
+  const int64_t lim = (int64_t)(n - w0);
+  const Stage st{stage + Stage::kSlots * wave, t & 63};
+  uint4 raw[Stage::P];
+  st.fetch(a + w0 + kPer - kChunk, kPer, lim - (kPer - kChunk), all, raw);
   const rows_all m = rp_rows(pw);
-  fr e[kPer];
-  static_for<0, kPer>([&](auto k_) {
-    constexpr int k = decltype(k_)::value;
-    e[k] = base + k < n ? fr_load(a + base + k) : fr_zero();
+  // Horner over the run in signed limbs (horner29), top chunk first; the next
+  // chunk is asked for before the chain over this one
+  v9 hv;
+  static_for<0, kPer / kChunk>([&](auto c_) {
+    constexpr int k0 = kPer - kChunk * (decltype(c_)::value + 1);
+    st.put(raw);
+    if constexpr (k0 > 0) st.fetch(a + w0 + (k0 - kChunk), kPer, lim - (k0 - kChunk), all, raw);
+    static_for<0, kChunk>([&](auto j_) {
+      constexpr int j = kChunk - 1 - decltype(j_)::value;
+      v9 x;
+      split29(st.get(j).l, x.l);
+      if constexpr (k0 + j == kPer - 1) hv = x;
+      else hv = v9_add(v9_mul_all<false>(hv, m), x);
+    });
   });
-  const fr h = horner29<kPer>(e, m);
-  fr_store(lt + tid, h);
-  const fr v = block_suffix<kLgPer>(h, l, pw);
-  if (t == 0) fr_store(partial + blk, v);
+  const fr h = v9_canonical(hv);
+  if constexpr (TAB) {
+    v9 v;
+    unpack_ext(h.l, v.l);
+    uint32_t f[9];
+    unpack_ext(fr_load(mutab + 64 - (t & 63)).l, f);
+    const fr S = run_suffix(v, f, wt, [&](int s, uint32_t* p) { unpack_ext(fr_load(pw + kLgPer + s).l, p); });
+    fr_store(lt + tid, S);
+    if (t == 0) fr_store(partial + blk, S);
+  } else {
+    fr_store(lt + tid, h);
+    const fr v = block_suffix<kLgPer>(h, l, pw);
+    if (t == 0) fr_store(partial + blk, v);
+  }
 }
 
 // out[i] = s_{i+1} within each block given carry[b] = s at the block's end
 // (nullptr: zero); total (block 0) = s_0.  out may equal a.
-// LT: the local Horner values come from sfx_run_reduce_kernel (lt); the
-// elements are then loaded only for the rescan, in two halves, so that fewer
-// values are live (more waves per SIMD).  Otherwise computed here.
-template <int LG, bool LT>
-__global__ void __launch_bounds__(kScanThreads) sfx_down_kernel(const fr* a, fr* out, uint64_t n, const fr* pw,
-                                                                 const fr* carry, fr* total, const fr* lt) {
+// LT: lt comes from sfx_run_reduce_kernel; the elements are then read only for
+// the rescan, in chunks through LDS (run_stage.hpp).  With TAB lt holds the run
+// suffixes and the carry at the end of run t is S_(t+1) + mu^(255 - t) K, one
+// product where the block suffix takes eight behind 16 barriers.  Otherwise
+// the local Horner values are scanned here.
+template <int LG, bool LT, bool TAB>
+__global__ void __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(LT ? 4 : 1)))
+sfx_down_kernel(const fr* a, fr* out, uint64_t n, const fr* pw,
+                                                                 const fr* carry, fr* total, const fr* lt,
+                                                                 const fr* mutab) {
+  static_assert(!TAB || LT, "run suffixes come from the reduce");
   constexpr int kPer = ScanGeom<LG>::kPer, kLgSeg = ScanGeom<LG>::kLgSeg, kLgPer = LG;
-  __shared__ uint4 l[2][kScanThreads];
+  __shared__ uint4 stage[LT ? Stage::kSlots * kScanThreads / 64 : 1];
   const int t = threadIdx.x;
   const uint64_t base = ((uint64_t)blockIdx.x << kLgSeg) + (uint64_t)t * kPer;
+  [[maybe_unused]] uint4 raw[Stage::P];
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const uint64_t w0 = ((uint64_t)blockIdx.x << kLgSeg) + (uint64_t)(64 * wave) * kPer;  // the wave's first element
+  const bool all = w0 + 64 * kPer <= n;
+  const int64_t lim = (int64_t)(n - w0);
+  [[maybe_unused]] const Stage st{stage + (LT ? Stage::kSlots * wave : 0), t & 63};
+  if constexpr (LT) st.fetch(a + w0 + (kPer - kChunk), kPer, lim - (kPer - kChunk), all, raw);
   const v9 row = rows29_make<true>(fr_load(pw));  // m's rows, spread where they are used
-  // local Horner: L = sum_k e_k m^k
-  fr h;
-  if constexpr (LT) {
-    h = fr_load(lt + ((uint64_t)blockIdx.x * kScanThreads + t));
-  } else {
-    fr e[kPer];
-    static_for<0, kPer>([&](auto k_) {
-      constexpr int k = decltype(k_)::value;
-      e[k] = base + k < n ? fr_load(a + base + k) : fr_zero();
-    });
-    h = horner29<kPer>(e, rows29_spread(row));
-  }
-  // fold the block carry into the last thread: s(start of thread 255) = L + m^kPer K
   fr K = carry ? fr_load(carry + blockIdx.x) : fr_zero();
-  if (t == kScanThreads - 1) h = fr_add(h, mulp(K, fr_load(pw + kLgPer)));
-  fr v = block_suffix<LG>(h, l, pw);  // s at the start of this thread's run
-  // carry-in at this thread's end = s at the start of thread t+1
-  fr cin = t + 1 < kScanThreads ? lds_get(l, t + 1) : K;
-  if (total && blockIdx.x == 0 && t == 0) fr_store(total, v);
+  fr cin;  // s at the start of thread t+1
+  if constexpr (TAB) {
+    cin = mulp(K, fr_load(mutab + (kScanThreads - 1 - t)));
+    if (t + 1 < kScanThreads) cin = fr_add(cin, fr_load(lt + ((uint64_t)blockIdx.x * kScanThreads + t + 1)));
+  } else {
+    // local Horner: L = sum_k e_k m^k
+    fr h;
+    if constexpr (LT) {
+      h = fr_load(lt + ((uint64_t)blockIdx.x * kScanThreads + t));
+    } else {
+      fr e[kPer];
+      static_for<0, kPer>([&](auto k_) {
+        constexpr int k = decltype(k_)::value;
+        e[k] = base + k < n ? fr_load(a + base + k) : fr_zero();
+      });
+      h = horner29<kPer>(e, rows29_spread(row));
+    }
+    // fold the block carry into the last thread: s(start of thread 255) = L + m^kPer K
+    if (t == kScanThreads - 1) h = fr_add(h, mulp(K, fr_load(pw + kLgPer)));
+    __shared__ uint4 l[2][kScanThreads];
+    const fr v = block_suffix<LG>(h, l, pw);  // s at the start of this thread's run
+    cin = t + 1 < kScanThreads ? lds_get(l, t + 1) : K;
+    if (total && blockIdx.x == 0 && t == 0) fr_store(total, v);
+  }
   // rescan: s_k = e_k + m s_{k+1}, out[base + k] = s_{k+1} (signed limbs,
   // canonical where stored); out may equal a: each half's elements are read
   // before its outputs are written, and the low half's outputs only overwrite
@@ -479,24 +580,41 @@ __global__ void __launch_bounds__(kScanThreads) sfx_down_kernel(const fr* a, fr*
   const rows_all m = rows29_spread(row);
   v9 sn;
   split29(cin.l, sn.l);
-  constexpr int G = kPer > 1 ? 2 : 1, Q = kPer / G;
-  static_for<0, G>([&](auto g_) {
-    constexpr int top = kPer - 1 - decltype(g_)::value * Q;  // highest index of this half
-    fr e[Q];
-    static_for<0, Q>([&](auto j_) {
-      constexpr int k = top - decltype(j_)::value;
-      e[top - k] = k > 0 && base + k < n ? fr_load(a + base + k) : fr_zero();
-    });
-    static_for<0, Q>([&](auto j_) {
-      constexpr int k = top - decltype(j_)::value;
-      if (base + k < n) fr_store(out + base + k, k == kPer - 1 ? cin : v9_canonical(sn));
-      if constexpr (k > 0) {
+  if constexpr (LT) {
+    // the next chunk is asked for before the chain over this one
+    static_for<0, kPer / kChunk>([&](auto c_) {
+      constexpr int k0 = kPer - kChunk * (decltype(c_)::value + 1);
+      st.put(raw);
+      if constexpr (k0 > 0) st.fetch(a + w0 + (k0 - kChunk), kPer, lim - (k0 - kChunk), all, raw);
+      static_for<0, kChunk>([&](auto j_) {
+        constexpr int j = kChunk - 1 - decltype(j_)::value, k = k0 + j;
         v9 x;
-        split29(e[top - k].l, x.l);
-        sn = v9_add(v9_mul_all<false>(sn, m), x);
-      }
+        split29(st.get(j).l, x.l);
+        st.set(j, k == kPer - 1 ? cin : v9_canonical(sn));
+        if constexpr (k > 0) sn = v9_add(v9_mul_all<false>(sn, m), x);
+      });
+      st.store(out + w0 + k0, kPer, lim - k0, all);
     });
-  });
+  } else {
+    constexpr int G = kPer > 1 ? 2 : 1, Q = kPer / G;
+    static_for<0, G>([&](auto g_) {
+      constexpr int top = kPer - 1 - decltype(g_)::value * Q;  // highest index of this half
+      fr e[Q];
+      static_for<0, Q>([&](auto j_) {
+        constexpr int k = top - decltype(j_)::value;
+        e[top - k] = k > 0 && base + k < n ? fr_load(a + base + k) : fr_zero();
+      });
+      static_for<0, Q>([&](auto j_) {
+        constexpr int k = top - decltype(j_)::value;
+        if (base + k < n) fr_store(out + base + k, k == kPer - 1 ? cin : v9_canonical(sn));
+        if constexpr (k > 0) {
+          v9 x;
+          split29(e[top - k].l, x.l);
+          sn = v9_add(v9_mul_all<false>(sn, m), x);
+        }
+      });
+    });
+  }
 }
 
 __global__ void zero_kernel(fr* p, uint64_t n) {
@@ -513,11 +631,11 @@ hipError_t fill_zero(fr* p, uint64_t n, hipStream_t s) {
 // doublings) is m R' in the stored form; squares stay in that form.  Level L
 // of a scan (values combined 4096^L at a time) uses pw + 12 L: its multiplier
 // is m^(4096^L), whose powers of two continue the same squaring chain.
-// tab (evaluation, 128 threads): also tab[t] = m^t R' for t < 256, which the
-// reduce multiplies each thread's value by; the second wave extends it by
-// doubling (step j fills [2^j, 2^(j+1)) from pw[j]) while thread 0 raises the
-// next square.
-__global__ void sfx_powers_kernel(const fr* src, int neg, fr* pw, int count, fr* tab) {
+// tab (128 threads): also tab[t] = m^(t 2^sh) R' for t < 256: sh = 0 for the
+// evaluation's reduce, which multiplies each thread's value by m^t, kLgPer for
+// the run suffixes.  The second wave extends it by doubling (step j fills
+// [2^j, 2^(j+1)) from pw[sh + j]) while thread 0 raises the next square.
+__global__ void sfx_powers_kernel(const fr* src, int neg, fr* pw, int count, fr* tab, int sh) {
   const int t = threadIdx.x;
   fr m;
   if (t == 0) {
@@ -535,9 +653,9 @@ __global__ void sfx_powers_kernel(const fr* src, int neg, fr* pw, int count, fr*
     if (t == 0) fr_store(pw + j, m);
     if (tab) __syncthreads();  // pw[j] and the table's entries below 2^j visible
     if (t == 0 && j + 1 < count) m = mulp(m, m);
-    if (tab && j < 8 && t >= 64) {
-      for (int i = t - 64; i < (1 << j); i += 64)
-        fr_store(tab + (1 << j) + i, mulp(fr_load(tab + i), fr_load(pw + j)));
+    if (tab && j >= sh && j < sh + 8 && t >= 64) {
+      const int h = 1 << (j - sh);
+      for (int i = t - 64; i < h; i += 64) fr_store(tab + h + i, mulp(fr_load(tab + i), fr_load(pw + j)));
     }
   }
 }
@@ -554,6 +672,11 @@ static int sfx_levels(uint64_t n) {
   return L;
 }
 static int sfx_pw_count(uint64_t n) { return kPw + kLgSeg * (sfx_levels(n) - 1); }
+// the entries that the powers kernel raises: level 0's, for a single block those
+// that its geometry reads (sfx_one_block: m^256, or mu^(2^s) up to s = 7)
+static int sfx_pw_first(uint64_t n) {
+  return n <= 512 ? 9 : n <= 1024 ? 10 : kPw;
+}
 // the entries beyond level 0's, for the first reduce launch (none for one level)
 static PwExt pw_ext(fr* pw, int np) { return np > kPw ? PwExt{pw, kPw, np} : PwExt{nullptr, 0, 0}; }
 
@@ -566,28 +689,33 @@ static uint64_t sfx_scratch_elems(uint64_t n) {
   return tot;
 }
 
+// the only block of a level: the smallest geometry that covers it, as the
+// chains of 2^LG dependent steps are what it takes (2001
+// coefficients: reduce 9.5 -> 6.9 us, sweep 25.4 -> 20.2 with 8 per thread
+// for 16; opening of 1001 63.6 -> 40.4 us)
+template <int LG>
+static void sfx_one_block(const fr* a, fr* out, uint64_t n, const fr* pw, fr* total, const fr* mt, hipStream_t s) {
+  const fr* none = nullptr;
+  if (out)
+    hipLaunchKernelGGL((sfx_down_kernel<LG, false, false>), dim3(1), dim3(kScanThreads), 0, s, a, out, n, pw, none, total, none,
+                       none);
+  else  // the reduce kernel's tree value is s_0
+    hipLaunchKernelGGL(sfx_reduce_kernel<LG>, dim3(1), dim3(kScanThreads), 0, s, a, n, pw, total,
+                       PwExt{nullptr, 0, 0}, mt);
+}
+
 // suffix scan with powers table pw (this level's m): out[i] = s_{i+1} (if out),
-// *total = s_0 (if total).  out == nullptr: reduction only.  A top level of at
-// most 256 values runs one element per thread.
+// *total = s_0 (if total).  out == nullptr: reduction only.  mt (the level
+// that holds the data): the powers kernel's table, of m^t for a reduction, of
+// m^(kPer t) with a down-sweep.
 static hipError_t suffix_scan(const fr* a, fr* out, uint64_t n, const fr* pw, fr* total, fr* scratch, hipStream_t s,
                               PwExt ext = PwExt{nullptr, 0, 0}, const fr* mt = nullptr) {
   if (n <= (uint64_t)kSeg) {
-    const bool tiny = n <= (uint64_t)kScanThreads;
-    if (out) {
-      if (tiny)
-        hipLaunchKernelGGL((sfx_down_kernel<0, false>), dim3(1), dim3(kScanThreads), 0, s, a, out, n, pw, (const fr*)nullptr,
-                           total, (const fr*)nullptr);
-      else
-        hipLaunchKernelGGL((sfx_down_kernel<kLgPer, false>), dim3(1), dim3(kScanThreads), 0, s, a, out, n, pw,
-                           (const fr*)nullptr, total, (const fr*)nullptr);
-    } else {
-      // one block: the reduce kernel's tree value is s_0
-      const PwExt none{nullptr, 0, 0};
-      if (tiny)
-        hipLaunchKernelGGL(sfx_reduce_kernel<0>, dim3(1), dim3(kScanThreads), 0, s, a, n, pw, total, none, mt);
-      else
-        hipLaunchKernelGGL(sfx_reduce_kernel<kLgPer>, dim3(1), dim3(kScanThreads), 0, s, a, n, pw, total, none, mt);
-    }
+    if (n <= 256) sfx_one_block<0>(a, out, n, pw, total, mt, s);
+    else if (n <= 512) sfx_one_block<1>(a, out, n, pw, total, mt, s);
+    else if (n <= 1024) sfx_one_block<2>(a, out, n, pw, total, mt, s);
+    else if (n <= 2048) sfx_one_block<3>(a, out, n, pw, total, mt, s);
+    else sfx_one_block<kLgPer>(a, out, n, pw, total, mt, s);
     return hipGetLastError();
   }
   const uint64_t nb = (n + kSeg - 1) / kSeg;
@@ -597,15 +725,23 @@ static hipError_t suffix_scan(const fr* a, fr* out, uint64_t n, const fr* pw, fr
   // with a down-sweep, the reduce runs over the down-sweep's runs and keeps
   // their local Horner values; a reduction alone reads strided (coalesced)
   const unsigned grid = sgrid(n) + (ext.count ? 1 : 0);
-  if (out)
-    hipLaunchKernelGGL(sfx_run_reduce_kernel, dim3(grid), dim3(kScanThreads), 0, s, a, n, pw, part, lt, ext);
+  const dim3 th(kScanThreads);
+  if (!out)
+    hipLaunchKernelGGL(sfx_reduce_kernel<kLgPer>, dim3(grid), th, 0, s, a, n, pw, part, ext, mt);
+  else if (mt)
+    hipLaunchKernelGGL(sfx_run_reduce_kernel<true>, dim3(grid), th, 0, s, a, n, pw, part, lt, ext, mt);
   else
-    hipLaunchKernelGGL(sfx_reduce_kernel<kLgPer>, dim3(grid), dim3(kScanThreads), 0, s, a, n, pw, part, ext, mt);
+    hipLaunchKernelGGL(sfx_run_reduce_kernel<false>, dim3(grid), th, 0, s, a, n, pw, part, lt, ext, mt);
   // carry[b] = s at the end of block b = sum_{b' > b} part[b'] (m^4096)^(b'-b-1)
   hipError_t e = suffix_scan(part, out ? carry : nullptr, nb, pw + kLgSeg, total, lt + nb * kScanThreads, s);
   if (e != hipSuccess || !out) return e;
-  hipLaunchKernelGGL((sfx_down_kernel<kLgPer, true>), dim3(sgrid(n)), dim3(kScanThreads), 0, s, a, out, n, pw,
-                     (const fr*)carry, (fr*)nullptr, (const fr*)lt);
+  fr* none = nullptr;
+  if (mt)
+    hipLaunchKernelGGL((sfx_down_kernel<kLgPer, true, true>), dim3(sgrid(n)), th, 0, s, a, out, n, pw,
+                       (const fr*)carry, none, (const fr*)lt, mt);
+  else
+    hipLaunchKernelGGL((sfx_down_kernel<kLgPer, true, false>), dim3(sgrid(n)), th, 0, s, a, out, n, pw,
+                       (const fr*)carry, none, (const fr*)lt, mt);
   return hipGetLastError();
 }
 
@@ -639,7 +775,9 @@ static hipError_t suffix_scan(const fr* a, fr* out, uint64_t n, const fr* pw, fr
 // The launch boundaries carry the tables and values between blocks; a
 // release/acquire hand-off inside one launch costs more than a launch here
 // (it writes back and invalidates the L2 of every XCD involved).
-constexpr uint64_t kLatMin = 1ull << 12;
+// from here up three launches beat the powers chain and its single block
+// (opening of 2001 42.3 against 47.9 us; of 1001 the single block's 40.4)
+constexpr uint64_t kLatMin = (1ull << 10) + 1;
 constexpr uint64_t kLatMax = 255ull * 256 * 28;  // runs of at most 28 coefficients (in registers)
 constexpr uint32_t kLatMaxG = 255;
 // workspace (Fr elements): A, B, P (256 each), mu^(2^s) (16), m^(K/2) (1),
@@ -845,12 +983,9 @@ __global__ void __launch_bounds__(kScanThreads) eval_lat_sum_kernel(const fr* ws
 
 // division, launch 2: the run suffixes of block b, S_t = sum_(t' >= t) L_t' mu^(t' - t)
 // (S_t replaces L_t), and the block value P_b = S_0
-// Six exchange steps inside the wave, then the sum over the waves after: with
-// D_w = s at the end of wave w, S_t += mu^(64 - lane) D_w.  The running value
-// is signed limbs: products with balanced digits (2^28) summed seven times.
 __global__ void __launch_bounds__(kScanThreads) div_lat_suffix_kernel(fr* ws) {
   __shared__ uint32_t wt[4][9];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int t = threadIdx.x, lane = t & 63;
   const uint64_t r = (uint64_t)blockIdx.x * kScanThreads + t;
   fr pw[7];  // mu^(2^s), loaded once before the steps
 #pragma unroll
@@ -859,38 +994,7 @@ __global__ void __launch_bounds__(kScanThreads) div_lat_suffix_kernel(fr* ws) {
   pbd_unpack(fr_load(ws + kWsA + 64 - lane).l, f);  // mu^(64 - lane)
   v9 v;
   unpack_ext(fr_load(ws + kWsL + r).l, v.l);
-#pragma unroll
-  for (int s = 0; s < 6; s++) {
-    v9 o;
-#pragma unroll
-    for (int i = 0; i < 9; i++) o.l[i] = (uint32_t)__shfl_down((int)v.l[i], 1 << s);
-    uint32_t p[9];
-    pbd_unpack(pw[s].l, p);
-    o = v9_mul<false, false, true>(o, p);
-    if (lane + (1 << s) < 64) v = v9_add(v, o);
-  }
-  if (lane == 0) {
-    const fr c = v9_canonical(v);
-    v9 b;
-    unpack_ext(c.l, b.l);
-#pragma unroll
-    for (int i = 0; i < 9; i++) wt[w][i] = b.l[i];
-  }
-  __syncthreads();
-  if (w < 3) {
-    v9 d;  // D_w: the later waves' values by Horner in mu^64
-    uint32_t p[9];
-    pbd_unpack(pw[6].l, p);
-#pragma unroll
-    for (int i = 0; i < 9; i++) d.l[i] = wt[3][i];
-    for (int k = 2; k > w; k--) {
-      d = v9_mul<false, false, true>(d, p);
-#pragma unroll
-      for (int i = 0; i < 9; i++) d.l[i] += wt[k][i];
-    }
-    v = v9_add(v, v9_mul<false, false, true>(d, f));
-  }
-  const fr S = v9_canonical(v);
+  const fr S = run_suffix(v, f, wt, [&](int s, uint32_t* p) { pbd_unpack(pw[s].l, p); });
   fr_store(ws + kWsL + r, S);
   if (t == 0) fr_store(ws + kWsP + blockIdx.x, S);
 }
@@ -905,7 +1009,7 @@ __global__ void __launch_bounds__(kScanThreads) div_lat_suffix_kernel(fr* ws) {
 // Every thread reads its half-run before writing it, so q may be a.
 template <int K>
 __global__ void __launch_bounds__(kScanThreads) div_lat_down_kernel(const fr* a, fr* q, uint64_t n, const fr* c,
-                                                                    fr* ws, uint32_t G, fr* rem) {
+                                                                    int neg, fr* ws, uint32_t G, fr* rem) {
   constexpr int H = K / 2;
   __shared__ uint4 l[2][kScanThreads];
   const int tid = threadIdx.x;
@@ -916,7 +1020,7 @@ __global__ void __launch_bounds__(kScanThreads) div_lat_down_kernel(const fr* a,
   const uint64_t base = r * K + (upper ? H : 0);
   fr v[H];
   load_run<H>(a, n, base, (uint64_t)(b + 1) * kScanThreads * K <= n, v);
-  v9 row = rows29_make<false>(load_m(c, 1));
+  v9 row = rows29_make<false>(load_m(c, neg));
   fr cb = b + 1 + tid < G ? mul_word_pbd(fr_load(ws + kWsP + b + 1 + tid), fr_load(ws + kWsB + tid)) : fr_zero();
   lds_put(l, tid, cb);
   __syncthreads();
@@ -981,8 +1085,9 @@ struct LatRuns {
 };
 template <int K>
 struct LatDown {
-  static void run(dim3 g, hipStream_t s, const fr* a, fr* q, uint64_t n, const fr* c, fr* ws, uint32_t G, fr* rem) {
-    hipLaunchKernelGGL(div_lat_down_kernel<K>, g, dim3(kScanThreads), 0, s, a, q, n, c, ws, G, rem);
+  static void run(dim3 g, hipStream_t s, const fr* a, fr* q, uint64_t n, const fr* c, int neg, fr* ws, uint32_t G,
+                  fr* rem) {
+    hipLaunchKernelGGL(div_lat_down_kernel<K>, g, dim3(kScanThreads), 0, s, a, q, n, c, neg, ws, G, rem);
   }
 };
 
@@ -997,12 +1102,12 @@ static hipError_t evaluate_lat(const fr* a, uint64_t n, const fr* x, fr* y, fr* 
   return hipGetLastError();
 }
 
-// in place: inout <- quotient by (X + c), rem <- remainder (if not null)
-static hipError_t div_lat(fr* inout, uint64_t n, const fr* c, fr* rem, fr* ws, hipStream_t s) {
+// q <- s_(i+1), rem <- s_0 (if not null) with m = -c (neg) or c; q may be a
+static hipError_t div_lat(const fr* a, fr* q, uint64_t n, const fr* c, int neg, fr* rem, fr* ws, hipStream_t s) {
   const uint32_t K = lat_run(n), G = lat_blocks(n, K);
-  lat_dispatch<LatRuns>(K, dim3(G + 1), s, (const fr*)inout, n, c, 1, ws, G, lat_steps(G), 1);
+  lat_dispatch<LatRuns>(K, dim3(G + 1), s, a, n, c, neg, ws, G, lat_steps(G), 1);
   hipLaunchKernelGGL(div_lat_suffix_kernel, dim3(G), dim3(kScanThreads), 0, s, ws);
-  lat_dispatch<LatDown>(K, dim3(2 * G), s, (const fr*)inout, inout, n, c, ws, G, rem);
+  lat_dispatch<LatDown>(K, dim3(2 * G), s, a, q, n, c, neg, ws, G, rem);
   return hipGetLastError();
 }
 
@@ -1023,12 +1128,22 @@ hipError_t grand_product(fr* inout, fr* incl_out, uint64_t n, fr* scratch, hipSt
   return prefix_product<false>(inout, inout, incl_out, n, scratch, s);
 }
 
-hipError_t div_linear(fr* inout, uint64_t n, const fr* c, fr* rem, fr* scratch, hipStream_t s) {
-  if (n >= kLatMin && n <= kLatMax) return div_lat(inout, n, c, rem, scratch, s);
+// the scan of a division by X + c (neg) or an evaluation and division at x:
+// q[i] = s_{i+1}, *total = s_0
+static hipError_t divide(const fr* a, fr* q, uint64_t n, const fr* x, int neg, fr* total, fr* scratch,
+                         hipStream_t s) {
+  if (n >= kLatMin && n <= kLatMax) return div_lat(a, q, n, x, neg, total, scratch, s);
   fr* pw = scratch;
   const int np = sfx_pw_count(n);
-  hipLaunchKernelGGL(sfx_powers_kernel, dim3(1), dim3(64), 0, s, c, 1, pw, std::min(np, kPw), (fr*)nullptr);
-  return suffix_scan(inout, inout, n, pw, rem, scratch + np, s, pw_ext(pw, np));
+  fr* mutab = scratch + np;  // mu^t for the run suffixes, when there is a level above
+  const bool tab = n > (uint64_t)kSeg;
+  hipLaunchKernelGGL(sfx_powers_kernel, dim3(1), dim3(tab ? 128 : 64), 0, s, x, neg, pw, sfx_pw_first(n),
+                     tab ? mutab : nullptr, kLgPer);
+  return suffix_scan(a, q, n, pw, total, mutab + kScanThreads, s, pw_ext(pw, np), tab ? mutab : nullptr);
+}
+
+hipError_t div_linear(fr* inout, uint64_t n, const fr* c, fr* rem, fr* scratch, hipStream_t s) {
+  return divide(inout, inout, n, c, 1, rem, scratch, s);
 }
 
 hipError_t evaluate(const fr* coeffs, uint64_t n, const fr* x, fr* y, fr* scratch, hipStream_t s) {
@@ -1037,17 +1152,14 @@ hipError_t evaluate(const fr* coeffs, uint64_t n, const fr* x, fr* y, fr* scratc
   const int np = sfx_pw_count(n);
   // the reduce's factors m^t (t < 256) as a table beside the powers
   fr* mt = scratch + np;
-  hipLaunchKernelGGL(sfx_powers_kernel, dim3(1), dim3(128), 0, s, x, 0, pw, std::min(np, kPw), mt);
+  hipLaunchKernelGGL(sfx_powers_kernel, dim3(1), dim3(128), 0, s, x, 0, pw, sfx_pw_first(n), mt, 0);
   return suffix_scan(coeffs, nullptr, n, pw, y, mt + kScanThreads, s, pw_ext(pw, np), mt);
 }
 
 // one scan for an evaluation + division pair: q(X) = (p(X) - p(z)) / (X - z)
 // (q[n-1] = 0) and y = p(z); the suffix s_i = a_i + z s_{i+1} gives both
 hipError_t eval_div(const fr* in, fr* q, uint64_t n, const fr* z, fr* y, fr* scratch, hipStream_t s) {
-  fr* pw = scratch;
-  const int np = sfx_pw_count(n);
-  hipLaunchKernelGGL(sfx_powers_kernel, dim3(1), dim3(64), 0, s, z, 0, pw, std::min(np, kPw), (fr*)nullptr);
-  return suffix_scan(in, q, n, pw, y, scratch + np, s, pw_ext(pw, np));
+  return divide(in, q, n, z, 0, y, scratch, s);
 }
 
 }  // namespace pl

@@ -1,4 +1,4 @@
-"""Grand product and batch inversion at the edges of their block geometries
+"""Grand product, batch inversion, evaluation and division at the edges of their block geometries
 (256 threads x 1, 2, 4, 8, 16 elements; one and several blocks), against the
 oracle, with zeros, ones and r - 1 among the inputs."""
 import numpy as np
@@ -59,3 +59,22 @@ def test_inverse_and_quotient_edges(pl, n):
     a, b = pl.to_dev(x), pl.to_dev(y)
     np.testing.assert_array_equal(pl.to_host(pl.vec_op("div", b, a, out=a)), po.mul(y, inv))
     np.testing.assert_array_equal(pl.to_host(pl.vec_op("div", b, xd, out=b)), po.mul(y, inv))
+
+
+# single blocks of each geometry, the latency form's smallest sizes, its largest
+# and the first above it (last wave's runs cut inside and at a chunk of four
+# elements), a second level of one and of several blocks
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 512, 513, 1024, 1025, 2048, 2049, 2052, 3071, 4095, 4097,
+                               255 * 256 * 28, 255 * 256 * 28 + 1, 2000003, 2000004, 2000015, 2000017,
+                               4096 * 512 + 1, 4096 * 1025, 4096 * 2049 - 3, 4096 * 4096 + 1])
+def test_evaluation_and_division_edges(pl, n):
+    import torch
+    print("eval/div edge", n, flush=True)
+    x, z = inputs(n, n), po.uniform(1, n + 7)
+    q, r = po.div(x, z)
+    xd, zd = pl.to_dev(x), pl.to_dev(z)
+    np.testing.assert_array_equal(pl.to_host(pl.evaluate(xd, zd)), po.eval_(x, z))
+    rem = torch.zeros((1, 4), dtype=torch.int64, device="cuda")
+    pl.div_linear(xd, zd, rem=rem)
+    np.testing.assert_array_equal(pl.to_host(xd), q)
+    np.testing.assert_array_equal(pl.to_host(rem).reshape(-1), np.asarray(r).reshape(-1))
