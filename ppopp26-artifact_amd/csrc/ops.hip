@@ -633,6 +633,12 @@ __global__ void __launch_bounds__(256) perm_terms_kernel(RatioArgs a, fr* rn, fr
 // absorbs (32 fr_inv_wave(W) is the R'-view word of 1 / (32 W/R')), so level
 // 0 yields the stored words S(z_i).
 
+// the product over the wave's lanes (R'-view, balanced digits), on every lane
+__device__ __forceinline__ void wave_product(v9& p) {
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) p = v9_mul<false, false, true>(p, shfl_xor9(p, m).l);
+}
+
 // Up-sweep over one level: thread products of num and den over each
 // thread's 8 consecutive elements (tn, td: one per thread of every block, for
 // the down-sweep) and the block products (bn, bd).  Half the block's 512
@@ -657,8 +663,7 @@ __global__ void __launch_bounds__(kUpThreads) gp_up_kernel(const fr* nv, const f
     p = k == 0 ? x : v9_mul<false, false, true>(p, x.l);
   });
   fr_store((den ? td : tn) + tid, v9_canonical(p));
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) p = v9_mul<false, false, true>(p, shfl_xor9(p, m).l);
+  wave_product(p);
   if ((t & 63) == 0) {
 #pragma unroll
     for (int i = 0; i < 9; i++) wt[w][i] = p.l[i];
@@ -685,17 +690,31 @@ __device__ __forceinline__ fr gp_inverse(const fr& total) {
 // with pre_t / suf_t the products over the block's threads before / after t.
 // TOP: a single block; the thread products are formed here and c =
 // gp_inverse(total den), or c = one with the total stored to *tot when a
-// later launch inverts it.  Otherwise c_b = carry[b] and the thread products
-// come from the up-sweep (tn, td).
+// later launch inverts it.  Otherwise the thread products come from the
+// up-sweep (tn, td) and c_b = carry[b], or with nab > 0 block products
+// (carry: nab of num, then nab of den) the block multiplies its own,
+// [prod_{b'<b} num] [prod_{b'>b} den].
 template <int LG, bool INCL, bool TOP>
 __device__ __forceinline__ void gp_down_body(const fr* nv, const fr* dv, const fr* tn, const fr* td, uint64_t n,
-                                             const fr* carry, fr* out, fr* tot,
-                                             uint32_t blk) {
+                                             const fr* carry, uint32_t nab, fr* out, fr* tot, uint32_t blk) {
   constexpr int kPer = 1 << LG;
   __shared__ uint32_t cinv[8];
   const int t = threadIdx.x;
   const uint64_t tid = (uint64_t)blk * kOpThreads + t;
   const uint64_t base = tid * kPer;
+  __shared__ uint32_t wc[4][9];
+  if constexpr (!TOP) {
+    if (nab) {  // first, while few registers are held: each wave's share of c_b
+      const uint32_t j = t;
+      v9 c;
+      split29((j < nab && j != blk ? fr_load(carry + (j < blk ? j : nab + j)) : rp_one()).l, c.l);
+      wave_product(c);
+      if ((t & 63) == 0) {
+#pragma unroll
+        for (int i = 0; i < 9; i++) wc[t >> 6][i] = c.l[i];
+      }
+    }
+  }
   v9 one;
   unpack_ext(rp_one().l, one.l);
   // local den suffixes S[k] (pbd words; a product of a value below 1.07 r and
@@ -738,7 +757,7 @@ __device__ __forceinline__ void gp_down_body(const fr* nv, const fr* dv, const f
   }
   const v9 mine = suf;
   block_scan2(pre, suf, one, TOP ? (int)((n + 64 * kPer - 1) / (64 * kPer)) : 4);
-  fr cw;
+  v9 c;
   if constexpr (TOP) {
     if (t < 64) {
       // total den product = suf_0 x (thread 0's product): lane 0's value
@@ -757,17 +776,16 @@ __device__ __forceinline__ void gp_down_body(const fr* nv, const fr* dv, const f
       }
     }
     __syncthreads();
+    split29(cinv, c.l);
+  } else if (nab) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) cw.l[i] = cinv[i];
+    for (int i = 0; i < 9; i++) c.l[i] = wc[0][i];  // past block_scan2's barrier
+#pragma unroll
+    for (int k = 1; k < 4; k++) c = v9_mul<false, false, true>(c, wc[k]);
   } else {
-    cw = fr_load(carry + blk);
+    split29(fr_load(carry + blk).l, c.l);
   }
-  v9 cur;
-  {
-    v9 a;
-    split29(cw.l, a.l);
-    cur = v9_mul<false, false, false>(v9_mul<false, false, false>(a, pre.l), suf.l);
-  }
+  v9 cur = v9_mul<false, false, false>(v9_mul<false, false, false>(c, pre.l), suf.l);
   static_for<0, kPer>([&](auto k_) {
     constexpr int k = decltype(k_)::value;
     const bool live = base + k < n;
@@ -787,24 +805,46 @@ __device__ __forceinline__ void gp_down_body(const fr* nv, const fr* dv, const f
 
 // bulk levels: three waves per SIMD (the local den suffixes stay in registers)
 // inv != nullptr: one more block than the level needs; block 0 (dispatched
-// first) has its wave 0 write gp_inverse(*tot) to inv while the other blocks
-// sweep (the inverse then multiplies the run carries, gp_run_down_kernel)
+// first) has its wave 0 write gp_inverse(total den product) to inv while the
+// other blocks sweep (the inverse then multiplies the run carries,
+// gp_run_down_kernel).  The total is *tot, or with nab > 0 the product of the
+// nab block products of den.
+// With nab > 0 (the level above is nab <= kOwnCarry block products) every block
+// multiplies its own carry, nine products of a wave, and the launch of the
+// level above goes: 2^20 rows 18 + 33 -> 38 us, the whole call 190 -> 165;
+// 2^15 79.4, 2^22 518.  With up to 512 block products, two per thread, 2^23
+// gained nothing (27 + 65 -> 87 us).
+constexpr uint32_t kOwnCarry = kOpThreads;
 template <bool INCL>
 __global__ void __launch_bounds__(kOpThreads) __attribute__((amdgpu_waves_per_eu(3)))
-gp_down_kernel(const fr* nv, const fr* dv, const fr* tn, const fr* td, uint64_t n, const fr* carry, fr* out,
-               const fr* tot, fr* inv) {
+gp_down_kernel(const fr* nv, const fr* dv, const fr* tn, const fr* td, uint64_t n, const fr* carry, uint32_t nab,
+               fr* out, const fr* tot, fr* inv) {
   uint32_t blk = blockIdx.x;
   if (inv) {
     if (blk == 0) {
       if (threadIdx.x < 64) {
-        const fr z = gp_inverse(fr_load(tot));
+        fr total;
+        if (nab) {
+          v9 p;
+          split29((threadIdx.x < nab ? fr_load(carry + nab + threadIdx.x) : rp_one()).l, p.l);
+          for (uint32_t j = threadIdx.x + 64; j < nab; j += 64) {
+            uint32_t w[9];
+            split29(fr_load(carry + nab + j).l, w);
+            p = v9_mul<false, false, true>(p, w);
+          }
+          wave_product(p);
+          total = v9_canonical(p);
+        } else {
+          total = fr_load(tot);
+        }
+        const fr z = gp_inverse(total);
         if (threadIdx.x == 0) fr_store(inv, z);
       }
       return;
     }
     blk--;
   }
-  gp_down_body<kOpLgPer, INCL, false>(nv, dv, tn, td, n, carry, out, nullptr, blk);
+  gp_down_body<kOpLgPer, INCL, false>(nv, dv, tn, td, n, carry, nab, out, nullptr, blk);
 }
 
 // the single-block top level
@@ -813,7 +853,7 @@ gp_down_kernel(const fr* nv, const fr* dv, const fr* tn, const fr* td, uint64_t 
 template <int LG, bool INCL>
 __global__ void __launch_bounds__(kOpThreads) gp_top_kernel(const fr* nv, const fr* dv, uint64_t n, fr* out,
                                                              fr* tot) {
-  gp_down_body<LG, INCL, true>(nv, dv, nullptr, nullptr, n, nullptr, out, tot, 0);
+  gp_down_body<LG, INCL, true>(nv, dv, nullptr, nullptr, n, nullptr, 0, out, tot, 0);
 }
 
 // Level 0: thread = run of 8 consecutive elements with carry c (the num
@@ -871,14 +911,20 @@ __global__ void __launch_bounds__(256) gp_run_down_kernel(const fr* nv, const fr
   });
 }
 
+// is there a level above level L of the grand product, which has n values?  More
+// than a block's do need one; the runs also from 1025 on, where an up-sweep, and
+// the inversion beside the sweep, beat one block that does both in turn with
+// eight values per thread (2^14 rows 88.6 -> 78.7 us; not at 2^12).
+static bool gp_level_above(int L, uint64_t n) { return n > (uint64_t)(L == 0 ? 4 * kOpThreads : kOpSeg); }
+
 // level sizes of the grand product: the runs of 8 elements (n_1 = ceil(n / 8)),
-// then n_{L+1} = ceil(n_L / 2048) while n_L > 2048; scratch holds den (n), the
+// then n_{L+1} = ceil(n_L / 2048) while gp_level_above; scratch holds den (n), the
 // run products (2 n_1), then per up-swept level the thread products (2 x 256
 // per block) and the next level's num and den, then the total and its inverse
 static uint64_t gp_scratch_elems(uint64_t n) {
   uint64_t m = (n + kOpPer - 1) / kOpPer;
   uint64_t tot = n + 2 * m + 2;  // + the total den product and its inverse
-  while (m > (uint64_t)kOpSeg) {
+  for (int L = 0; gp_level_above(L, m); L++) {
     const uint64_t nb = (m + kOpSeg - 1) / kOpSeg;
     tot += 2 * nb * kOpThreads + 2 * nb;
     m = nb;
@@ -1076,7 +1122,7 @@ hipError_t perm_grand_product(const fr* const w[3], const fr* const sg[3], const
   int top = 0;
   lv[0] = {rn, rd, nullptr, nullptr, nr};
   fr* p = rd + nr;
-  while (lv[top].n > (uint64_t)kOpSeg) {
+  while (gp_level_above(top, lv[top].n)) {
     Level& c = lv[top];
     const uint64_t nb = (c.n + kOpSeg - 1) / kOpSeg;
     c.tn = p;
@@ -1090,17 +1136,20 @@ hipError_t perm_grand_product(const fr* const w[3], const fr* const sg[3], const
     lv[++top] = {bn, bd, nullptr, nullptr, nb};
   }
   // carries in place over each level's num (the runs' carries over rn).  With
-  // a level between the top and the runs, the top stores the total den product
-  // and the first sweep below it inverts it in an extra block.
+  // a level between the top and the runs, the first sweep below the top inverts
+  // the total den product in an extra block; a top of at most kOwnCarry block
+  // products has no launch of its own.
   fr* tot = top > 0 ? p : nullptr;
   fr* inv = top > 0 ? p + 1 : nullptr;
-  gp_top<false>(lv[top].nv, lv[top].dv, lv[top].n, lv[top].nv, tot, s);
+  const bool own = top > 0 && lv[top].n <= kOwnCarry;
+  if (!own) gp_top<false>(lv[top].nv, lv[top].dv, lv[top].n, lv[top].nv, tot, s);
   for (int L = top - 1; L >= 0; L--) {
     const Level& c = lv[L];
     const bool first = L == top - 1;
     const unsigned nb = (unsigned)((c.n + kOpSeg - 1) / kOpSeg) + (first ? 1 : 0);
     hipLaunchKernelGGL(gp_down_kernel<false>, dim3(nb), dim3(kOpThreads), 0, s, c.nv, c.dv, c.tn, c.td, c.n,
-                       (const fr*)lv[L + 1].nv, c.nv, (const fr*)tot, first ? inv : nullptr);
+                       (const fr*)lv[L + 1].nv, first && own ? (uint32_t)lv[top].n : 0u, c.nv, (const fr*)tot,
+                       first ? inv : nullptr);
   }
   hipLaunchKernelGGL(gp_run_down_kernel, dim3((unsigned)((nr + 255) / 256)), dim3(256), 0, s, (const fr*)z,
                      (const fr*)scratch, n, (const fr*)rn, (const fr*)inv, z);

@@ -78,3 +78,19 @@ def test_evaluation_and_division_edges(pl, n):
     pl.div_linear(xd, zd, rem=rem)
     np.testing.assert_array_equal(pl.to_host(xd), q)
     np.testing.assert_array_equal(pl.to_host(rem).reshape(-1), np.asarray(r).reshape(-1))
+
+
+# a top level with its own launch (more than 256 block products), and around the
+# row counts where one block of run products hands over to two levels
+@pytest.mark.parametrize("lg", [13, 14, 23])
+def test_perm_grand_product_is_the_ratios_product(pl, lg):
+    print("perm gp levels", lg, flush=True)
+    n = 1 << lg
+    k = np.concatenate([po.from_u64(v) for v in (1, 7, 13)])
+    col = [pl.to_dev(po.uniform(n, po.seed(po.OP_GP, lg, 60 + j))) for j in range(6)]
+    beta, gamma = pl.to_dev(po.uniform(1, 5)), pl.to_dev(po.uniform(1, 6))
+    col[3][n // 3] = 0
+    dom = pl.Domain(lg)
+    ratio = pl.perm_ratio(col[:3], col[3:], beta, gamma, k, dom)
+    z = pl.perm_ratio(col[:3], col[3:], beta, gamma, k, dom, grand_product=True)
+    np.testing.assert_array_equal(pl.to_host(z), pl.to_host(pl.grand_product(ratio)))
