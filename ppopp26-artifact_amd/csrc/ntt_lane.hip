@@ -38,21 +38,6 @@
 
 namespace pl {
 
-struct LaneArgs {
-  const fr* in;
-  fr* out;
-  const fr* premul;     // optional factor per input element [(poly & pm_mask) << lgN | pos], pbd words of c R'
-  const fr* lin;        // w_N^e, e < N, pbd words of w R'
-  const fr* fin;        // (s, s i^k), k < 4: s = 1, or 1/N for the inverse (pbd words times R')
-  const fr* post;       // LAST: such pairs per output index instead (NttCall::post), or null
-  uint64_t in_pstride;  // element stride between input polys (0: shared input)
-  uint64_t nlines;
-  uint32_t pm_mask;
-  uint32_t lgN;
-  uint32_t lgI;         // LAST: output interleave
-  uint32_t inverse;
-};
-
 // the limb of lane CTRL's choice within the quad
 template <int P0, int P1, int P2, int P3>
 __device__ __forceinline__ uint32_t quad(uint32_t v) {
@@ -74,7 +59,7 @@ __device__ __forceinline__ uint32_t lane_pos(uint32_t tau, int mu, int lr) {
 constexpr int lane_threads(int m) { return 1 << (m > 8 ? m : 8); }
 
 template <int m, bool LAST>
-__global__ void __launch_bounds__(lane_threads(m), 4) ntt_lane_kernel(LaneArgs a) {
+__device__ __forceinline__ void ntt_lane_body(const LaneArgs& a, const uint32_t blk) {
   constexpr int T = lane_threads(m);
   constexpr int C = T >> m;  // columns per workgroup
   constexpr int LGC = C == 1 ? 0 : 8 - m;
@@ -88,7 +73,7 @@ __global__ void __launch_bounds__(lane_threads(m), 4) ntt_lane_kernel(LaneArgs a
   const uint32_t lg = a.lgN;
   const uint32_t nmask = (1u << lg) - 1;
   const uint32_t lgL = lg - m;  // log2 lines per polynomial
-  const uint64_t line_of = (uint64_t)blockIdx.x * C + c;
+  const uint64_t line_of = (uint64_t)blk * C + c;
   // lanes beyond the launch's lines work on its last line and store nothing
   const uint64_t line = line_of < a.nlines ? line_of : a.nlines - 1;
   uint64_t poly;
@@ -209,22 +194,63 @@ __global__ void __launch_bounds__(lane_threads(m), 4) ntt_lane_kernel(LaneArgs a
 }
 
 template <int m, bool LAST>
-static void launch_lane(const LaneArgs& a, hipStream_t s) {
-  constexpr int C = lane_threads(m) >> m;
-  hipLaunchKernelGGL((ntt_lane_kernel<m, LAST>), dim3((unsigned)((a.nlines + C - 1) / C)), dim3(lane_threads(m)), 0, s,
-                     a);
+__global__ void __launch_bounds__(lane_threads(m), 4) ntt_lane_kernel(LaneArgs a) {
+  ntt_lane_body<m, LAST>(a, blockIdx.x);
+}
+
+// Ragged form, as ntt_pass_ragged_kernel: one launch for the columns of many
+// transforms, of one column size; directions mix, the factors' index has it.
+template <int m, bool LAST>
+__global__ void __launch_bounds__(lane_threads(m), 4)
+    ntt_lane_ragged_kernel(const LaneArgs* __restrict__ segs, const uint32_t* __restrict__ seg_block0, uint32_t nsegs) {
+  const uint32_t b = blockIdx.x;
+  uint32_t lo = 0, hi = nsegs - 1;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi + 1) >> 1;
+    if (seg_block0[mid] <= b) lo = mid;
+    else hi = mid - 1;
+  }
+  ntt_lane_body<m, LAST>(segs[lo], b - seg_block0[lo]);
+}
+
+uint32_t lane_blocks(int m, uint64_t nlines) {
+  const int lgC = m >= 8 ? 0 : 8 - m;
+  return (uint32_t)((nlines + (1u << lgC) - 1) >> lgC);
+}
+
+// f(m, last) as compile-time values
+template <class F>
+static void lane_dispatch(int m, bool last, F f) {
+  auto both = [&](auto m_) {
+    if (last) f(m_, std::true_type());
+    else f(m_, std::false_type());
+  };
+  switch (m) {
+    case 4: f(std::integral_constant<int, 4>(), std::true_type()); break;
+    case 5: both(std::integral_constant<int, 5>()); break;
+    case 6: both(std::integral_constant<int, 6>()); break;
+    case 7: both(std::integral_constant<int, 7>()); break;
+    case 8: both(std::integral_constant<int, 8>()); break;
+    case 9: both(std::integral_constant<int, 9>()); break;
+    default: both(std::integral_constant<int, 10>()); break;
+  }
 }
 
 static void launch_lane_m(int m, bool last, const LaneArgs& a, hipStream_t s) {
-  switch (m) {
-    case 4: launch_lane<4, true>(a, s); break;
-    case 5: last ? launch_lane<5, true>(a, s) : launch_lane<5, false>(a, s); break;
-    case 6: last ? launch_lane<6, true>(a, s) : launch_lane<6, false>(a, s); break;
-    case 7: last ? launch_lane<7, true>(a, s) : launch_lane<7, false>(a, s); break;
-    case 8: last ? launch_lane<8, true>(a, s) : launch_lane<8, false>(a, s); break;
-    case 9: last ? launch_lane<9, true>(a, s) : launch_lane<9, false>(a, s); break;
-    default: last ? launch_lane<10, true>(a, s) : launch_lane<10, false>(a, s); break;
-  }
+  lane_dispatch(m, last, [&](auto m_, auto last_) {
+    constexpr int M = decltype(m_)::value;
+    hipLaunchKernelGGL((ntt_lane_kernel<M, decltype(last_)::value>), dim3(lane_blocks(M, a.nlines)),
+                       dim3(lane_threads(M)), 0, s, a);
+  });
+}
+
+void launch_lane_ragged(int m, bool last, const LaneArgs* segs, const uint32_t* seg_block0, uint32_t nsegs,
+                        uint32_t nblocks, hipStream_t s) {
+  lane_dispatch(m, last, [&](auto m_, auto last_) {
+    constexpr int M = decltype(m_)::value;
+    hipLaunchKernelGGL((ntt_lane_ragged_kernel<M, decltype(last_)::value>), dim3(nblocks), dim3(lane_threads(M)), 0, s,
+                       segs, seg_block0, nsegs);
+  });
 }
 
 // fin[dir][k] = (s, s i^(+-k)) in the factors' form; ii[dir] = i^(+-1) = w_256^(+-64)
@@ -280,35 +306,40 @@ bool lane_form(const Domain& d, const NttCall& c) {
   return d.lane_lin && (n <= 1ull << 18 || (d.lg > 12 && n < 1ull << 19));
 }
 
-hipError_t lane_launch(const Domain& d, const NttCall& c, hipStream_t s) {
+int lane_args(const Domain& d, const NttCall& c, LaneArgs (&a)[2], int (&m)[2]) {
   const int lg = d.lg;
   const bool one = lg <= kLaneOne;
-  if (c.premul && one) return hipErrorInvalidValue;  // the caller multiplies first
-  LaneArgs a;
-  memset(&a, 0, sizeof(a));
-  a.lin = d.lane_lin;
-  a.fin = d.lane_fin + (c.inverse ? 8 : 0);
-  a.lgN = lg;
-  a.lgI = c.lgI;
-  a.inverse = c.inverse;
-  a.in = c.in;
-  a.in_pstride = c.in_pstride;
-  a.pm_mask = c.pm_mask;
-  const int m0 = one ? lg : (lg + 1) / 2, m1 = lg - m0;
-  if (!one) {
-    if (!c.tmp) return hipErrorInvalidValue;
-    a.premul = c.premul;
-    a.out = c.tmp;
-    a.nlines = (uint64_t)c.npoly << (lg - m0);
-    launch_lane_m(m0, false, a, s);
-    a.premul = nullptr;
-    a.in = c.tmp;
-    a.in_pstride = 1ull << lg;
-  }
-  a.out = c.out;
-  a.post = c.post;
-  a.nlines = one ? c.npoly : (uint64_t)c.npoly << (lg - m1);
-  launch_lane_m(one ? m0 : m1, true, a, s);
+  memset(a, 0, sizeof(a));
+  a[0].lin = d.lane_lin;
+  a[0].fin = d.lane_fin + (c.inverse ? 8 : 0);
+  a[0].lgN = lg;
+  a[0].lgI = c.lgI;
+  a[0].inverse = c.inverse;
+  a[0].in = c.in;
+  a[0].in_pstride = c.in_pstride;
+  a[0].pm_mask = c.pm_mask;
+  a[0].out = c.out;
+  a[0].post = c.post;
+  m[0] = one ? lg : (lg + 1) / 2;
+  a[0].nlines = (uint64_t)c.npoly << (lg - m[0]);
+  if (one) return 1;
+  a[1] = a[0];
+  a[0].premul = c.premul;
+  a[0].out = c.tmp;
+  a[0].post = nullptr;
+  m[1] = lg - m[0];
+  a[1].in = c.tmp;
+  a[1].in_pstride = 1ull << lg;
+  a[1].nlines = (uint64_t)c.npoly << m[0];
+  return 2;
+}
+
+hipError_t lane_launch(const Domain& d, const NttCall& c, hipStream_t s) {
+  if (d.lg <= kLaneOne ? c.premul != nullptr : !c.tmp) return hipErrorInvalidValue;  // one launch: the caller multiplies first
+  LaneArgs a[2];
+  int m[2];
+  const int np = lane_args(d, c, a, m);
+  for (int p = 0; p < np; p++) launch_lane_m(m[p], p == np - 1, a[p], s);
   return hipGetLastError();
 }
 

@@ -108,6 +108,26 @@ bool lane_form(const Domain& d, const NttCall& c);
 // i times f[i] (stored form), i < N: the transform then leaves f[i] x_i
 hipError_t lane_post_table(const Domain& d, const fr* f, fr* post, hipStream_t s);
 hipError_t lane_launch(const Domain& d, const NttCall& c, hipStream_t s);
+struct LaneArgs {
+  const fr* in;
+  fr* out;
+  const fr* premul;     // optional factor per input element [(poly & pm_mask) << lgN | pos], pbd words of c R'
+  const fr* lin;        // w_N^e, e < N, pbd words of w R'
+  const fr* fin;        // (s, s i^k), k < 4: s = 1, or 1/N for the inverse (pbd words times R')
+  const fr* post;       // LAST: such pairs per output index instead (NttCall::post), or null
+  uint64_t in_pstride;  // element stride between input polys (0: shared input)
+  uint64_t nlines;
+  uint32_t pm_mask;
+  uint32_t lgN;
+  uint32_t lgI;         // LAST: output interleave
+  uint32_t inverse;
+};
+// the launches of a transform in this form (1 or 2): arguments and log2 column sizes
+int lane_args(const Domain& d, const NttCall& c, LaneArgs (&a)[2], int (&m)[2]);
+uint32_t lane_blocks(int m, uint64_t nlines);
+// one launch for segments of one column size 2^m; the tables are on the device
+void launch_lane_ragged(int m, bool last, const LaneArgs* segs, const uint32_t* seg_block0, uint32_t nsegs,
+                        uint32_t nblocks, hipStream_t s);
 
 hipError_t ntt_launch(const Domain& d, const NttCall& c, hipStream_t s);
 hipError_t ntt_launch_one(const Domain& d, const NttCall& c, int p, const fr* in, uint64_t in_pstride,

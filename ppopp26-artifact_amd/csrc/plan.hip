@@ -77,8 +77,17 @@ hipError_t phase_plan(PhasePlan& ph, const std::vector<Item>& items, Bump& bump,
   hipError_t e = hipSuccess;
   ph = PhasePlan();
   ph.items = items;
-  std::map<std::tuple<int, int, int, int, int>, size_t> gidx;
+  std::map<std::tuple<int, int, int, int, int>, size_t> gidx, lidx;
   int n_eval = 0;
+  // Few elements in all: the transforms take the one-element-per-lane form, by
+  // the line lane_form draws for one call (a batch; a server's launch tables
+  // hold pass arguments only).  22 polynomials of 2^10 .. 2^13: 119.9 -> 83.2 us,
+  // five launches of some 8 us for six of 11 to 27 with a few workgroups each.
+  uint64_t elems = 0;
+  for (const Item& it : items)
+    if (it.op == IT_NTT || it.op == IT_INTT || it.op == IT_LDE)
+      elems += 1ull << (it.lg + (it.op == IT_LDE ? it.lg_blowup : 0));
+  const bool lanes = !tables && elems <= 1ull << 18;
   for (size_t i = 0; i < ph.items.size(); i++) {
     const Item& it = ph.items[i];
     const uint64_t n = 1ull << it.lg;
@@ -120,6 +129,27 @@ hipError_t phase_plan(PhasePlan& ph, const std::vector<Item>& items, Bump& bump,
     if (need_tmp)
       c.tmp = it.use_shared_tmp ? it.shared_tmp : (fr*)bump.get(((size_t)c.npoly << it.lg) * sizeof(fr));
     ph.plain_calls.push_back({d, c});
+    if (lanes && d->lane_lin && !(c.premul && it.lg <= kLaneOne)) {
+      LaneArgs la[2];
+      int m[2];
+      const int np = lane_args(*d, c, la, m);
+      for (int p = 0; p < np; p++) {
+        const bool last = p == np - 1;
+        auto f = lidx.emplace(std::make_tuple(p, m[p], 0, last ? 1 : 0, 0), ph.groups.size());
+        if (f.second) {
+          RaggedGroup g;
+          g.level = p;
+          g.last = last;
+          g.lane_m = m[p];
+          ph.groups.push_back(g);
+        }
+        RaggedGroup& g = ph.groups[f.first->second];
+        g.seg_block0.push_back(g.nblocks);
+        g.lsegs.push_back(la[p]);
+        g.nblocks += lane_blocks(m[p], la[p].nlines);
+      }
+      continue;
+    }
     PassArgs a;
     if (!pass_args_regular(*d, c, 0, a)) {
       ph.irregular.push_back({d, c});
@@ -151,7 +181,8 @@ hipError_t phase_plan(PhasePlan& ph, const std::vector<Item>& items, Bump& bump,
   std::stable_sort(ph.groups.begin(), ph.groups.end(),
                    [](const RaggedGroup& x, const RaggedGroup& y) { return x.level < y.level; });
   for (auto& g : ph.groups) {
-    g.d_segs = (PassArgs*)tb.get(g.segs.size() * sizeof(PassArgs));
+    if (g.lane_m) g.d_lsegs = (LaneArgs*)tb.get(g.lsegs.size() * sizeof(LaneArgs));
+    else g.d_segs = (PassArgs*)tb.get(g.segs.size() * sizeof(PassArgs));
     g.d_seg_block0 = (uint32_t*)tb.get(g.seg_block0.size() * sizeof(uint32_t));
   }
   if (n_eval) ph.negz_all = (fr*)bump.get(n_eval * sizeof(fr));
@@ -165,7 +196,9 @@ __global__ void neg_copy_kernel(const fr* z, fr* out) {
 hipError_t phase_upload(PhasePlan& ph, hipStream_t s) {
   hipError_t e = hipSuccess;
   for (auto& g : ph.groups) {
-    if (e == hipSuccess)
+    if (e == hipSuccess && g.lane_m)
+      e = hipMemcpyAsync(g.d_lsegs, g.lsegs.data(), g.lsegs.size() * sizeof(LaneArgs), hipMemcpyHostToDevice, s);
+    else if (e == hipSuccess)
       e = hipMemcpyAsync(g.d_segs, g.segs.data(), g.segs.size() * sizeof(PassArgs), hipMemcpyHostToDevice, s);
     if (e == hipSuccess)
       e = hipMemcpyAsync(g.d_seg_block0, g.seg_block0.data(), g.seg_block0.size() * sizeof(uint32_t),
@@ -175,6 +208,10 @@ hipError_t phase_upload(PhasePlan& ph, hipStream_t s) {
 }
 
 static void launch_ragged(const RaggedGroup& g, hipStream_t s) {
+  if (g.lane_m) {
+    launch_lane_ragged(g.lane_m, g.last, g.d_lsegs, g.d_seg_block0, (uint32_t)g.lsegs.size(), g.nblocks, s);
+    return;
+  }
   const uint32_t ns = (uint32_t)g.segs.size();
   switch (g.la) {
     case 0: launch_pass_ragged_la0(g.inv, g.last, g.scale, g.d_segs, g.d_seg_block0, ns, g.nblocks, s); break;

@@ -59,6 +59,9 @@ struct RaggedGroup {
   int level = 0, la = 0;
   bool inv = false, last = false, scale = false;
   std::vector<PassArgs> segs;
+  int lane_m = 0;  // > 0: a launch of the one-element-per-lane form, columns of 2^lane_m (lsegs)
+  std::vector<LaneArgs> lsegs;
+  LaneArgs* d_lsegs = nullptr;
   std::vector<uint32_t> seg_block0;
   PassArgs* d_segs = nullptr;
   uint32_t* d_seg_block0 = nullptr;

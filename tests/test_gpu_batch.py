@@ -207,3 +207,27 @@ def test_batch_point_rewritten_between_runs(pl):
                 np.testing.assert_array_equal(pl.to_host(items[0]["y"]), y_ref)
                 np.testing.assert_array_equal(pl.to_host(items[0]["out"]), q_ref)
         b.close()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_batch_of_small_transforms(pl, graph):
+    # few elements in all: the one-element-per-lane form in ragged launches, one
+    # launch deep (lg <= 9) and two, columns that share a workgroup and that do
+    # not, both directions and extensions in one launch, beside the other forms
+    spec = [("ntt", lg, 0) for lg in (2, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15)]
+    spec += [("intt", lg, 0) for lg in (4, 6, 9, 10, 11, 13, 16)]
+    spec += [("lde", 5, 2), ("lde", 9, 1), ("lde", 10, 2), ("lde", 11, 3), ("lde", 12, 1)]
+    spec += [("eval_div", lg, 0) for lg in (10, 11)]
+    items = make_items(pl, spec, 900)
+    b = pl.Batch(items, graph=graph)
+    for rep in range(3):
+        for it in items:
+            it["out"].zero_()
+        b.run()
+        for it, (out, y) in zip(items, snapshot(pl, items)):
+            print("small batch item", it["op"], it["lg"], it["lg_blowup"], flush=True)
+            ref, ry = oracle(it)
+            np.testing.assert_array_equal(out, ref)
+            if ry is not None:
+                np.testing.assert_array_equal(y, ry)
+    b.close()
