@@ -80,10 +80,12 @@ struct ScanGeom {
 // its block products and everything a level above reads are in R'-form
 // (RF true).  At 2^21 the only block of the upper level took 37-54 us on
 // chains of 16 products and eight barrier-separated scan steps; with two
-// elements per thread and the scan inside the wave, 9-12 us.  Bounds: with w = 32 x R < 2^261 x / r a step maps |h| to at most
-// 0.453 |h| + r / 2 with centred Montgomery digits (BM), so |h| < 0.96 r from
-// h = S(x_0) < r; in R'-form a step of values within 1.1 r lies in (-1.02 r,
-// 0.02 r).  Both fit a pbd word (1.104 r).
+// elements per thread and the scan inside the wave, 9-12 us.  Bounds: a word of
+// at most r enters as w = 32 x R <= 32 r, so a step maps |h| to at most
+// 0.453 |h| + r / 2 with centred Montgomery digits (BM), and |h| < 0.96 r from
+// h = S(x_0) <= r; in R'-form a step of values within 1.1 r lies in (-1.02 r,
+// 0.02 r).  Both fit a pbd word (1.104 r).  pfx_reduce_kernel packs nothing, so
+// it takes any 256-bit words (16 steps stay within 9 r).
 
 // nine 29-bit digits of 32 x (x any 256-bit word)
 __device__ __forceinline__ void split29_x32(const uint32_t* x, uint32_t* a) {
@@ -94,6 +96,17 @@ __device__ __forceinline__ void split29_x32(const uint32_t* x, uint32_t* a) {
     a[i] = funnel_r(x[(b >> 5) + 1], x[b >> 5], b & 31) & kMask29;
   }
   a[8] = x[7] >> 3;
+}
+
+// a word of x's class below (1 + 2^-30) r: what the running products' bounds
+// above ask of a caller's word.  Canonical words fail the one comparison; any
+// other 256-bit word (below 2.21 r) is at most two subtractions away.
+__device__ __forceinline__ void fr_near_canonical(fr& x) {
+  while (x.l[7] > r_limb(7)) {
+    uint32_t b = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) x.l[i] = __builtin_subc(x.l[i], r_limb(i), b, &b);
+  }
 }
 
 // 32 v for balanced digits of a value within 1.1 r, again balanced
@@ -188,6 +201,7 @@ pfx_down_kernel(const fr* in, fr* out_excl, fr* out_incl, uint64_t n, const fr* 
   v9 h;
   static_for<0, kPer>([&](auto k_) {
     constexpr int k = decltype(k_)::value;
+    if constexpr (!RF) fr_near_canonical(e[k]);
     if constexpr (k == 0) {
       h = one;  // no element of this thread: R'-form one (never stored)
       if (rem > 0) unpack_ext(e[0].l, h.l);
@@ -197,7 +211,7 @@ pfx_down_kernel(const fr* in, fr* out_excl, fr* out_incl, uint64_t n, const fr* 
       else split29_x32(e[k].l, w);
       h = v9_mul<false, !RF, true>(h, w);
     }
-    pbd_pack(h.l, e[k].l);  // canonical words and products fit
+    pbd_pack(h.l, e[k].l);  // words below 1.1 r and products fit
   });
   // thread products in R'-form, their exclusive prefix across the block
   v9 p = RF || rem <= 0 ? h : v9_x32(h);
