@@ -794,10 +794,12 @@ static hipError_t suffix_scan(const fr* a, fr* out, uint64_t n, const fr* pw, fr
 constexpr uint64_t kLatMin = (1ull << 10) + 1;
 constexpr uint64_t kLatMax = 255ull * 256 * 28;  // runs of at most 28 coefficients (in registers)
 constexpr uint32_t kLatMaxG = 255;
-// workspace (Fr elements): A, B, P (256 each), mu^(2^s) (16), m^(K/2) (1),
-// L (256 G; the division replaces it by the run suffixes S), and for the
-// division the upper-half Horner values H (256 G)
-constexpr uint64_t kWsA = 0, kWsB = 256, kWsP = 512, kWsPw = 768, kWsHalf = 784, kWsL = 800;
+// workspace (Fr elements): A, B, P (256 each), mu^(2^s) (16), m^(K/2) (1), m
+// (1), L (256 G; the division replaces it by the run suffixes S), and for the
+// division the upper-half Horner values H (256 G).  The caller's point is read
+// in launch 1 alone: the value, the remainder and the quotient, all written
+// after it, may lie over the point.
+constexpr uint64_t kWsA = 0, kWsB = 256, kWsP = 512, kWsPw = 768, kWsHalf = 784, kWsM = 785, kWsL = 800;
 
 // the multiplier of a scan in stored form: x, or -c for a division by X + c
 __device__ __forceinline__ fr load_m(const fr* x, int neg) {
@@ -872,7 +874,9 @@ __global__ void __launch_bounds__(kScanThreads) lat_runs_kernel(const fr* a, uin
     if (t == 0) ready = 0;
     __syncthreads();
     if (w == 0) {
-      const v9 xp = m_rp(load_m(x, neg));
+      const fr m = load_m(x, neg);
+      if (t == 0) fr_store(ws + kWsM, m);
+      const v9 xp = m_rp(m);
       v9 mu = xp;  // m^K R', left to right; K is even, so m^(K/2) precedes the last squaring
       for (int bit = 30 - __builtin_clz(K); bit >= 0; bit--) {
         if (bit == 0 && t == 0) {
@@ -1022,8 +1026,8 @@ __global__ void __launch_bounds__(kScanThreads) div_lat_suffix_kernel(fr* ws) {
 // s_i = a_i + m s_(i+1).  Block 0 also writes the remainder s_0 = P_0 + M C_0.
 // Every thread reads its half-run before writing it, so q may be a.
 template <int K>
-__global__ void __launch_bounds__(kScanThreads) div_lat_down_kernel(const fr* a, fr* q, uint64_t n, const fr* c,
-                                                                    int neg, fr* ws, uint32_t G, fr* rem) {
+__global__ void __launch_bounds__(kScanThreads) div_lat_down_kernel(const fr* a, fr* q, uint64_t n, fr* ws,
+                                                                    uint32_t G, fr* rem) {
   constexpr int H = K / 2;
   __shared__ uint4 l[2][kScanThreads];
   const int tid = threadIdx.x;
@@ -1034,7 +1038,7 @@ __global__ void __launch_bounds__(kScanThreads) div_lat_down_kernel(const fr* a,
   const uint64_t base = r * K + (upper ? H : 0);
   fr v[H];
   load_run<H>(a, n, base, (uint64_t)(b + 1) * kScanThreads * K <= n, v);
-  v9 row = rows29_make<false>(load_m(c, neg));
+  v9 row = rows29_make<false>(fr_load(ws + kWsM));
   fr cb = b + 1 + tid < G ? mul_word_pbd(fr_load(ws + kWsP + b + 1 + tid), fr_load(ws + kWsB + tid)) : fr_zero();
   lds_put(l, tid, cb);
   __syncthreads();
@@ -1099,9 +1103,8 @@ struct LatRuns {
 };
 template <int K>
 struct LatDown {
-  static void run(dim3 g, hipStream_t s, const fr* a, fr* q, uint64_t n, const fr* c, int neg, fr* ws, uint32_t G,
-                  fr* rem) {
-    hipLaunchKernelGGL(div_lat_down_kernel<K>, g, dim3(kScanThreads), 0, s, a, q, n, c, neg, ws, G, rem);
+  static void run(dim3 g, hipStream_t s, const fr* a, fr* q, uint64_t n, fr* ws, uint32_t G, fr* rem) {
+    hipLaunchKernelGGL(div_lat_down_kernel<K>, g, dim3(kScanThreads), 0, s, a, q, n, ws, G, rem);
   }
 };
 
@@ -1121,7 +1124,7 @@ static hipError_t div_lat(const fr* a, fr* q, uint64_t n, const fr* c, int neg, 
   const uint32_t K = lat_run(n), G = lat_blocks(n, K);
   lat_dispatch<LatRuns>(K, dim3(G + 1), s, a, n, c, neg, ws, G, lat_steps(G), 1);
   hipLaunchKernelGGL(div_lat_suffix_kernel, dim3(G), dim3(kScanThreads), 0, s, ws);
-  lat_dispatch<LatDown>(K, dim3(2 * G), s, a, q, n, c, neg, ws, G, rem);
+  lat_dispatch<LatDown>(K, dim3(2 * G), s, a, q, n, ws, G, rem);
   return hipGetLastError();
 }
 
