@@ -303,6 +303,13 @@ hipError_t lane_post_table(const Domain& d, const fr* f, fr* post, hipStream_t s
 
 bool lane_form(const Domain& d, const NttCall& c) {
   const uint64_t n = (uint64_t)c.npoly << d.lg;
+  // One launch stores outputs while other workgroups still read.  In place each
+  // reads its polynomials before it stores them; an output that lies over its
+  // input in another way goes to the passes, which from 2^7 points on read all
+  // of the input first.
+  if (d.lg <= kLaneOne && !c.premul && !(c.in == c.out && c.in_pstride == 1ull << d.lg && !c.lgI) &&
+      ranges_meet(c.in, c.in_pstride * (c.npoly - 1) + (1ull << d.lg), c.out, n))
+    return false;
   return d.lane_lin && (n <= 1ull << 18 || (d.lg > 12 && n < 1ull << 19));
 }
 

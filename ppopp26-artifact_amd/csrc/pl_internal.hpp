@@ -92,6 +92,11 @@ struct NttCall {
   const fr* post = nullptr;
 };
 
+// whether a[0..na) and b[0..nb) share an element
+inline bool ranges_meet(const fr* a, uint64_t na, const fr* b, uint64_t nb) {
+  return (uintptr_t)a < (uintptr_t)(b + nb) && (uintptr_t)b < (uintptr_t)(a + na);
+}
+
 // The one-element-per-lane form: whole transforms of 2^4 .. 2^kLaneMaxLg
 // points, one launch up to 2^kLaneOne points, where a column still fits one CU
 // well (us per call, one transform: 2^9 in one launch 9.2, 2^10 in one 16.4

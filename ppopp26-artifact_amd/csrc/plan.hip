@@ -72,6 +72,21 @@ size_t cached_domain_bytes() {
 
 // ---- planning --------------------------------------------------------------
 
+static bool transforms(const Item& it) { return it.op == IT_NTT || it.op == IT_INTT || it.op == IT_LDE; }
+static uint64_t out_elems(const Item& it) { return 1ull << (it.lg + (it.op == IT_LDE ? it.lg_blowup : 0)); }
+
+// whether item i stores over what another transform of the phase reads, or over
+// its own input other than in place: such an item may not store in the phase's
+// first launches, where the others' inputs are read
+static bool stores_over_input(const std::vector<Item>& items, size_t i) {
+  const Item& w = items[i];
+  for (size_t j = 0; j < items.size(); j++)
+    if (transforms(items[j]) && !(j == i && w.in == w.out) &&
+        ranges_meet(w.out, out_elems(w), items[j].in, 1ull << items[j].lg))
+      return true;
+  return false;
+}
+
 hipError_t phase_plan(PhasePlan& ph, const std::vector<Item>& items, Bump& bump, Bump* tables) {
   Bump& tb = tables ? *tables : bump;
   hipError_t e = hipSuccess;
@@ -85,8 +100,7 @@ hipError_t phase_plan(PhasePlan& ph, const std::vector<Item>& items, Bump& bump,
   // five launches of some 8 us for six of 11 to 27 with a few workgroups each.
   uint64_t elems = 0;
   for (const Item& it : items)
-    if (it.op == IT_NTT || it.op == IT_INTT || it.op == IT_LDE)
-      elems += 1ull << (it.lg + (it.op == IT_LDE ? it.lg_blowup : 0));
+    if (transforms(it)) elems += out_elems(it);
   const bool lanes = !tables && elems <= 1ull << 18;
   for (size_t i = 0; i < ph.items.size(); i++) {
     const Item& it = ph.items[i];
@@ -129,7 +143,7 @@ hipError_t phase_plan(PhasePlan& ph, const std::vector<Item>& items, Bump& bump,
     if (need_tmp)
       c.tmp = it.use_shared_tmp ? it.shared_tmp : (fr*)bump.get(((size_t)c.npoly << it.lg) * sizeof(fr));
     ph.plain_calls.push_back({d, c});
-    if (lanes && d->lane_lin && !(c.premul && it.lg <= kLaneOne)) {
+    if (lanes && d->lane_lin && (it.lg > kLaneOne || !(c.premul || stores_over_input(ph.items, i)))) {
       LaneArgs la[2];
       int m[2];
       const int np = lane_args(*d, c, la, m);
