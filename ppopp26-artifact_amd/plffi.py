@@ -183,8 +183,12 @@ def _stream(stream):
     if stream is not None:
         return ctypes.c_void_p(stream.cuda_stream)
     # the current stream's handle without a Stream object around it: 0.3 us of a
-    # call's host time instead of 3.1 (a whole small call took 7.1)
-    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+    # call's host time instead of 3.1 (a whole small call took 7.1).  The function
+    # is not part of torch's public interface: where it is missing, the public way.
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(raw(torch.cuda.current_device()))
 
 
 class Domain:
