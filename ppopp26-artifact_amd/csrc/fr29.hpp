@@ -164,6 +164,35 @@ PL_HD29 void mont29_word(const uint32_t* a, const uint32_t* w, uint32_t* t) {
   t[8] = (uint32_t)acc;
 }
 
+// (a w + b v) / 2^261 mod r: two products with one reduction, 234
+// multiply-adds where two mont29 take 306.  For |a_i|, |b_i| < 2^30 and
+// balanced factor digits (|w_j|, |v_j| <= 2^28) a column stays below
+// 18 * 2^58 + 8 * 2^58 + 2^35 < 2^62.8; output digits plain.  With
+// T = (a w + b v) / 2^261 the value lies in (T - r, T], or with WORD, whose
+// last digit of m is taken as in mont29_word, in (T + r/2, T + 3r/2).
+template <bool WORD>
+PL_HD29 void dual29(const uint32_t* a, const uint32_t* w, const uint32_t* b, const uint32_t* v, uint32_t* t) {
+  uint32_t m[9];
+  int64_t acc = 0;
+#pragma unroll
+  for (int k = 0; k < 17; k++) {
+    const int lo = k > 8 ? k - 8 : 0, hi = k < 8 ? k : 8;
+#pragma unroll
+    for (int i = lo; i <= hi; i++)
+      acc += (int64_t)(int32_t)a[i] * (int64_t)(int32_t)w[k - i] + (int64_t)(int32_t)b[i] * (int64_t)(int32_t)v[k - i];
+#pragma unroll
+    for (int i = lo; i <= hi; i++)
+      if (i < k) acc -= (int64_t)(int32_t)m[i] * (int64_t)r29(k - i);
+    const uint32_t dig = WORD && k == 8 ? sext29((uint32_t)acc) - (1u << 29) : ((uint32_t)acc & kMask29);
+    if (k <= 8)
+      m[k] = dig;
+    else
+      t[k - 9] = dig;
+    acc = (acc - (int64_t)(int32_t)dig) >> 29;  // exact
+  }
+  t[8] = (uint32_t)acc;
+}
+
 // t = x w for a fixed factor w given as nine pre-reduced rows: rows[9 j + i]
 // holds digit j of W_i = w 2^(29 (i + D)) mod r, W_i in (-0.51 r, 0.51 r) with
 // balanced digits (rows29_entry builds them).  V = sum_i x_i W_i is congruent
@@ -391,11 +420,7 @@ __device__ __forceinline__ void mont29_word_dev(const uint32_t* x, const uint32_
   t[8] = (uint32_t)acc[17];
 }
 
-// (a w + b v) / 2^261 mod r: two per-lane products with one reduction, 234
-// multiply-adds where two mont29 take 306.  For |a_i|, |b_i| < 2^30 and
-// balanced factor digits a column stays below 18 * 2^58 + 8 * 2^58 + 2^35 <
-// 2^62.8; output digits plain.  With T = (a w + b v) / 2^261 the value lies in
-// (T - r, T], or with WORD in (T + r/2, T + 3r/2) as in mont29_word.
+// dual29 on the device
 template <bool WORD>
 __device__ __forceinline__ void dual29_dev(const uint32_t* a, const uint32_t* w, const uint32_t* b,
                                            const uint32_t* v, uint32_t* t) {
