@@ -5,7 +5,7 @@
 // elements occupies 128 waves of the 1024 that the chip's SIMDs could each take;
 // below about 2^18 elements their time is that chain of products, not the
 // chip's rate.  Here a lane holds one element and a column of M' = 2^m points
-// (4 <= m <= 10) is one workgroup or part of one: m / 2 radix-4 steps (a
+// (4 <= m <= 9) is one workgroup or part of one: m / 2 radix-4 steps (a
 // radix-2 step first when m is odd), each one exchange through LDS and one
 // product per lane.  A quad of lanes holds the four inputs x_q of a radix-4
 // step; lane k forms its output with the twiddle that follows,
@@ -56,6 +56,8 @@ __device__ __forceinline__ uint32_t lane_pos(uint32_t tau, int mu, int lr) {
   return (sub << mu) + (q << (mu - lr)) + j;
 }
 
+constexpr int kLaneMaxM = 9;  // the largest column that lane_args asks for
+static_assert(kLaneOne == kLaneMaxM && (kLaneMaxLg + 1) / 2 <= kLaneMaxM, "lane_dispatch has every column size");
 constexpr int lane_threads(int m) { return 1 << (m > 8 ? m : 8); }
 
 template <int m, bool LAST>
@@ -64,8 +66,7 @@ __device__ __forceinline__ void ntt_lane_body(const LaneArgs& a, const uint32_t 
   constexpr int C = T >> m;  // columns per workgroup
   constexpr int LGC = C == 1 ? 0 : 8 - m;
   constexpr int NS = (m + 1) / 2;
-  constexpr bool DB = T <= 512;  // two exchange buffers: one barrier per step
-  __shared__ uint3 ex[DB ? 2 : 1][3][T];
+  __shared__ uint3 ex[2][3][T];  // two exchange buffers: one barrier per step
 
   const uint32_t tid = threadIdx.x;
   const uint32_t c = (tid >> 2) & (C - 1);
@@ -167,8 +168,7 @@ __device__ __forceinline__ void ntt_lane_body(const LaneArgs& a, const uint32_t 
     if constexpr (s + 1 < NS) {
       const uint32_t wr = (c << m) + lane_pos(tau, lane_mu(m, s), lr);
       const uint32_t rd = (c << m) + lane_pos(tau, lane_mu(m, s + 1), lane_lr(m, s + 1));
-      uint3(*const b)[T] = ex[DB ? s & 1 : 0];
-      if constexpr (!DB && s > 0) __syncthreads();  // the previous exchange's reads are done
+      uint3(*const b)[T] = ex[s & 1];
 #pragma unroll
       for (int h = 0; h < 3; h++) b[h][wr] = make_uint3(x.l[3 * h], x.l[3 * h + 1], x.l[3 * h + 2]);
       __syncthreads();
@@ -231,8 +231,7 @@ static void lane_dispatch(int m, bool last, F f) {
     case 6: both(std::integral_constant<int, 6>()); break;
     case 7: both(std::integral_constant<int, 7>()); break;
     case 8: both(std::integral_constant<int, 8>()); break;
-    case 9: both(std::integral_constant<int, 9>()); break;
-    default: both(std::integral_constant<int, 10>()); break;
+    default: both(std::integral_constant<int, kLaneMaxM>()); break;
   }
 }
 
