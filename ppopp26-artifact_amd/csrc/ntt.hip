@@ -376,8 +376,7 @@ static void launch_pass_la(int la, bool inv, bool last, const PassArgs& a, hipSt
     case 0: launch_pass_la0(inv, last, a, s); break;
     case 1: launch_pass_la1(inv, last, a, s); break;
     case 2: launch_pass_la2(inv, last, a, s); break;
-    case 3: launch_pass_la3(inv, last, a, s); break;
-    default: launch_pass_la4(inv, last, a, s); break;
+    default: launch_pass_la3(inv, last, a, s); break;
   }
 }
 

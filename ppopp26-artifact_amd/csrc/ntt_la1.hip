@@ -1,4 +1,4 @@
-// Pass kernels for columns of 2^5 points (forward/inverse, intermediate/last).
+// Pass kernels for columns of 2^4 points (forward/inverse, intermediate/last).
 #include "ntt_pass.hpp"
 
 namespace pl {

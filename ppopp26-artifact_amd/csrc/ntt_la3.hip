@@ -1,4 +1,4 @@
-// Pass kernels for columns of 2^7 points (forward/inverse, intermediate/last).
+// Pass kernels for columns of 2^6 points (forward/inverse, intermediate/last).
 #include "ntt_pass.hpp"
 
 namespace pl {

@@ -201,27 +201,12 @@ constexpr int kLines = 1 << kLgLines;
 constexpr int kWavesPerSimd = 4;     // that the register allocation must allow
 constexpr int kPhases = 3;           // LDS exchange rounds
 constexpr int kW = 9 / kPhases;      // limbs per exchange round
-static_assert(kW * kPhases == 9, "the exchange rounds cover the nine limbs");
+static_assert(kW == 3 && kW * kPhases == 9, "rounds of one uint3 cover the nine limbs");
 
-template <int W> struct lds_vec;
-template <> struct lds_vec<4> { typedef uint4 type; };
-template <> struct lds_vec<3> { typedef uint3 type; };
-template <> struct lds_vec<2> { typedef uint2 type; };
-template <> struct lds_vec<1> { typedef uint32_t type; };
-
-template <int W>
-__device__ __forceinline__ typename lds_vec<W>::type pack_limbs(const uint32_t* v) {
-  if constexpr (W == 4) return make_uint4(v[0], v[1], v[2], v[3]);
-  else if constexpr (W == 3) return make_uint3(v[0], v[1], v[2]);
-  else if constexpr (W == 2) return make_uint2(v[0], v[1]);
-  else return v[0];
-}
-template <int W>
-__device__ __forceinline__ void unpack_limbs(uint32_t* v, const typename lds_vec<W>::type& q) {
-  if constexpr (W == 4) { v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w; }
-  else if constexpr (W == 3) { v[0] = q.x; v[1] = q.y; v[2] = q.z; }
-  else if constexpr (W == 2) { v[0] = q.x; v[1] = q.y; }
-  else v[0] = q;
+// the limbs of one round
+__device__ __forceinline__ uint3 pack_limbs(const uint32_t* v) { return make_uint3(v[0], v[1], v[2]); }
+__device__ __forceinline__ void unpack_limbs(uint32_t* v, const uint3& q) {
+  v[0] = q.x; v[1] = q.y; v[2] = q.z;
 }
 
 // One pass over columns of M' = 8*A points, A = 2^LA; blk = tile index.
@@ -244,7 +229,7 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
   constexpr int A = 1 << LA;
   constexpr int m = LA + kLgPerT;
   constexpr int F2 = kPerT / A;   // DFT_A groups per lane in sub-step 2
-  typedef typename lds_vec<kW>::type vec;
+  typedef uint3 vec;
   // kW limbs of every tile element (the exchange), and in the last pass first
   // 16 bytes of every element (the loads)
   constexpr size_t kLdsBytes = LAST ? (size_t)16 << (kLgLines + m) : LA > 0 ? sizeof(vec) << (kLgLines + m) : 16;
@@ -423,7 +408,7 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
       if constexpr (h > 0) __syncthreads();  // previous round's reads done before overwrite
       static_for<0, kPerT>([&](auto k2_) {
         constexpr int k2 = decltype(k2_)::value;
-        lds[((k2 * A + rho1) << kLgLines) + lc] = pack_limbs<kW>(hv[k2]);
+        lds[((k2 * A + rho1) << kLgLines) + lc] = pack_limbs(hv[k2]);
       });
       __syncthreads();
       // sub-step 2 gathers: DFT_A over rho1 for F2 values of k2 of one line
@@ -431,7 +416,7 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
         constexpr int f = decltype(f_)::value;
         static_for<0, A>([&](auto r1_) {
           constexpr int r1 = decltype(r1_)::value;
-          unpack_limbs<kW>(&y[f * A + r1].l[kW * h], lds[(((wv * F2 + f) * A + r1) << kLgLines) + lc]);
+          unpack_limbs(&y[f * A + r1].l[kW * h], lds[(((wv * F2 + f) * A + r1) << kLgLines) + lc]);
         });
       });
     });
@@ -609,11 +594,9 @@ PL_DECLARE_RAGGED(0)
 PL_DECLARE_RAGGED(1)
 PL_DECLARE_RAGGED(2)
 PL_DECLARE_RAGGED(3)
-PL_DECLARE_RAGGED(4)
 void launch_pass_la0(bool inv, bool last, const PassArgs& a, hipStream_t s);
 void launch_pass_la1(bool inv, bool last, const PassArgs& a, hipStream_t s);
 void launch_pass_la2(bool inv, bool last, const PassArgs& a, hipStream_t s);
 void launch_pass_la3(bool inv, bool last, const PassArgs& a, hipStream_t s);
-void launch_pass_la4(bool inv, bool last, const PassArgs& a, hipStream_t s);
 
 }  // namespace pl

@@ -231,8 +231,7 @@ static void launch_ragged(const RaggedGroup& g, hipStream_t s) {
     case 0: launch_pass_ragged_la0(g.inv, g.last, g.scale, g.d_segs, g.d_seg_block0, ns, g.nblocks, s); break;
     case 1: launch_pass_ragged_la1(g.inv, g.last, g.scale, g.d_segs, g.d_seg_block0, ns, g.nblocks, s); break;
     case 2: launch_pass_ragged_la2(g.inv, g.last, g.scale, g.d_segs, g.d_seg_block0, ns, g.nblocks, s); break;
-    case 3: launch_pass_ragged_la3(g.inv, g.last, g.scale, g.d_segs, g.d_seg_block0, ns, g.nblocks, s); break;
-    default: launch_pass_ragged_la4(g.inv, g.last, g.scale, g.d_segs, g.d_seg_block0, ns, g.nblocks, s); break;
+    default: launch_pass_ragged_la3(g.inv, g.last, g.scale, g.d_segs, g.d_seg_block0, ns, g.nblocks, s); break;
   }
 }
 
