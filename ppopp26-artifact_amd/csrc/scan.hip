@@ -1142,6 +1142,9 @@ uint64_t scan_scratch_elems(uint64_t n) {
 uint64_t grand_product_scratch_elems(uint64_t n) { return pfx_scratch_elems(n); }
 
 hipError_t grand_product(fr* inout, fr* incl_out, uint64_t n, fr* scratch, hipStream_t s) {
+  // in one buffer the exclusive products stay: the sweep stores an element's
+  // inclusive product after its exclusive one
+  if (incl_out == inout) incl_out = nullptr;
   return prefix_product<false>(inout, inout, incl_out, n, scratch, s);
 }
 
