@@ -9,8 +9,10 @@
 // coset steps read, LDE_distribute_powers, kernels.cuh:122-144) unless the
 // caller gives another shift.  The forward transform runs the library's pass
 // kernels with the coset powers fused into the first pass (the premultiplied
-// pass of the LDE: a table of pbd words of g^i R'); the inverse multiplies the
-// iNTT's output by a table of g^-i.  The reference splits the coset transform
+// pass of the LDE: a table of pbd words of g^i R').  The inverse takes g^-i in
+// the last factors of the one-element-per-lane form where the iNTT runs as that
+// (lane_post_table), and multiplies the passes' output by a table of g^-i above.
+// The reference splits the coset transform
 // into chunked steps (init, forward1/2/3, each a kernel set over a chunk);
 // here the same three-call shape maps onto whole-vector passes
 // (pl_coset_ntt_step): step 1 the first pass (coset powers fused), step 2 the

@@ -24,8 +24,9 @@
 // product centres its last Montgomery digit and adds r, mont29_word) with the
 // twiddle w_N^(J kappa),
 // then contiguous rows in natural order.  Against the pass kernels, one forward
-// transform: 2^9 24.6 -> 9.2 us, 2^12 30.3 -> 10.5, 2^14 42.0 -> 11.5, 2^16
-// 46.0 -> 14.5, 2^18 57.4 -> 43.2 (the caller's own launches take 7.4 of it).
+// transform in a stream of calls: 2^5 13.2 -> 5.2 us, 2^9 25.1 -> 9.3, 2^12 30.8
+// -> 10.4, 2^14 42.1 -> 11.1, 2^16 46.0 -> 14.9, 2^18 58.0 -> 44.6 (before, with
+// the passes of then; pl_internal.hpp has both forms as they are now).
 //
 // Bounds: inputs are plain digits in [0, 2^29), so the sums have |l| < 2^30;
 // values: a caller's 2^256 < 2.21 r makes the first sums 4.42 r each and the

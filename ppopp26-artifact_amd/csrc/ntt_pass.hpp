@@ -30,8 +30,8 @@
 // 2^20: 2.98 -> 2.64 ms; the per-lane twiddles of a 16-column tile of two
 // waves before).  Longer tiles leave two workgroups of eight waves on a CU,
 // so loads and stores hide less behind the other's products than with eight
-// of two: 2^24, a middle pass, 0.42 -> 0.33 ms with 757 -> 534 VALU
-// instructions per element.  Loading the next tile's words into the registers
+// of two: 2^24, a middle pass, 0.42 -> 0.32 ms with 757 -> 519 VALU
+// instructions per element (plain digits, below, included).  Loading the next tile's words into the registers
 // that the results leave (a workgroup looping over 2 .. 16 tiles) was slower
 // (2^24: 1.32 -> 1.42 ms): the passes wait for VALU issue and for memory, not
 // for single loads.
@@ -490,9 +490,10 @@ __device__ __forceinline__ void ntt_pass_body(const PassArgs& a, const uint64_t 
     const fr* tw = a.tw + j;
     // Each twiddle is asked for one product ahead, before the result in
     // between is stored: memory operations complete in order, so a load issued
-    // after a store would wait for it too (NTT 2^24 1.38 -> 1.33 ms by turns;
-    // the middle passes issue VALU on 82 % of the cycles, pass 0 and the
-    // last, nearer the memory rate, on 64 and 61 %).
+    // after a store would wait for it too (NTT 2^24 1.38 -> 1.33 ms by turns).
+    // VALU instructions per busy cycle of the sequencers, where the multiply-add
+    // probe reaches 7.65: the middle passes 7.0 and 7.2, pass 0 and the last,
+    // nearer the memory rate, 6.1 and 5.8.
     auto row = [&](int i) { return (uint64_t)((wv * F2 + i / A) + kPerT * (i % A)) << a.lgS; };
     fr next = fr_load(tw + row(0));
     mem_here();

@@ -811,8 +811,8 @@ __device__ __forceinline__ void gp_down_body(const fr* nv, const fr* dv, const f
 // nab block products of den.
 // With nab > 0 (the level above is nab <= kOwnCarry block products) every block
 // multiplies its own carry, nine products of a wave, and the launch of the
-// level above goes: 2^20 rows 18 + 33 -> 38 us, the whole call 190 -> 165;
-// 2^15 79.4, 2^22 518.  With up to 512 block products, two per thread, 2^23
+// level above goes: 2^20 rows 18 + 33 -> 38 us, the whole call 190 -> 178 (173
+// to 184 from one card to another); 2^15 79.4, 2^22 544.  With up to 512 block products, two per thread, 2^23
 // gained nothing (27 + 65 -> 87 us).
 constexpr uint32_t kOwnCarry = kOpThreads;
 template <bool INCL>

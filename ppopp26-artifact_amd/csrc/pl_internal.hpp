@@ -99,12 +99,28 @@ inline bool ranges_meet(const fr* a, uint64_t na, const fr* b, uint64_t nb) {
 
 // The one-element-per-lane form: whole transforms of 2^4 .. 2^kLaneMaxLg
 // points, one launch up to 2^kLaneOne points, where a column still fits one CU
-// well (us per call, one transform: 2^9 in one launch 9.2, 2^10 in one 16.4
-// and in two 10.3).  lane_form's line lies where the pass kernels, with eight
-// elements per lane and half the instructions, have filled the chip (us per
-// call, lane form against passes): 2^18 elements in all, 2^12 points 28.8 /
-// 42.4, 2^15 36.1 / 51.5, 2^18 46.1 / 69.1; 2^19 elements, 2^12 points (two
-// passes) 47.5 / 47.2, 2^15 61.6 / 60.7, 2^18 79.7 / 74.0.
+// well (us per call, one transform: 2^9 in one launch 9.3, 2^10 in two 10.1, in
+// one it was 16.4).
+//
+// lane_form's line: a lane's chain of products is much shorter than in a pass,
+// but an element costs about twice the instructions, so the form loses once
+// there are enough elements to fill the chip, and the later the more launches
+// the passes take.  us per call, lane form /
+// passes, inverse, by elements in all (2^17 times):
+//            1           2           3           4           5
+//   2^7   8.8/19.0   14.2/22.1   20.0/29.6   25.7/36.7   30.3/35.8
+//   2^9  10.3/24.4   18.0/27.4   24.9/32.6   30.9/35.3   38.1/40.8
+//   2^10 15.4/24.5   26.2/26.9   35.6/30.2   43.6/35.7   48.7/41.7
+//   2^12 16.4/37.2   28.5/39.8   39.7/41.2   49.0/43.6   53.9/43.2
+//   2^13 17.4/38.5   30.5/45.1   42.0/54.1   51.9/59.9   59.9/63.7
+//   2^15 19.8/40.7   35.1/47.9   46.9/49.4   58.3/53.8   71.8/65.3
+//   2^17 25.5/54.6   41.8/59.6   56.1/63.3   71.1/69.3   87.0/70.6
+//   2^18             44.8/65.1               81.3/68.9
+// Up to 2^18 elements it is ahead for every size (level at 2^10).  Against two
+// passes (2^10 .. 2^12) the two cross between there and 3 * 2^17, against three
+// (2^13 on) between 3 * 2^17 and 5 * 2^17: from 2^13 on the line is 2^19, which
+// costs 2^15 up to 10 % near its end (3.75: 57.4/52.4) and gains 2^13 15 %.  The
+// single launches up to 2^9 would be ahead to 5 * 2^17; the line leaves that.
 constexpr int kLaneMaxLg = 18, kLaneOne = 9;
 constexpr int kLaneFin = 16;  // elements of the factor pairs
 hipError_t lane_tables(Domain& d, fr* fin, hipStream_t s);

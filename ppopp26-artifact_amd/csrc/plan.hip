@@ -94,10 +94,12 @@ hipError_t phase_plan(PhasePlan& ph, const std::vector<Item>& items, Bump& bump,
   ph.items = items;
   std::map<std::tuple<int, int, int, int, int>, size_t> gidx, lidx;
   int n_eval = 0;
-  // Few elements in all: the transforms take the one-element-per-lane form, by
-  // the line lane_form draws for one call (a batch; a server's launch tables
-  // hold pass arguments only).  22 polynomials of 2^10 .. 2^13: 119.9 -> 83.2 us,
-  // five launches of some 8 us for six of 11 to 27 with a few workgroups each.
+  // Few elements in all: the transforms take the one-element-per-lane form (a
+  // batch; a server's launch tables hold pass arguments only), up to the 2^18
+  // elements at which it is ahead for every size in one call: a batch mixes
+  // sizes, so lane_form's higher line for the larger ones is not used.  22
+  // polynomials of 2^10 .. 2^13: 115 -> 83 us, five launches of some 8 us for
+  // six of 11 to 27 with a few workgroups each.
   uint64_t elems = 0;
   for (const Item& it : items)
     if (transforms(it)) elems += out_elems(it);

@@ -480,7 +480,9 @@ __global__ void __launch_bounds__(kScanThreads) sfx_reduce_kernel(const fr* a, u
 // The runs come as 128-byte chunks through LDS (run_stage.hpp).
 // Division of 2^24: this kernel 230 -> 200 us, bound by its products; the
 // down-sweep 331 -> 195, a copy's time; with the chunks alone, the scans as
-// before, 200 and 266.  Opening 841 -> 784 us, of 2^22 290 -> 263.
+// before, 200 and 266.  (After half a second of the same load this kernel takes
+// 177, the down-sweep 191.)  Opening of 2^24 + 5 coefficients 845 us, of 2^22 + 5
+// 262; 1010 and 340 with the scans before these and the factor per lane.
 template <bool TAB>
 __global__ void __launch_bounds__(kScanThreads) sfx_run_reduce_kernel(const fr* a, uint64_t n, const fr* pw,
                                                                       fr* partial, fr* lt, PwExt ext,
